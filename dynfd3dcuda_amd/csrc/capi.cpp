@@ -64,6 +64,8 @@ struct FieldRef {
   int planes = 0;  // planes of such an array
   int f0 = 0, fn = 0;  // fn > 0: only the fields f0 .. f0+fn-1 of each plane are exchanged
   bool host = false;   // a host-side value (read only)
+  int swap_n = 0;      // > 0: nine fields of swap_n planes, [field][plane][words] for the caller, on the device
+  size_t swap_stride = 0;  // [plane][field][words] with the planes this many words apart
 };
 
 FieldRef field(Ctx& c, const std::string& n) {
@@ -114,6 +116,8 @@ FieldRef field(Ctx& c, const std::string& n) {
       int a = f / 2;
       long cnt = 9L * c.pml.N * (a == 0 ? (long)c.d.nj * c.d.nk : a == 1 ? (long)c.d.nk * c.d.ni : (long)c.d.ni * c.d.nj);
       f32(c.pml.Y[f], cnt);
+      r.swap_n = a == 0 ? c.pml.N : c.d.ni;
+      r.swap_stride = cnt / r.swap_n * c.pml.parts(a);
     }
   } else if (c.p.Rupture && c.setup_done) {
     if (n == "FW") f32(F.W, 18 * nyz);
@@ -514,6 +518,19 @@ int cgfdm_fault_smooth(cgfdm_ctx* h) {
 // of ny) and the device's plane-interleaved [plane][field][k][jpad + j] with
 // rows of py; to_dev selects the direction.  The slab buffer is the one
 // exception on the caller's side: it is [plane][field][k][j] there too.
+// Between the caller's [field][plane][words] and the device's
+// [plane][field][words], planes swap_stride words apart.
+static size_t swap_bytes(const FieldRef& r) {  // device extent of such a field
+  return ((r.swap_n - 1) * r.swap_stride + r.count / r.swap_n) * dsize(r.dtype);
+}
+static void swap_copy(const FieldRef& r, const char* from, char* to, bool to_dev) {
+  const size_t np = (size_t)r.swap_n, row = r.count / 9 / np * dsize(r.dtype);
+  for (size_t f = 0; f < 9; f++)
+    for (size_t i = 0; i < np; i++) {
+      const size_t dev = i * r.swap_stride * dsize(r.dtype) + f * row, ref = (f * np + i) * row;
+      std::memcpy(to + (to_dev ? dev : ref), from + (to_dev ? ref : dev), row);
+    }
+}
 static size_t dev_words(const Ctx& c, const FieldRef& r) { return (size_t)r.planes * r.nf * c.d.pyz; }
 static void interleave_copy(const Ctx& c, const FieldRef& r, const char* from, char* to, bool to_dev) {
   const size_t es = dsize(r.dtype), nz = (size_t)c.d.nz, ny = (size_t)c.d.ny, py = (size_t)c.d.py;
@@ -551,7 +568,10 @@ int cgfdm_get_field(cgfdm_ctx* h, const char* name, void* dst, size_t bytes) {
   }
   if (hipError_t e = hipStreamSynchronize(c.stream)) return fail(CGFDM_EHIP, hipGetErrorString(e));
   if (!r.nf) {
-    if (hipMemcpy(dst, r.ptr, bytes, hipMemcpyDeviceToHost) != hipSuccess) return fail(CGFDM_EHIP, "copy failed");
+    std::vector<char> tmp(r.swap_n ? swap_bytes(r) : 0);
+    if (hipMemcpy(r.swap_n ? tmp.data() : dst, r.ptr, r.swap_n ? tmp.size() : bytes, hipMemcpyDeviceToHost) != hipSuccess)
+      return fail(CGFDM_EHIP, "copy failed");
+    if (r.swap_n) swap_copy(r, tmp.data(), (char*)dst, false);
     return 0;
   }
   std::vector<char> tmp(dev_words(c, r) * dsize(r.dtype));
@@ -574,7 +594,13 @@ int cgfdm_put_field(cgfdm_ctx* h, const char* name, const void* src, size_t byte
   if (r.host) return fail(CGFDM_EPARAM, std::string("read-only field ") + name);
   if (hipError_t e = hipStreamSynchronize(c.stream)) return fail(CGFDM_EHIP, hipGetErrorString(e));
   if (!r.nf) {
-    if (hipMemcpy(r.ptr, src, bytes, hipMemcpyHostToDevice) != hipSuccess) return fail(CGFDM_EHIP, "copy failed");
+    std::vector<char> tmp(r.swap_n ? swap_bytes(r) : 0);
+    if (r.swap_n) {  // the other face's words between this one's stay as they are
+      if (hipMemcpy(tmp.data(), r.ptr, tmp.size(), hipMemcpyDeviceToHost) != hipSuccess) return fail(CGFDM_EHIP, "copy failed");
+      swap_copy(r, (const char*)src, tmp.data(), true);
+    }
+    if (hipMemcpy(r.ptr, r.swap_n ? tmp.data() : src, r.swap_n ? tmp.size() : bytes, hipMemcpyHostToDevice) != hipSuccess)
+      return fail(CGFDM_EHIP, "copy failed");
     return 0;
   }
   // read-modify-write keeps the row padding of the device array as it is
@@ -718,6 +744,23 @@ int cgfdm_check_field(cgfdm_ctx* h, const char* name, long long* nonfinite, long
   if (r.dtype != 0) return fail(CGFDM_EPARAM, std::string("not an FP32 field: ") + name);
   std::string err;
   const int fn = r.fn ? r.fn : r.nf;
+  if (r.swap_n && r.swap_stride != r.count / r.swap_n) {  // planes of one absorbing face, one after another
+    long long bad = 0, ghost = 0;
+    double most = 0.0;
+    for (int i = 0; i < r.swap_n; i++) {
+      long long b = 0, g = 0;
+      double m = 0.0;
+      if (field_check_host(c, (const float*)r.ptr + i * r.swap_stride, 0, 0, 1, (long)(r.count / r.swap_n), &b, &g, &m, err))
+        return fail(CGFDM_EHIP, err);
+      bad += b;
+      ghost += g;
+      most = std::max(most, m);
+    }
+    if (nonfinite) *nonfinite = bad;
+    if (ghost_nonzero) *ghost_nonzero = ghost;
+    if (maxabs) *maxabs = most;
+    return 0;
+  }
   const int rc = r.nf ? field_check_host(c, (const float*)r.ptr, r.nf, r.f0, fn, 0, nonfinite, ghost_nonzero, maxabs, err)
                       : field_check_host(c, (const float*)r.ptr, 0, 0, 1, (long)r.count, nonfinite, ghost_nonzero, maxabs, err);
   return rc ? fail(CGFDM_EHIP, err) : 0;

@@ -135,9 +135,13 @@ struct FaultDev {
 
 struct PmlDev {
   float *A[3], *B[3], *D[3];  // 1-D profiles along x (ni), y (nj), z (nk); D stored as d/beta
-  float *Y[6], *S[6], *T[6];  // aux per face x1 x2 y1 y2 z1 z2: [9][pni][pnk][pnj]
+  // aux per face x1 x2 y1 y2 z1 z2: nine fields [pnk][pnj] for each of its
+  // planes; the planes of a face are parts(axis) * 9 * pnk * pnj words apart
+  // (along y and z the two faces of the axis alternate plane by plane)
+  float *Y[6], *S[6], *T[6];
   int on[6];
   int N;
+  int parts(int ax) const { return ax == 0 ? 1 : on[2 * ax] + on[2 * ax + 1]; }
 };
 
 // ---------------------------------------------------------------------------
@@ -202,7 +206,6 @@ struct Ctx {
   float *slabH = nullptr;       // [7][9][nz][ny] fault-slab RHS
   float *matVx2Vz = nullptr, *matVy2Vz = nullptr;  // [nx][ny][9]
   float *cj[3] = {nullptr, nullptr, nullptr};      // Cerjan 1-D profiles (nx, ny, nz incl. ghosts)
-  void* wave_cold = nullptr;    // device copy of the off-hot-path pointer table
   void* wave_work = nullptr;    // stage-kernel work list (two int4 per block)
   float* trac_top = nullptr;    // free surface: traction vectors of the six top rows [nx][6][9][ny]
   float* img_top = nullptr;     // free surface: image velocity RHS of the three top rows [3][3][ni][nj]
@@ -280,6 +283,6 @@ int stream_probe_host(int nread, int nwrite, size_t bytes_per_array, int reps, d
 int mlp_train_host(float* blob, const float* feat, const float* target, long n, int epochs, int batch, float lr,
                    unsigned seed, float* loss_hist, std::string& err);
 void launch_fill(Ctx& c, float* p, long n, float v);
-int upload_wave_cold(Ctx& c);  // nonzero on a HIP error
+int upload_wave_work(Ctx& c);  // nonzero on a HIP error
 
 }  // namespace cgfdm

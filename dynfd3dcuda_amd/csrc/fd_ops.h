@@ -135,16 +135,16 @@ __device__ __forceinline__ float rk_combine_o(int irk, float rka, float rkb, flo
 
 }  // namespace fd
 
-// Pointer tables used off the hot path (PML, Cerjan, free-surface maps) live
-// in device memory so that runtime face indices do not force the kernel
-// argument block into scratch.
+// Absorbing-layer arrays and profiles (PML, Cerjan) and free-surface maps, a
+// part of the stage kernels' arguments.
 struct WaveCold {
   const float* pA[3];
   const float* pB[3];
   const float* pD[3];
-  float* auxY[6];
-  float* auxS[6];
-  float* auxT[6];
+  const float* auxY[6];  // auxiliary value of each face
+  float* axY[3];         // auxiliary value, step start and accumulator of each axis's faces (its low face's base)
+  float* axS[3];
+  float* axT[3];
   const float* cj[3];
   const float* mVx;
   const float* mVy;

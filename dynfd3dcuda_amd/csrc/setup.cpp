@@ -960,15 +960,23 @@ int host_setup(Ctx& c, std::string& err) {
     c.pml.B[a] = dmalloc<float>(c, fb.size()); upload(c.pml.B[a], fb);
     c.pml.D[a] = dmalloc<float>(c, fd.size()); upload(c.pml.D[a], fd);
   }
-  for (int f = 0; f < 6; f++) {
-    c.pml.on[f] = p.usePML ? on[f] : 0;
-    if (!c.pml.on[f]) continue;
-    int a = f / 2;
-    long n = 9L * p.PML_N * (a == 0 ? (long)nj * nk : a == 1 ? (long)nk * ni : (long)ni * nj);
-    c.pml.Y[f] = dmalloc<float>(c, n);
-    c.pml.S[f] = dmalloc<float>(c, n);
-    c.pml.T[f] = dmalloc<float>(c, n);
-    if (!c.pml.Y[f] || !c.pml.S[f] || !c.pml.T[f]) { err = "hipMalloc failed for PML"; return 6; }
+  for (int f = 0; f < 6; f++) c.pml.on[f] = p.usePML ? on[f] : 0;
+  for (int a = 0; a < 3; a++) {  // one array of each kind for the faces of an axis
+    const int faces = c.pml.on[2 * a] + c.pml.on[2 * a + 1];
+    if (!faces) continue;
+    const long n = 9L * p.PML_N * (a == 0 ? (long)nj * nk : a == 1 ? (long)nk * ni : (long)ni * nj);  // words of a face
+    const long part = a == 0 ? n : n / ni;  // words from the low to the high face
+    float* v[3];
+    for (float*& q : v) {
+      q = dmalloc<float>(c, faces * n);
+      if (!q) { err = "hipMalloc failed for PML"; return 6; }
+    }
+    int m = 0;
+    for (int f = 2 * a; f < 2 * a + 2; f++)
+      if (c.pml.on[f]) {
+        c.pml.Y[f] = v[0] + m * part; c.pml.S[f] = v[1] + m * part; c.pml.T[f] = v[2] + m * part;
+        m++;
+      }
   }
 
   // Cerjan: damp(i,j,k) = min of three 1-D profiles over the interior
@@ -1148,7 +1156,7 @@ int host_setup(Ctx& c, std::string& err) {
     if (!c.slabH || !F.newton_stats) { err = "hipMalloc failed for the fault"; return 6; }
   }
   c.hW = nullptr;
-  if (upload_wave_cold(c)) { err = "hipMalloc/hipMemcpy failed for the stage-kernel tables"; return 6; }
+  if (upload_wave_work(c)) { err = "hipMalloc/hipMemcpy failed for the stage-kernel tables"; return 6; }
   if (hipDeviceSynchronize() != hipSuccess) { err = "HIP error during setup upload"; return 6; }
   return 0;
 }

@@ -17,7 +17,15 @@ WaveArgs<MT> make_args(Ctx& c, const StageBufs& b, int irk, bool rhs_only, float
   a.rhs = rhs_out;
   a.ttop = c.trac_top;
   a.itop = c.img_top;
-  a.cold = (const WaveCold*)c.wave_cold;
+  WaveCold& w = a.cold;
+  for (int x = 0; x < 3; x++) { w.pA[x] = c.pml.A[x]; w.pB[x] = c.pml.B[x]; w.pD[x] = c.pml.D[x]; w.cj[x] = c.cj[x]; }
+  for (int f = 0; f < 6; f++) { w.auxY[f] = c.pml.Y[f]; w.on[f] = c.pml.on[f]; }
+  for (int x = 0; x < 3; x++) {
+    const int f = c.pml.on[2 * x] ? 2 * x : 2 * x + 1;  // the axis's first absorbing face
+    w.axY[x] = c.pml.Y[f]; w.axS[x] = c.pml.S[f]; w.axT[x] = c.pml.T[f];
+  }
+  w.mVx = c.matVx2Vz; w.mVy = c.matVy2Vz;
+  w.N = c.pml.N;
   bool any = false;
   for (int f = 0; f < 6; f++) any |= c.pml.on[f] != 0;
   a.pml = any ? 1 : 0;
@@ -80,24 +88,13 @@ int interior_lo_j(const Params& p) {
   return (band + TJ - 1) / TJ * TJ;
 }
 
-// Uploads the off-hot-path pointer table and builds the stage-kernel work
-// lists.  The interior box excludes every face band where a PML profile or
+// Builds the stage-kernel work lists and allocates the free-surface buffers.  The interior box excludes every face band where a PML profile or
 // the Cerjan sponge is non-trivial and the three free-surface rows; its
 // tiles start at the box edge so that no interior tile straddles a band.
 // Interior items come first (chunks sized for about 4096 blocks in total, so
 // 256 CUs stay balanced), then the edge items; each list is chunk-major so that
 // one XCD's contiguous share covers neighbouring tiles.
-int upload_wave_cold(Ctx& c) {
-  WaveCold w{};
-  for (int x = 0; x < 3; x++) { w.pA[x] = c.pml.A[x]; w.pB[x] = c.pml.B[x]; w.pD[x] = c.pml.D[x]; w.cj[x] = c.cj[x]; }
-  for (int f = 0; f < 6; f++) { w.auxY[f] = c.pml.Y[f]; w.auxS[f] = c.pml.S[f]; w.auxT[f] = c.pml.T[f]; w.on[f] = c.pml.on[f]; }
-  w.mVx = c.matVx2Vz; w.mVy = c.matVy2Vz;
-  w.N = c.pml.N;
-  if (!c.wave_cold) {
-    if (hipMalloc(&c.wave_cold, sizeof(WaveCold)) != hipSuccess) return 1;
-    c.allocations.push_back(c.wave_cold);
-  }
-  if (hipMemcpy(c.wave_cold, &w, sizeof w, hipMemcpyHostToDevice) != hipSuccess) return 1;
+int upload_wave_work(Ctx& c) {
   if (c.p.FreeSurface && !c.trac_top) {  // the image stencil reaches six rows down (NZ >= 7)
     if (hipMalloc(&c.trac_top, sizeof(float) * 9 * 6 * (size_t)c.d.nx * c.d.ny) != hipSuccess) return 1;
     c.allocations.push_back(c.trac_top);

@@ -91,6 +91,40 @@ __device__ __forceinline__ float bldm(Rsrc r, uint32_t voff, uint32_t soff) {
     return bld<kStream>(r, voff, soff);
   }
 }
+// The auxiliary arrays of an absorbing face hold, for each of its planes pi,
+// nine fields of pnk x pnj words (pp): word (c, pi, pk, pj) at
+// pi*stride + c*pp + pk*pnj + pj.  The two faces of an axis share an array:
+// along x the high face's planes follow the low face's, along y and z the
+// high face's nine fields follow the low face's within each plane.  The
+// plane index is uniform in a block, so one plane of an axis is one buffer
+// resource (its low face's base, np nine-field parts long), addressed like a
+// plane of the volume arrays, with a lane's side in its byte offset.
+__device__ __forceinline__ Rsrc aux_rsrc(const float* a, int pi, uint32_t pp, uint32_t np) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a) + (size_t)pi * np * 9 * pp, (short)0, (int)(np * 9 * pp * 4),
+                                           kBufWord3);
+}
+// A uniform word of an array that no kernel writes (the 1-D profiles): a
+// scalar load, which does not queue behind the vector loads in flight.
+__device__ __forceinline__ float uni(const float* p, int i) {
+  return ((const __attribute__((address_space(4))) float*)p)[i];
+}
+// The same uniform value, with what is computed from it kept at its use: the
+// eight field offsets of each auxiliary array, taken out of the plane loop,
+// do not fit the scalar registers and were read back from vector lanes (866
+// v_readlane in the loop of the 64 x 4 band tiles).
+template <class V>
+__device__ __forceinline__ V here(V v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
+typedef const __attribute__((address_space(4))) WaveCold* ColdPtr;  // in the kernel arguments
+// A register whose value does not matter: read only where every lane that
+// reads it has loaded it, it needs no zeroing.
+__device__ __forceinline__ float any_value() {
+  float v;
+  asm volatile("" : "=v"(v));
+  return v;
+}
 // Word of field c at padded plane x, column jk (plain loads, off the hot path).
 __device__ __forceinline__ float wat(const float* W, int c, int x, uint32_t jk, uint32_t nyz) {
   return W[((size_t)x * 9 + c) * nyz + jk];
@@ -175,7 +209,7 @@ struct WaveArgs {
   float* __restrict__ rhs;
   float* ttop;  // traction vectors of the six top rows (free surface)
   float* itop;  // image velocity RHS of the three top rows (free surface)
-  const WaveCold* __restrict__ cold;
+  WaveCold cold;  // absorbing layers and free-surface maps, indexed with constants only
   const int4* __restrict__ work;  // two int4 per block: (j0, k0, first plane, end plane), (j lanes, k rows, first active j lane, first active k row)
   unsigned nyz;                   // words of one field of one plane (py*nz, padded rows)
   int py, jpad;                   // row pitch and front pad of volume rows
@@ -240,10 +274,9 @@ __global__ void __launch_bounds__(256) image_top_kernel(WaveArgs<MT> a) {
   const float rrhojac = 1.0f / (mat_(M, 12, x, col, a.nyz, a.mref) * mat_(M, 9, x, col, a.nyz, a.mref));
   float rb[3] = {1.0f, 1.0f, 1.0f};
   if (a.pml) {
-    const WaveCold* cold = a.cold;
-    rb[0] = 1.0f / cold->pB[0][i];
-    rb[1] = 1.0f / cold->pB[1][j];
-    rb[2] = 1.0f / cold->pB[2][k];
+    rb[0] = 1.0f / a.cold.pB[0][i];
+    rb[1] = 1.0f / a.cold.pB[1][j];
+    rb[2] = 1.0f / a.cold.pB[2][k];
   }
   const int fl[3] = {FX, FY, FZ};
   const int r0 = k - (nk - 6);  // 3, 4, 5
@@ -303,17 +336,6 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
   constexpr int QLO = FX > 0 ? -1 : -3;  // queue holds planes i+QLO .. i+QLO+4
   constexpr int CTR = -QLO;
   __shared__ float lds[2][9][LK][LJ];
-  // the absorbing layers' uniform descriptors, staged once per block: read
-  // through `cold` inside the plane loop they would be fetched again from
-  // global memory after every store (a chain of dependent round trips per
-  // plane and face), and registers for them would spill
-  __shared__ const float* s_auxY[6];
-  __shared__ const float* s_pBx;
-  __shared__ const float* s_cjx;
-  __shared__ const float* s_mV[2];
-  __shared__ int s_on[6];
-  __shared__ int s_N;
-
   const int item = xcd_remap((int)blockIdx.x, a.nwork);
   const int4 wk = a.work[2 * item], we = a.work[2 * item + 1];
   const int j0 = wk.x, k0 = wk.y, ibeg = wk.z, iend = wk.w;
@@ -332,7 +354,6 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
   const uint32_t mcol = col * (uint32_t)sizeof(MT);
   const uint32_t pb = nyz * 4, mpb = nyz * (uint32_t)sizeof(MT);  // bytes of one field of one plane
   const float* __restrict__ Win = a.Win;
-  const WaveCold* __restrict__ cold = a.cold;
 
   // this thread's halo cell: 4 full rows of LJ cells, then 4 side cells per row
   int hlk = 0, hlj = 0;
@@ -353,15 +374,9 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
   }
   const uint32_t hcol4 = hcol << 2;
 
-  if (KIND >= 1 && threadIdx.y == 0 && threadIdx.x < 6) {
-    s_auxY[threadIdx.x] = cold->auxY[threadIdx.x];
-    s_on[threadIdx.x] = cold->on[threadIdx.x];
-    if (threadIdx.x == 0) { s_N = cold->N; s_pBx = cold->pB[0]; s_cjx = cold->cj[0]; }
-    if (threadIdx.x < 2) s_mV[threadIdx.x] = threadIdx.x ? cold->mVy : cold->mVx;
-  }
   float rb2 = 1.0f, rb3 = 1.0f, cjk = 1.0f;
-  if (act && pml) { rb2 = 1.0f / cold->pB[1][j]; rb3 = 1.0f / cold->pB[2][k]; }
-  if (act && cerjan) cjk = fminf(cold->cj[1][j + 3], cold->cj[2][k + 3]);
+  if (act && pml) { rb2 = 1.0f / a.cold.pB[1][j]; rb3 = 1.0f / a.cold.pB[2][k]; }
+  if (act && cerjan) cjk = fminf(a.cold.cj[1][j + 3], a.cold.cj[2][k + 3]);
 
   float q[5][9];
 #pragma unroll
@@ -411,7 +426,7 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
       const float rrho = 1.0f / MET(12);
       const float l2m = lam + 2.0f * mu;
       const float rDH = a.rDH;
-      const float rb1 = pml ? 1.0f / s_pBx[i] : 1.0f;
+      const float rb1 = pml ? 1.0f / uni(a.cold.pB[0], i) : 1.0f;
       const float(*L)[LK][LJ] = lds[b];
       const int lj = tj + HJL, lk = tk + HKL;
       // one-sided DRP difference of field c along each axis (macdrp.h:91-95),
@@ -442,8 +457,8 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
         float dzv[3];
         if (k == nk - 1) {  // DzV from the traction-free condition (wave.cu:207-232)
           const uint32_t ij = ((uint32_t)(j + 3) + (uint32_t)(i + 3) * (uint32_t)ny) * 9;
-          const float* mVx = s_mV[0];
-          const float* mVy = s_mV[1];
+          const float* mVx = a.cold.mVx;
+          const float* mVy = a.cold.mVy;
           const float dxv[3] = {rDH * Dx(0), rDH * Dx(1), rDH * Dx(2)}, dyv[3] = {rDH * Dy(0), rDH * Dy(1), rDH * Dy(2)};
 #pragma unroll
           for (int r = 0; r < 3; r++)
@@ -477,7 +492,7 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
       // themselves are advanced afterwards by pml_aux_kernel from the same
       // stage input.
       if (pml) {
-        const int N = s_N;
+        const int N = a.cold.N;
 #pragma unroll
         for (int ax = 0; ax < 3; ax++) {
           const int li = ax == 0 ? i : ax == 1 ? j : k;
@@ -486,15 +501,16 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
           for (int side = 0; side < 2; side++) {
             const int f = 2 * ax + side;
             const int off = side ? nn - N : 0;
-            if (!s_on[f] || li < off || li >= off + N) continue;
-            const uint32_t pi = ax == 0 ? i - off : i, pj = ax == 1 ? j - off : j, pk = ax == 2 ? k - off : k;
-            const uint32_t pnj = ax == 1 ? N : nj, pnk = ax == 2 ? N : nk, pni = ax == 0 ? N : ni;
-            const size_t ps = (size_t)pni * pnj * pnk;
-            const uint32_t pa4 = (pj + pk * pnj + pi * pnj * pnk) << 2;
+            if (!a.cold.on[f] || li < off || li >= off + N) continue;
+            const int pi = ax == 0 ? i - off : i;
+            const uint32_t pj = ax == 1 ? j - off : j, pk = ax == 2 ? k - off : k;
+            const uint32_t pnj = ax == 1 ? N : nj, pnk = ax == 2 ? N : nk, pp = pnj * pnk;
+            const uint32_t pa4 = (pj + pk * pnj) << 2;
             const float rbb = ax == 0 ? rb1 : ax == 1 ? rb2 : rb3;  // 1 / beta at li
-            const float* Y = s_auxY[f];
+            const uint32_t np = ax == 0 ? 1u : (uint32_t)(a.cold.on[2 * ax] + a.cold.on[2 * ax + 1]);
+            const Rsrc ry = aux_rsrc(a.cold.auxY[f], pi, pp, np);
 #pragma unroll
-            for (int c = 0; c < 9; c++) h[c] += -ldo(Y + c * ps, pa4) * rbb;
+            for (int c = 0; c < 9; c++) h[c] += -bld(ry, pa4, c * 4 * pp) * rbb;
           }
         }
       }
@@ -507,7 +523,7 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
 #pragma unroll
         for (int c = 0; c < 9; c++) bst(r, col4, c * pb, h[c]);
       } else {
-        const float damp = cerjan ? fminf(s_cjx[i + 3], cjk) : 1.0f;
+        const float damp = cerjan ? fminf(uni(a.cold.cj[0], i + 3), cjk) : 1.0f;
         const bool keep_t = damp != 1.0f || (a.fault && i == a.ii0);
         const Rsrc rs = plane_rsrc(a.S, i + 3, 9, nyz), rt = plane_rsrc(a.T, i + 3, 9, nyz);
         const Rsrc ro = plane_rsrc(a.Wout, i + 3, 9, nyz);
@@ -636,18 +652,6 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
   constexpr int LEAD = RING ? QLEAD : 1;
   constexpr int NS = LEAD + 1;
   __shared__ float lds[NS][9][LK][LJ];
-  // BAND: the absorbing layers' uniform descriptors, staged once per block
-  __shared__ float* s_auxY[6];
-  __shared__ float* s_auxS[6];
-  __shared__ float* s_auxT[6];
-  __shared__ const float* s_pA[3];
-  __shared__ const float* s_pB[3];
-  __shared__ const float* s_pD[3];
-  __shared__ const float* s_pBx;
-  __shared__ const float* s_cjx;
-  __shared__ int s_on[6];
-  __shared__ int s_N;
-  __shared__ const float* s_mV[2];  // TOP: the free-surface velocity maps
   // the media palette of the bfloat16-deviation form, staged once per block
   __shared__ float4 s_pal[std::is_same<MT, MetBf16Delta>::value ? kMaxMediaPalette : 1];
 
@@ -710,41 +714,50 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
       }
   };
 
-  // BAND: per lane, the axes whose absorbing band (one side) holds the
-  // point's column (j, k), their 1/beta, and the sponge factor of the column
+  // BAND: per lane, the sides of the y and z absorbing bands that hold the
+  // point's column (j, k), its 1/beta along them, the sponge factor of the
+  // column, and for a column in one of those bands its auxiliary ODE's
+  // coefficients d/beta and -(alpha + d/beta).  The uniform descriptors are
+  // kernel arguments picked with constant indices, and every auxiliary access
+  // is a buffer access from a uniform plane base.  Through pointers staged in
+  // LDS they were flat accesses, which count as LDS operations too: the
+  // first LDS read of the compute waited for all of them, and the 1/beta of
+  // the next plane for every load ahead of it.  With this, one branch per
+  // stage around the nine fields and the argument reads below, the bands of
+  // 400 x 300 x 200 take 2.85 instead of 3.28 ms per step, of 800 x 1000 x 500
+  // (MetricBF16 2) 16.1 instead of 17.9; on grids of a few million points,
+  // where a plane's instructions are what a block waits for, 15-30% less.
   const bool pml = BAND && a.pml, cerjan = BAND && a.cerjan;
   float rb2 = 1.0f, rb3 = 1.0f, cjk = 1.0f;
-  int N = 0;
-  bool inj = false, ink = false;
-  uint32_t offj = 0, offk = 0;
+  float ad_d = 0.0f, ad_a = 0.0f;
+  const int N = BAND ? a.cold.N : 0;
+  int sj = -1, sk = -1;  // side (0 low, 1 high) of the y and z band holding the column, -1 outside
   if constexpr (BAND) {
-    if (threadIdx.y == 0 && threadIdx.x < 6) {
-      s_auxY[threadIdx.x] = a.cold->auxY[threadIdx.x];
-      s_auxS[threadIdx.x] = a.cold->auxS[threadIdx.x];
-      s_auxT[threadIdx.x] = a.cold->auxT[threadIdx.x];
-      s_on[threadIdx.x] = a.cold->on[threadIdx.x];
-      if (threadIdx.x < 3) {
-        s_pA[threadIdx.x] = a.cold->pA[threadIdx.x];
-        s_pB[threadIdx.x] = a.cold->pB[threadIdx.x];
-        s_pD[threadIdx.x] = a.cold->pD[threadIdx.x];
-      }
-      if (threadIdx.x == 0) { s_N = a.cold->N; s_pBx = a.cold->pB[0]; s_cjx = a.cold->cj[0]; }
-      if (TOP && threadIdx.x < 2) s_mV[threadIdx.x] = threadIdx.x ? a.cold->mVy : a.cold->mVx;
-    }
-    if (act && pml) { rb2 = 1.0f / a.cold->pB[1][j]; rb3 = 1.0f / a.cold->pB[2][k]; }
-    if (act && cerjan) cjk = fminf(a.cold->cj[1][j + 3], a.cold->cj[2][k + 3]);
-    __syncthreads();
-    if (pml) {
-      N = s_N;
-      if (s_on[2] && j < N) { inj = true; offj = 0; }
-      else if (s_on[3] && j >= nj - N) { inj = true; offj = nj - N; }
-      if (s_on[4] && k < N) { ink = true; offk = 0; }
-      else if (s_on[5] && k >= nk - N) { ink = true; offk = nk - N; }
+    if (act && pml) { rb2 = 1.0f / a.cold.pB[1][j]; rb3 = 1.0f / a.cold.pB[2][k]; }
+    if (act && cerjan) cjk = fminf(a.cold.cj[1][j + 3], a.cold.cj[2][k + 3]);
+    if (act && pml) {
+      if (a.cold.on[2] && j < N) sj = 0;
+      else if (a.cold.on[3] && j >= nj - N) sj = 1;
+      if (a.cold.on[4] && k < N) sk = 0;
+      else if (a.cold.on[5] && k >= nk - N) sk = 1;
+      if (sj >= 0) { ad_d = a.cold.pD[1][j]; ad_a = -(a.cold.pA[1][j] + ad_d); }
+      else if (sk >= 0) { ad_d = a.cold.pD[2][k]; ad_a = -(a.cold.pA[2][k] + ad_d); }
     }
   }
+  const bool injl = sj >= 0, inkl = sk >= 0;
+  const ColdPtr kcold = (ColdPtr)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() +
+                                  offsetof(WaveArgs<MT>, cold));
+  const uint32_t xpp = (uint32_t)nk * nj, ypp = (uint32_t)nk * N, zpp = (uint32_t)N * nj;  // words of a field of a face plane
+  const uint32_t nyf = BAND ? a.cold.on[2] + a.cold.on[3] : 0, nzf = BAND ? a.cold.on[4] + a.cold.on[5] : 0;
+  // byte offset of the lane's word in the first field of its x, y and z face
+  // plane (the high y and z faces follow the low ones within a plane)
+  const uint32_t xo4 = BAND ? (uint32_t)(j + k * nj) << 2 : 0u;
+  const uint32_t yo4 = BAND ? ((sj == 1 ? j - (nj - N) + (a.cold.on[2] ? 9 * ypp : 0u) : j) + (uint32_t)(k * N)) << 2 : 0u;
+  const uint32_t zo4 = BAND ? (j + (sk == 1 ? (k - (nk - N)) * nj + (a.cold.on[4] ? 9 * zpp : 0u) : (uint32_t)(k * nj))) << 2 : 0u;
+  const int xoff1 = BAND ? (a.cold.on[0] ? N : 0) : 0;  // first plane of the high x face
   // 1/beta of plane i along x and the sponge factor of plane i (uniform)
-  auto rb_x = [&](int i) { return pml ? 1.0f / s_pBx[i] : 1.0f; };
-  auto cj_x = [&](int i) { return cerjan ? s_cjx[i + 3] : 1.0f; };
+  auto rb_x = [&](int i) { return pml ? 1.0f / uni(a.cold.pB[0], i) : 1.0f; };
+  auto cj_x = [&](int i) { return cerjan ? uni(a.cold.cj[0], i + 3) : 1.0f; };
 
   float q[5][9];
 #pragma unroll
@@ -806,7 +819,7 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
     const Rsrc rs = plane_rsrc(a.S, i + 3, 9, nyz), rt = plane_rsrc(a.T, i + 3, 9, nyz);
     float sv[9], tv[9];
 #pragma unroll
-    for (int c = 0; c < 9; c++) { sv[c] = 0.0f; tv[c] = 0.0f; }
+    for (int c = 0; c < 9; c++) { sv[c] = any_value(); tv[c] = any_value(); }
     if (!a.rhs_only && !slab && irk != 0) {
       if (irk != 1 || keep_t) {
 #pragma unroll
@@ -817,70 +830,70 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
         for (int c = 0; c < 9; c++) sv[c] = bld<kStream>(rs, col4, c * pb);
       }
     }
-    // BAND: the face along each axis whose band holds the point, and the aux
-    // words of plane i (pmlx.cu:126-210 and the y/z variants), all issued
-    // with S and T: the first face's value in ya; for a point on that face
-    // alone and the fused auxiliary update, its step-start (S) and
-    // accumulator (T) words in sa and ta; for a point on two or three faces
-    // (an edge of the absorbing box, whose auxiliary fields pml_aux_kernel
-    // advances) the second and third faces' values in sa and ta instead
+    // BAND: the faces whose band holds the point, and the aux words of plane
+    // i (pmlx.cu:126-210 and the y/z variants), all issued with S and T: the
+    // first face's value in ya; for a point on that face alone and the fused
+    // auxiliary update, its step-start (S) and accumulator (T) words in sa
+    // and ta; for a point on two or three faces (an edge of the absorbing
+    // box, whose auxiliary fields pml_aux_kernel advances) the second and
+    // third faces' values in sa and ta instead.  The x band is uniform; a
+    // lane's y or z face is one of two, each under its own mask.
     float ya[9], sa[9], ta[9];
-    bool inx = false;
-    int fa = -1, fb = -1;               // first and second face axes of the point
-    int nfc = 0;                        // faces holding the point
-    int fo[3] = {0, 0, 0};              // face of each axis
-    uint32_t pa4s[3] = {0, 0, 0};       // aux byte offset of the point in the face of each axis
-    auto face_ps = [&](int ax) { return (size_t)(ax == 0 ? N : ni) * (ax == 1 ? N : nj) * (ax == 2 ? N : nk); };
+    bool inx = false, fuse1 = false;
+    int pix = 0;
+    // the axes' arrays, read again from the kernel arguments in every plane
+    // (kept in registers across the loop they spill to vector lanes)
+    const ColdPtr cold = here(kcold);
+    // applies f(resource, byte offset, bytes of a field) to the lane's word
+    // of its x, y or z face in the axis's array
+    auto on_x = [&](float* arr, auto f) { f(aux_rsrc(arr, pix, xpp, 1), xo4, here(4 * xpp)); };
+    auto on_y = [&](float* arr, auto f) { f(aux_rsrc(arr, i, ypp, nyf), yo4, here(4 * ypp)); };
+    auto on_z = [&](float* arr, auto f) { f(aux_rsrc(arr, i, zpp, nzf), zo4, here(4 * zpp)); };
+    auto ld9 = [](float(&v)[9]) {
+      return [&v](Rsrc r, uint32_t o, uint32_t fb) {
+#pragma unroll
+        for (int c = 0; c < 9; c++) v[c] = bld(r, o, c * fb);
+      };
+    };
     if constexpr (BAND) {
 #pragma unroll
-      for (int c = 0; c < 9; c++) { ya[c] = 0.0f; sa[c] = 0.0f; ta[c] = 0.0f; }
+      for (int c = 0; c < 9; c++) { ya[c] = any_value(); sa[c] = any_value(); ta[c] = any_value(); }
       if (pml) {
-        uint32_t offi = 0;
-        if (s_on[0] && i < N) { inx = true; offi = 0; }
-        else if (s_on[1] && i >= ni - N) { inx = true; offi = ni - N; }
+        if (a.cold.on[0] && i < N) { inx = true; pix = i; }
+        else if (a.cold.on[1] && i >= ni - N) { inx = true; pix = i - (ni - N) + xoff1; }
         const bool fuse = !TOP && a.aux_fused && !a.rhs_only;
-#pragma unroll
-        for (int ax = 0; ax < 3; ax++) {
-          const bool in = ax == 0 ? inx : ax == 1 ? inj : ink;
-          if (!act || !in) continue;
-          const uint32_t off = ax == 0 ? offi : ax == 1 ? offj : offk;
-          fo[ax] = 2 * ax + (off != 0);
-          const uint32_t pi = ax == 0 ? i - offi : i, pj = ax == 1 ? j - offj : j, pk = ax == 2 ? k - offk : k;
-          const uint32_t pnj = ax == 1 ? N : nj, pnk = ax == 2 ? N : nk;
-          pa4s[ax] = (pj + pk * pnj + pi * pnj * pnk) << 2;
-          if (fa < 0) fa = ax;
-          else if (fb < 0) fb = ax;
-          nfc++;
-        }
-        if (fa >= 0) {
-          const int f = fo[fa];
-          const size_t ps = face_ps(fa);
-          const uint32_t pa4 = pa4s[fa];
-#pragma unroll
-          for (int c = 0; c < 9; c++) ya[c] = ldo(s_auxY[f] + c * ps, pa4);
-          if (nfc == 1 && fuse && (irk == 2 || irk == 3)) {  // stage 1 derives the accumulator
-#pragma unroll
-            for (int c = 0; c < 9; c++) ta[c] = ldo(s_auxT[f] + c * ps, pa4);
+        const bool need_t = fuse && irk >= 2, need_s = fuse && (irk == 1 || irk == 2);  // stage 1 derives the accumulator
+        if (inx) {
+          fuse1 = fuse && act && !injl && !inkl;
+          if (act) {
+            on_x(cold->axY[0], ld9(ya));
+            if (injl) on_y(cold->axY[1], ld9(sa));
+            else if (inkl) on_z(cold->axY[2], ld9(sa));
+            if (injl && inkl) on_z(cold->axY[2], ld9(ta));
           }
-          if (nfc == 1 && fuse && (irk == 1 || irk == 2)) {
-#pragma unroll
-            for (int c = 0; c < 9; c++) sa[c] = ldo(s_auxS[f] + c * ps, pa4);
+          if (fuse1) {
+            if (need_t) on_x(cold->axT[0], ld9(ta));
+            if (need_s) on_x(cold->axS[0], ld9(sa));
           }
-        }
-        if (nfc >= 2) {  // the second face's value
-          const size_t ps = face_ps(fb);
-#pragma unroll
-          for (int c = 0; c < 9; c++) sa[c] = ldo(s_auxY[fo[fb]] + c * ps, pa4s[fb]);
-        }
-        if (nfc == 3) {  // the third face's value (the axes are then 0, 1, 2)
-          const size_t ps = face_ps(2);
-#pragma unroll
-          for (int c = 0; c < 9; c++) ta[c] = ldo(s_auxY[fo[2]] + c * ps, pa4s[2]);
+        } else {
+          fuse1 = fuse && injl != inkl;
+          if (injl) {
+            on_y(cold->axY[1], ld9(ya));
+            if (inkl) on_z(cold->axY[2], ld9(sa));
+            if (fuse1) {
+              if (need_t) on_y(cold->axT[1], ld9(ta));
+              if (need_s) on_y(cold->axS[1], ld9(sa));
+            }
+          } else if (inkl) {
+            on_z(cold->axY[2], ld9(ya));
+            if (fuse1) {
+              if (need_t) on_z(cold->axT[2], ld9(ta));
+              if (need_s) on_z(cold->axS[2], ld9(sa));
+            }
+          }
         }
       }
     }
-    // aux value c of the face along axis ax (a face holding the point)
-    auto aux_y = [&](int ax, int c) { return ax == fa ? ya[c] : ax == fb ? sa[c] : ta[c]; };
 
     if (act) {
       auto MET = [&](int c) { return met_raw_get<MT>(mw, c, a.mref, palette ? s_pal : nullptr); };
@@ -921,8 +934,8 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
           float dzv[3];
           if (k == nk - 1) {  // traction-free condition (wave.cu:207-232)
             const uint32_t ij = ((uint32_t)(j + 3) + (uint32_t)(i + 3) * (uint32_t)a.ny) * 9;
-            const float* mVx = s_mV[0];
-            const float* mVy = s_mV[1];
+            const float* mVx = a.cold.mVx;
+            const float* mVy = a.cold.mVy;
             const float dxv[3] = {rDH * Dx(0), rDH * Dx(1), rDH * Dx(2)}, dyv[3] = {rDH * Dy(0), rDH * Dy(1), rDH * Dy(2)};
 #pragma unroll
             for (int r = 0; r < 3; r++)
@@ -951,55 +964,65 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
       }
       if constexpr (BAND) {
         if (pml) {
+          // -aux/beta of each face holding the point, x then y then z
+          if (inx) {
 #pragma unroll
-          for (int ax = 0; ax < 3; ax++) {
-            const bool in = ax == 0 ? inx : ax == 1 ? inj : ink;
-            const float rbb = ax == 0 ? rb1 : ax == 1 ? rb2 : rb3;  // 1 / beta at the point
-            if (in) {
+            for (int c = 0; c < 9; c++) h[c] += -ya[c] * rb1;
+          }
+          if (injl) {
 #pragma unroll
-              for (int c = 0; c < 9; c++) h[c] += -aux_y(ax, c) * rbb;
-            }
+            for (int c = 0; c < 9; c++) h[c] += -(inx ? sa[c] : ya[c]) * rb2;
+          }
+          if (inkl) {
+#pragma unroll
+            for (int c = 0; c < 9; c++) h[c] += -(injl ? (inx ? ta[c] : sa[c]) : (inx ? sa[c] : ya[c])) * rb3;
           }
           // the fused auxiliary update (what pml_aux_kernel does for the
           // point, with the same arithmetic): aux' = -(alpha + d) aux +
           // d * RHS_axis, RHS_axis from the plain derivative along the face's
-          // axis, advanced with the RK4 stage combine
-          if (!TOP && a.aux_fused && !a.rhs_only && nfc == 1) {  // a point on one face only
-            const float rka = a.rka, rkb = a.rkb;
+          // axis, advanced with the RK4 stage combine; points on one face only
+          if (!TOP && a.aux_fused && !a.rhs_only) {
+            auto advance = [&](auto D, float e0, float e1, float e2, float d1, float ad1, float* aY, float* aS, float* aT, auto on) {
+              const float rka = a.rka, rkb = a.rkb;
+              float dd[9], ah[9], w[9];
 #pragma unroll
-            for (int ax = 0; ax < 3; ax++) {
-              if (ax != fa) continue;
-              float dd[9];
+              for (int c = 0; c < 9; c++) dd[c] = rDH * D(c);
 #pragma unroll
-              for (int c = 0; c < 9; c++) dd[c] = rDH * (ax == 0 ? Dx(c) : ax == 1 ? Dy(c) : Dz(c));
-              const float e0 = ax == 0 ? xix : ax == 1 ? etx : ztx;
-              const float e1 = ax == 0 ? xiy : ax == 1 ? ety : zty;
-              const float e2 = ax == 0 ? xiz : ax == 1 ? etz : ztz;
-              const int li = ax == 0 ? i : ax == 1 ? j : k;
-              const float d1 = s_pD[ax][li], ad1 = -(s_pA[ax][li] + d1);
-              const int f = fo[ax];
-              const size_t ps = face_ps(ax);
-              const uint32_t pa4 = pa4s[ax];
-              float* Y = s_auxY[f];
-              float* S = s_auxS[f];
-              float* T = s_auxT[f];
+              for (int c = 0; c < 9; c++) ah[c] = ad1 * ya[c] + d1 * axis_rhs_c(c, dd, e0, e1, e2, rrho, lam, l2m, mu);
+              auto st9 = [](const float(&v)[9]) {
+                return [&v](Rsrc r, uint32_t o, uint32_t fb) {
 #pragma unroll
-              for (int c = 0; c < 9; c++) {
-                const float y = aux_y(ax, c);
-                const float ah = ad1 * y + d1 * axis_rhs_c(c, dd, e0, e1, e2, rrho, lam, l2m, mu);
-                float w;
-                if (irk == 0) {  // the accumulator is derived in stage 1 (rk_derived_t)
-                  sto(S + c * ps, pa4, y);
-                  w = y + rka * ah;
-                } else if (irk == 3) {
-                  w = ta[c] + rkb * ah;
-                } else {
-                  const float t = irk == 1 ? rk_derived_t(sa[c], y) : ta[c];
-                  sto(T + c * ps, pa4, t + rkb * ah);
-                  w = sa[c] + rka * ah;
+                  for (int c = 0; c < 9; c++) bst<kReuse>(r, o, c * fb, v[c]);
+                };
+              };
+              if (irk == 0) {  // the accumulator is derived in stage 1 (rk_derived_t)
+                on(aS, st9(ya));
+#pragma unroll
+                for (int c = 0; c < 9; c++) w[c] = ya[c] + rka * ah[c];
+              } else if (irk == 3) {
+#pragma unroll
+                for (int c = 0; c < 9; c++) w[c] = ta[c] + rkb * ah[c];
+              } else {
+                if (irk == 1) {
+#pragma unroll
+                  for (int c = 0; c < 9; c++) ta[c] = rk_derived_t(sa[c], ya[c]);
                 }
-                sto(Y + c * ps, pa4, w);
+#pragma unroll
+                for (int c = 0; c < 9; c++) ta[c] = ta[c] + rkb * ah[c];
+                on(aT, st9(ta));
+#pragma unroll
+                for (int c = 0; c < 9; c++) w[c] = sa[c] + rka * ah[c];
               }
+              on(aY, st9(w));
+            };
+            if (inx) {
+              if (fuse1) {
+                const float d1 = uni(cold->pD[0], i);
+                advance(Dx, xix, xiy, xiz, d1, -(uni(cold->pA[0], i) + d1), cold->axY[0], cold->axS[0], cold->axT[0], on_x);
+              }
+            } else {
+              if (fuse1 && injl) advance(Dy, etx, ety, etz, ad_d, ad_a, cold->axY[1], cold->axS[1], cold->axT[1], on_y);
+              if (fuse1 && inkl) advance(Dz, ztx, zty, ztz, ad_d, ad_a, cold->axY[2], cold->axS[2], cold->axT[2], on_z);
             }
           }
         }
@@ -1015,20 +1038,27 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
         // RK_Syn (rk4.cu:20-33); the damping factor is 1 in the interior
         const Rsrc ro = plane_rsrc(a.Wout, i + 3, 9, nyz);
         const float rka = a.rka, rkb = a.rkb;
+        // one branch per stage around its nine fields, not one per field
+        if (irk == 0) {
+          if (keep_t) {
 #pragma unroll
-        for (int c = 0; c < 9; c++) {
-          float w;
-          if (irk == 0) {
-            if (keep_t) bst(rt, col4, c * pb, q[CTR][c] + rkb * h[c]);
-            w = q[CTR][c] + rka * h[c];
-          } else if (irk == 3) {
-            w = tv[c] + rkb * h[c];
-          } else {
-            const float t = irk == 1 && !keep_t ? rk_derived_t(sv[c], q[CTR][c]) : tv[c];
-            bst(rt, col4, c * pb, t + rkb * h[c]);
-            w = sv[c] + rka * h[c];
+            for (int c = 0; c < 9; c++) bst(rt, col4, c * pb, q[CTR][c] + rkb * h[c]);
           }
-          bst(ro, col4, c * pb, w * damp);
+#pragma unroll
+          for (int c = 0; c < 9; c++) bst(ro, col4, c * pb, (q[CTR][c] + rka * h[c]) * damp);
+        } else if (irk == 3) {
+#pragma unroll
+          for (int c = 0; c < 9; c++) bst(ro, col4, c * pb, (tv[c] + rkb * h[c]) * damp);
+        } else {
+          if (irk == 1 && !keep_t) {
+#pragma unroll
+            for (int c = 0; c < 9; c++) tv[c] = rk_derived_t(sv[c], q[CTR][c]);
+          }
+#pragma unroll
+          for (int c = 0; c < 9; c++) {
+            bst(rt, col4, c * pb, tv[c] + rkb * h[c]);
+            bst(ro, col4, c * pb, (sv[c] + rka * h[c]) * damp);
+          }
         }
       }
     }
@@ -1082,6 +1112,7 @@ struct PmlAuxArgs {
   const int* __restrict__ boxes;
   int nbox;
   int flag[3];  // one-sided operator sign along each axis
+  int np[3];    // nine-field parts of a plane of each axis's auxiliary arrays
   int N;
   int ni, nj, nk, ny, py, jpad;
   unsigned pyz;
@@ -1114,8 +1145,8 @@ __global__ void __launch_bounds__(256) pml_aux_kernel(PmlAuxArgs<MT> a) {
   const int ax = f >> 1, N = a.N, flag = pick3(ax, a.flag);
   const int nn = ax == 0 ? a.ni : ax == 1 ? a.nj : a.nk;
   const int off = (f & 1) ? nn - N : 0;
-  const int pnj = ax == 1 ? N : a.nj, pnk = ax == 2 ? N : a.nk, pni = ax == 0 ? N : a.ni;
-  const long ps = (long)pni * pnj * pnk;
+  const int pnj = ax == 1 ? N : a.nj, pnk = ax == 2 ? N : a.nk;
+  const long pp = (long)pnj * pnk;
   const long idx = (long)(b - bx[7]) * 256L + threadIdx.x;
   if (idx >= (long)bnj * bnk * bni) return;
   const int pj = bj0 + (int)(idx % bnj);
@@ -1124,7 +1155,7 @@ __global__ void __launch_bounds__(256) pml_aux_kernel(PmlAuxArgs<MT> a) {
   // planes are read by neighbouring blocks), k on the others
   const int pk = bk0 + (ax == 0 ? (int)(t / bni) : (int)(t % bnk));
   const int pi = bi0 + (ax == 0 ? (int)(t % bni) : (int)(t / bnk));
-  const long pa = pj + (long)pk * pnj + (long)pi * pnj * pnk;  // aux layout [c][pi][pk][pj]
+  const long pa = pj + (long)pk * pnj + (long)pi * pick3(ax, a.np) * 9 * pp;  // aux layout (aux_rsrc)
   const int i = pi + (ax == 0 ? off : 0), j = pj + (ax == 1 ? off : 0), k = pk + (ax == 2 ? off : 0);
   const int li = ax == 0 ? i : ax == 1 ? j : k;
   const unsigned pyz = a.pyz;
@@ -1164,7 +1195,7 @@ __global__ void __launch_bounds__(256) pml_aux_kernel(PmlAuxArgs<MT> a) {
   float* T = pick6(f, a.T);
 #pragma unroll
   for (int c = 0; c < 9; c++) {
-    const long q = c * ps + pa;
+    const long q = c * pp + pa;
     const float y = Y[q];
     float ah = ad1 * y + d1 * axis_rhs_c(c, dd, e0, e1, e2, rrho, lam, l2m, mu);
     if (fsx && c >= 3) ah += pml_fs_term(c, z1, ztx, zty, ztz, lam, l2m, mu, c0);
@@ -1289,6 +1320,7 @@ void launch_wave_t(WaveArgs<MT> a, const Ctx& c, hipStream_t s) {
     p.rDH = a.rDH; p.rka = a.rka; p.rkb = a.rkb; p.irk = a.irk; p.freenode = a.freenode;
     p.flag[0] = FX; p.flag[1] = FY; p.flag[2] = FZ;
     for (int ax = 0; ax < 3; ax++) { p.pA[ax] = c.pml.A[ax]; p.pB[ax] = c.pml.B[ax]; p.pD[ax] = c.pml.D[ax]; }
+    for (int ax = 0; ax < 3; ax++) p.np[ax] = c.pml.parts(ax);
     p.mat[0] = c.matVx2Vz; p.mat[1] = c.matVy2Vz;
     for (int f = 0; f < 6; f++) { p.Y[f] = c.pml.Y[f]; p.S[f] = c.pml.S[f]; p.T[f] = c.pml.T[f]; }
     // the boxes (upload_wave_cold): every face whole, or with the fused
