@@ -101,36 +101,17 @@ __device__ __forceinline__ void accum_axis(float* h, F D, float e0, float e1, fl
   h[1] += r2 * d; h[2] += r1 * d;
 }
 
-// RK_Syn stage combine (rk4.cu:20-33) of one value: irk 0 starts the
-// accumulator T and returns w + rka h; irk 1,2 add to T and return
-// S + rka h; irk 3 returns T + rkb h.
-__device__ __forceinline__ float rk_combine(int irk, float rka, float rkb, float w, float h, const float* S, float* T, long x) {
+// RK_Syn stage combine (rk4.cu:20-33) of one value from its words already
+// loaded: irk 0 starts the accumulator t and returns w + rka h; irk 1,2 add
+// to t and return s + rka h; irk 3 returns t + rkb h.
+__device__ __forceinline__ float rk_words(int irk, float rka, float rkb, float w, float h, float s, float& t) {
   if (irk == 0) {
-    T[x] = w + rkb * h;
+    t = w + rkb * h;
     return w + rka * h;
   }
-  if (irk == 3) return T[x] + rkb * h;
-  T[x] = T[x] + rkb * h;
-  return S[x] + rka * h;
-}
-
-// Loads and stores at a 32-bit byte offset from a wave-uniform base, so the
-// compiler can address with one 32-bit VGPR against a scalar base.
-template <class T>
-__device__ __forceinline__ T ldo(const T* base, uint32_t bo) { return *(const T*)((const char*)base + bo); }
-template <class T>
-__device__ __forceinline__ void sto(T* base, uint32_t bo, T v) { *(T*)((char*)base + bo) = v; }
-
-// Same combine at byte offset bo of the field bases S, T.
-__device__ __forceinline__ float rk_combine_o(int irk, float rka, float rkb, float w, float h, const float* S, float* T,
-                                              uint32_t bo) {
-  if (irk == 0) {
-    sto(T, bo, w + rkb * h);
-    return w + rka * h;
-  }
-  if (irk == 3) return ldo(T, bo) + rkb * h;
-  sto(T, bo, ldo(T, bo) + rkb * h);
-  return ldo(S, bo) + rka * h;
+  if (irk == 3) return t + rkb * h;
+  t = t + rkb * h;
+  return s + rka * h;
 }
 
 }  // namespace fd

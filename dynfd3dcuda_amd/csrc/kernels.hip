@@ -128,76 +128,116 @@ __device__ int nr_search(double x, double psi, double A, double Vhat, double coe
   return iter;
 }
 
+// fault2wave (transform.cu:224-403): the stress and velocity of the fault
+// plane from its T1 and the mean of the split nodes' words (fw[c][m], both
+// sides), through the metric of plane i0 (mt[r][axis], the Jacobian jac);
+// o holds Vx Vy Vz Txx Tyy Tzz Txy Txz Tyz.
+struct FaultMetric {
+  float mt[3][3], jac;
+};
+__device__ __forceinline__ FaultMetric load_fault_metric(const FArgs& a, long p) {
+  return {{{LMF(a, 0, p), LMF(a, 3, p), LMF(a, 6, p)},
+           {LMF(a, 1, p), LMF(a, 4, p), LMF(a, 7, p)},
+           {LMF(a, 2, p), LMF(a, 5, p), LMF(a, 8, p)}},
+          LMF(a, 9, p)};
+}
+__device__ __forceinline__ void fault2wave(const FaultMetric& f, const float* T1, const float (&fw)[9][2], float* o) {
+  const float(*mt)[3] = f.mt;
+  float rj = 1.0f / f.jac;
+  float inv[3][3];
+  inv[0][0] = mt[1][1] * mt[2][2] - mt[2][1] * mt[1][2];
+  inv[0][1] = mt[2][1] * mt[0][2] - mt[0][1] * mt[2][2];
+  inv[0][2] = mt[0][1] * mt[1][2] - mt[0][2] * mt[1][1];
+  inv[1][0] = mt[1][2] * mt[2][0] - mt[1][0] * mt[2][2];
+  inv[1][1] = mt[0][0] * mt[2][2] - mt[2][0] * mt[0][2];
+  inv[1][2] = mt[1][0] * mt[0][2] - mt[0][0] * mt[1][2];
+  inv[2][0] = mt[1][0] * mt[2][1] - mt[1][1] * mt[2][0];
+  inv[2][1] = mt[2][0] * mt[0][1] - mt[0][0] * mt[2][1];
+  inv[2][2] = mt[0][0] * mt[1][1] - mt[0][1] * mt[1][0];
+  float det = 1.0f / (inv[0][0] * mt[0][0] + inv[0][1] * mt[1][0] + inv[0][2] * mt[2][0]);
+  float tr[3][3];
+  for (int c = 0; c < 3; c++) {
+    tr[c][0] = T1[c];
+    tr[c][1] = (fw[3 + c][0] + fw[3 + c][1]) * 0.5f;
+    tr[c][2] = (fw[6 + c][0] + fw[6 + c][1]) * 0.5f;
+  }
+  float sg[3][3];
+  for (int r = 0; r < 3; r++)
+    for (int cc = 0; cc < 3; cc++)
+      sg[r][cc] = (tr[r][0] * inv[0][cc] + tr[r][1] * inv[1][cc] + tr[r][2] * inv[2][cc]) * det * rj;
+  for (int c = 0; c < 3; c++) o[c] = (fw[c][0] + fw[c][1]) * 0.5f;
+  o[3] = sg[0][0];
+  o[4] = sg[1][1];
+  o[5] = sg[2][2];
+  o[6] = (sg[0][1] + sg[1][0]) * 0.5f;
+  o[7] = (sg[0][2] + sg[2][0]) * 0.5f;
+  o[8] = (sg[1][2] + sg[2][1]) * 0.5f;
+}
+
+// The fault kernels load everything a node needs before they store anything:
+// the compiler may not move a load above a store that might alias it, so
+// loads between stores were a chain of memory round trips (fault_pre on the
+// 30 x 80 x 50 grid, where the latency shows bare: 20 -> 12 us; fault_post
+// 16 -> 8 us).
+
+// What the shared end of the trial reads.
+struct TailIn {
+  float si[3], mT[3], fw[9][2];
+  FaultMetric fm;
+  int t0_flag;
+};
+__device__ __forceinline__ TailIn load_tail(const FArgs& a, const FaultDev& F, long q, long pf, long pc) {
+  const long nyz = a.nyz;
+  TailIn t;
+  t.si[0] = F.str_init_x[q]; t.si[1] = F.str_init_y[q]; t.si[2] = F.str_init_z[q];
+  t.mT[0] = F.mT11[pf]; t.mT[1] = F.mT12[pf]; t.mT[2] = F.mT13[pf];
+#pragma unroll
+  for (int c = 0; c < 9; c++) {
+    t.fw[c][0] = F.W[c * 2 * nyz + pf];
+    t.fw[c][1] = F.W[c * 2 * nyz + nyz + pf];
+  }
+  t.fm = load_fault_metric(a, pc + a.i0 * a.mps);
+  t.t0_flag = F.init_t0_flag[q];
+  return t;
+}
+
 // Shared end of the friction trial (trial_slipweakening.cu:640-709,
 // trial_ratestate.cu:800-880): T1 on the fault plane with the optional
 // viscosity term, the stage traction averages, rupture time, then
 // fault2wave (transform.cu:224-403) into the stage input at i0.
-__device__ __forceinline__ void fault_tail(const FArgs& a, const FaultDev& F, long q, long pf, long pc,
+__device__ __forceinline__ void fault_tail(const FArgs& a, const FaultDev& F, long q, long pf, long pc, const TailIn& in,
                                            const float* Tau, float Tau_n, bool ifchange, float ratecheck,
                                            const float* Trial, float jacvec, const float* s1, const float* s2) {
-  const long nyz = a.nyz, pyz = a.pyz, wps = a.wps, mps = a.mps;
+  const long nyz = a.nyz, pyz = a.pyz, wps = a.wps;
   const int i0 = a.i0, irk = a.irk;
   const float DT = a.DT;
   long p1 = 3 * nyz + pf;
   float T1[3];
   if (ifchange) {
-    T1[0] = (Tau[0] - F.str_init_x[q]) * jacvec;
-    T1[1] = (Tau[1] - F.str_init_y[q]) * jacvec;
-    T1[2] = (Tau[2] - F.str_init_z[q]) * jacvec;
+    T1[0] = (Tau[0] - in.si[0]) * jacvec;
+    T1[1] = (Tau[1] - in.si[1]) * jacvec;
+    T1[2] = (Tau[2] - in.si[2]) * jacvec;
   } else {
     T1[0] = Trial[0]; T1[1] = Trial[1]; T1[2] = Trial[2];
   }
   float vis = a.viscosity * DT;
-  float h1 = (T1[0] - F.mT11[pf]) / DT, h2 = (T1[1] - F.mT12[pf]) / DT, h3 = (T1[2] - F.mT13[pf]) / DT;
+  float h1 = (T1[0] - in.mT[0]) / DT, h2 = (T1[1] - in.mT[1]) / DT, h3 = (T1[2] - in.mT[2]) / DT;
   if (irk == 3) { F.hT11[pf] = h1; F.hT12[pf] = h2; F.hT13[pf] = h3; }
   T1[0] += vis * h1; T1[1] += vis * h2; T1[2] += vis * h3;
   F.T11[p1] = T1[0]; F.T12[p1] = T1[1]; F.T13[p1] = T1[2];
   F.tTs1[q] = Tau[0] * s1[0] + Tau[1] * s1[1] + Tau[2] * s1[2];
   F.tTs2[q] = Tau[0] * s2[0] + Tau[1] * s2[1] + Tau[2] * s2[2];
   F.tTn[q] = Tau_n;
-  if (!F.init_t0_flag[q] && ratecheck > 1e-3f) {
+  if (!in.t0_flag && ratecheck > 1e-3f) {
     F.init_t0[q] = a.it * DT;
     F.init_t0_flag[q] = 1;
     F.flag_rup[q] = 1;
   }
-
-  // ---- fault2wave into the stage input at i0
-  {
-    const long p = pc + i0 * mps, pw = pc + i0 * wps;
-    float mt[3][3] = {{LMF(a, 0, p), LMF(a, 3, p), LMF(a, 6, p)},
-                      {LMF(a, 1, p), LMF(a, 4, p), LMF(a, 7, p)},
-                      {LMF(a, 2, p), LMF(a, 5, p), LMF(a, 8, p)}};
-    float rj = 1.0f / LMF(a, 9, p);
-    float inv[3][3];
-    inv[0][0] = mt[1][1] * mt[2][2] - mt[2][1] * mt[1][2];
-    inv[0][1] = mt[2][1] * mt[0][2] - mt[0][1] * mt[2][2];
-    inv[0][2] = mt[0][1] * mt[1][2] - mt[0][2] * mt[1][1];
-    inv[1][0] = mt[1][2] * mt[2][0] - mt[1][0] * mt[2][2];
-    inv[1][1] = mt[0][0] * mt[2][2] - mt[2][0] * mt[0][2];
-    inv[1][2] = mt[1][0] * mt[0][2] - mt[0][0] * mt[1][2];
-    inv[2][0] = mt[1][0] * mt[2][1] - mt[1][1] * mt[2][0];
-    inv[2][1] = mt[2][0] * mt[0][1] - mt[0][0] * mt[2][1];
-    inv[2][2] = mt[0][0] * mt[1][1] - mt[0][1] * mt[1][0];
-    float det = 1.0f / (inv[0][0] * mt[0][0] + inv[0][1] * mt[1][0] + inv[0][2] * mt[2][0]);
-    float tr[3][3];
-    for (int c = 0; c < 3; c++) {
-      tr[c][0] = T1[c];
-      tr[c][1] = (F.W[(3 + c) * 2 * nyz + pf] + F.W[(3 + c) * 2 * nyz + nyz + pf]) * 0.5f;
-      tr[c][2] = (F.W[(6 + c) * 2 * nyz + pf] + F.W[(6 + c) * 2 * nyz + nyz + pf]) * 0.5f;
-    }
-    float sg[3][3];
-    for (int r = 0; r < 3; r++)
-      for (int cc = 0; cc < 3; cc++)
-        sg[r][cc] = (tr[r][0] * inv[0][cc] + tr[r][1] * inv[1][cc] + tr[r][2] * inv[2][cc]) * det * rj;
-    float* W = a.Wi0;
-    for (int c = 0; c < 3; c++) W[c * pyz + pw] = (F.W[c * 2 * nyz + pf] + F.W[c * 2 * nyz + nyz + pf]) * 0.5f;
-    W[3 * pyz + pw] = sg[0][0];
-    W[4 * pyz + pw] = sg[1][1];
-    W[5 * pyz + pw] = sg[2][2];
-    W[6 * pyz + pw] = (sg[0][1] + sg[1][0]) * 0.5f;
-    W[7 * pyz + pw] = (sg[0][2] + sg[2][0]) * 0.5f;
-    W[8 * pyz + pw] = (sg[1][2] + sg[2][1]) * 0.5f;
-  }
+  float o[9];
+  fault2wave(in.fm, T1, in.fw, o);
+  float* W = a.Wi0 + pc + i0 * wps;
+#pragma unroll
+  for (int c = 0; c < 9; c++) W[c * pyz] = o[c];
 }
 
 // fault_pre: state_rk (rk4.cu:791-938) + trial_sw (trial_slipweakening.cu:23-732)
@@ -210,114 +250,145 @@ __global__ void __launch_bounds__(256) fault_pre_kernel(FArgs a) {
   long q = j + (long)k * a.nj;
   if (F.united[q]) return;
   const int j1 = j + 3, k1 = k + 3, ny = a.ny;
-  const long nyz = a.nyz, pyz = a.pyz, wps = a.wps, mps = a.mps, pf = j1 + (long)k1 * ny, pv = pf * 3;
+  const long nyz = a.nyz, mps = a.mps, pf = j1 + (long)k1 * ny, pv = pf * 3;
   const long pc = a.jpad + j1 + (long)k1 * a.py;  // volume column
   const int i0 = a.i0;
   const float DH = a.DH, rDH = a.rDH, DT = a.DT, DH2 = DH * DH;
+  float hslip;
   const double RA[4] = {0.5, 0.5, 1.0, 1e10}, RB[4] = {1.0 / 6.0, 1.0 / 3.0, 1.0 / 3.0, 1.0 / 6.0};
   const int irk = a.irk;
   const double rka = RA[irk] * a.DTd, rkb = RB[irk] * a.DTd;
+  // ---- loads: the node's own words first, then the stencils
   float s1[3] = {F.vec_s1[pv], F.vec_s1[pv + 1], F.vec_s1[pv + 2]};
   float s2[3] = {F.vec_s2[pv], F.vec_s2[pv + 1], F.vec_s2[pv + 2]};
+  TailIn tin = load_tail(a, F, q, pf, pc);
+  double st = F.State[q], slip = F.slip[q];
+  double mState = 0.0, tState = 0.0, mslip = 0.0, tslip = 0.0;
+  if (irk != 0) { mState = F.mState[q]; tState = F.tState[q]; mslip = F.mslip[q]; tslip = F.tslip[q]; }
+  double RS_a = 0.0, RS_b = 0.0, RS_L = 0.0, RS_Vw = 0.0;
+  if (a.friction >= 1) { RS_a = F.a[q]; RS_b = F.b[q]; RS_L = F.L[q]; }
+  if (a.friction >= 2) RS_Vw = F.Vw[q];
+  const double tp_p = a.friction >= 1 && F.TP_P ? F.TP_P[q] : 0.0;
+  float T0v[3] = {0.f, 0.f, 0.f}, dT0v[3] = {0.f, 0.f, 0.f};
+  if (a.stress_type == 1) {
+    T0v[0] = F.T0x[q]; T0v[1] = F.T0y[q]; T0v[2] = F.T0z[q];
+    dT0v[0] = F.dT0x[q]; dT0v[1] = F.dT0y[q]; dT0v[2] = F.dT0z[q];
+  }
+  float mu1 = 0.0f, Dc = 0.0f, C0 = 0.0f;
+  if (a.friction == 0) { mu1 = F.str_peak[q]; Dc = F.Dc[q]; C0 = F.C0[q]; }
+  float mdV[3];  // step-start split-node velocity jump
+  for (int c = 0; c < 3; c++) mdV[c] = F.mW[c * 2 * nyz + nyz + pf] - F.mW[c * 2 * nyz + pf];
+  const float T1c[3] = {F.T11[3 * nyz + pf], F.T12[3 * nyz + pf], F.T13[3 * nyz + pf]};
+  // conservative traction on planes i0-+1..3, R and lumped mass
+  const int km = a.nk - k;
+  const int ry = F.rup_index_y[q], rz = F.rup_index_z[q];
+  float Tp[2][3][3];  // [side][distance - 1][component]
+  float rhof[2], jac3[2];
+#pragma unroll
+  for (int m = 0; m < 2; m++) {
+    rhof[m] = F.rho_f[m * nyz + pf];
+    jac3[m] = LMF(a, 9, pc + (i0 + (2 * m - 1) * 3) * mps);  // J of i0-+3, as the reference's inner loop leaves it
+#pragma unroll
+    for (int l = 1; l <= 3; l++) trac(a, a.W, i0 + (2 * m - 1) * l, pc, 0, Tp[m][l - 1]);
+  }
+  float R[2][3], Mr[2], jac_l = 1.f, rho_l = 1.f;
+#pragma unroll
+  for (int m = 0; m < 2; m++) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      float y[7], v[7];
+#pragma unroll
+      for (int l = -3; l <= 3; l++) {
+        y[l + 3] = F.W[(3 + c) * 2 * nyz + m * nyz + pf + l];
+        v[l + 3] = F.W[(6 + c) * 2 * nyz + m * nyz + pf + (long)l * ny];
+      }
+      if (a.freenode && km <= 3) {  // odd image above the surface row
+        if (km == 1) { v[3] = 0.0f; v[4] = -v[2]; v[5] = -v[1]; v[6] = -v[0]; }
+        else if (km == 2) { v[4] = 0.0f; v[5] = -v[3]; v[6] = -v[2]; }
+        else { v[5] = 0.0f; v[6] = -v[4]; }
+      }
+      const float DyT = (ry % 7 ? d22(&y[3], 1, a.FY) : drp(&y[3], 1, a.FY)) * rDH;
+      const float DzT = (rz % 7 ? d22(&v[3], 1, a.FZ) : drp(&v[3], 1, a.FZ)) * rDH;
+      const float r = A1 * Tp[m][0][c] + A2 * Tp[m][1][c] + A3 * Tp[m][2][c];
+      R[m][c] = 0.5f * ((2 * m - 1) * r + (DyT + DzT) * DH) * DH2;
+    }
+    Mr[m] = 0.5f * jac3[m] * rhof[m] * DH * DH2;
+    jac_l = jac3[m]; rho_l = rhof[m];
+  }
 
   // ---- state_rk: slip (and state) RK4 with the current split-node rate
   {
     float dV[3];
-    for (int c = 0; c < 3; c++) dV[c] = F.W[c * 2 * nyz + nyz + pf] - F.W[c * 2 * nyz + pf];
+    for (int c = 0; c < 3; c++) dV[c] = tin.fw[c][1] - tin.fw[c][0];
     float vs1 = dV[0] * s1[0] + dV[1] * s1[1] + dV[2] * s1[2];
     float vs2 = dV[0] * s2[0] + dV[1] * s2[1] + dV[2] * s2[2];
     float hs = sqrtf(vs2 * vs2 + vs1 * vs1);
+    hslip = hs;
     F.hslip[q] = hs;
     double V = fmax((double)hs, 1e-30);
-    double st = F.State[q];
     double hState = 0.0;
     if (a.friction == 1) {
-      double b = F.b[q], L = F.L[q];
-      hState = b * a.V0 / L * (exp((a.f0 - st) / b) - V / a.V0);
+      hState = RS_b * a.V0 / RS_L * (exp((a.f0 - st) / RS_b) - V / a.V0);
     } else if (a.friction >= 2) {
-      double A = F.a[q], b = F.b[q], L = F.L[q], Vw = F.Vw[q];
-      double flv = a.f0 - (b - A) * log(V / a.V0);
-      double fss = a.fw + (flv - a.fw) / pow(1. + pow(V / Vw, 8), 0.125);
+      const double A = RS_a;
+      double flv = a.f0 - (RS_b - A) * log(V / a.V0);
+      double fss = a.fw + (flv - a.fw) / pow(1. + pow(V / RS_Vw, 8), 0.125);
       double psiss = A * (log(sinh(fss / A)) + log(2. * (a.V0 / V)));
-      hState = -V / L * (st - psiss);
+      hState = -V / RS_L * (st - psiss);
     }
     if (irk == 0) {
-      F.mState[q] = st; F.tState[q] = st + rkb * hState;
-      F.mslip[q] = F.slip[q]; F.tslip[q] = F.slip[q] + rkb * hs;
+      mState = st; tState = st + rkb * hState;
+      mslip = slip; tslip = slip + rkb * hs;
+      F.mState[q] = mState; F.tState[q] = tState;
+      F.mslip[q] = mslip; F.tslip[q] = tslip;
     } else if (irk < 3) {
-      F.tState[q] += rkb * hState;
-      F.tslip[q] += rkb * hs;
+      F.tState[q] = tState + rkb * hState;
+      F.tslip[q] = tslip + rkb * hs;
     }
-    if (irk == 3) { F.State[q] = F.tState[q] + rkb * hState; F.slip[q] = F.tslip[q] + rkb * hs; }
-    else { F.State[q] = F.mState[q] + rka * hState; F.slip[q] = F.mslip[q] + rka * hs; }
+    if (irk == 3) { st = tState + rkb * hState; slip = tslip + rkb * hs; }
+    else { st = mState + rka * hState; slip = mslip + rka * hs; }
+    F.State[q] = st;
+    F.slip[q] = slip;
   }
 
-  // ---- trial: conservative traction on planes i0-+1..3, R and lumped mass
-  if (irk == 0) { F.mT11[pf] = F.T11[3 * nyz + pf]; F.mT12[pf] = F.T12[3 * nyz + pf]; F.mT13[pf] = F.T13[3 * nyz + pf]; }
-  const int km = a.nk - k;
-  float R[2][3], Mr[2], jac_l = 1.f, rho_l = 1.f;
-  for (int m = 0; m < 2; m++) {
-    float rho = F.rho_f[m * nyz + pf];
-    float jac = 1.f;
-    for (int l = 1; l <= 3; l++) {
-      const int ii = i0 + (2 * m - 1) * l;
-      jac = LMF(a, 9, pc + ii * mps);
-      float o[3];
-      trac(a, a.W, ii, pc, 0, o);
-      long pl = (3 + (2 * m - 1) * l) * nyz + pf;
-      F.T11[pl] = o[0]; F.T12[pl] = o[1]; F.T13[pl] = o[2];
-    }
-    float DyT[3], DzT[3];
-    for (int c = 0; c < 3; c++) {
-      const float* t2 = &F.W[(3 + c) * 2 * nyz + m * nyz + pf];
-      DyT[c] = (F.rup_index_y[q] % 7 ? d22(t2, 1, a.FY) : drp(t2, 1, a.FY)) * rDH;
-      float v[7];
-      for (int l = -3; l <= 3; l++) v[l + 3] = F.W[(6 + c) * 2 * nyz + m * nyz + pf + (long)l * ny];
-      if (a.freenode && km <= 3) {
-        v[km + 2] = 0.0f;
-        for (int l = km + 3; l < 7; l++) v[l] = -v[2 * (km + 2) - l];
-      }
-      DzT[c] = (F.rup_index_z[q] % 7 ? d22(&v[3], 1, a.FZ) : drp(&v[3], 1, a.FZ)) * rDH;
-    }
-    const float* TT[3] = {F.T11, F.T12, F.T13};
-    for (int c = 0; c < 3; c++) {
-      const float* T = TT[c];
-      float r = m == 0 ? A1 * T[2 * nyz + pf] + A2 * T[1 * nyz + pf] + A3 * T[0 * nyz + pf]
-                       : A1 * T[4 * nyz + pf] + A2 * T[5 * nyz + pf] + A3 * T[6 * nyz + pf];
-      R[m][c] = 0.5f * ((2 * m - 1) * r + (DyT[c] + DzT[c]) * DH) * DH2;
-    }
-    Mr[m] = 0.5f * jac * rho * DH * DH2;  // J of i0-+3, as the reference's inner loop leaves it
-    jac_l = jac; rho_l = rho;
+  // ---- trial
+  if (irk == 0) {
+    F.mT11[pf] = T1c[0]; F.mT12[pf] = T1c[1]; F.mT13[pf] = T1c[2];
+    for (int c = 0; c < 3; c++) tin.mT[c] = T1c[c];
   }
+#pragma unroll
+  for (int m = 0; m < 2; m++)
+#pragma unroll
+    for (int l = 1; l <= 3; l++) {
+      const long pl = (3 + (2 * m - 1) * l) * nyz + pf;
+      F.T11[pl] = Tp[m][l - 1][0]; F.T12[pl] = Tp[m][l - 1][1]; F.T13[pl] = Tp[m][l - 1][2];
+    }
   float t = irk == 0 ? a.it * DT : (irk == 3 ? (a.it + 1) * DT : (a.it + 0.5f) * DT);
-  long pm = pc + i0 * mps;
-  float n[3] = {LMF(a, 0, pm), LMF(a, 1, pm), LMF(a, 2, pm)};
+  float n[3] = {tin.fm.mt[0][0], tin.fm.mt[1][0], tin.fm.mt[2][0]};
   float n0 = sqrtf(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
-  float jacvec = LMF(a, 9, pm) * n0;
+  float jacvec = tin.fm.jac * n0;
   for (int c = 0; c < 3; c++) n[c] /= n0;
-  float dV[3];
-  for (int c = 0; c < 3; c++) dV[c] = F.mW[c * 2 * nyz + nyz + pf] - F.mW[c * 2 * nyz + pf];
+  const float(&dV)[3] = mdV;
   float Tau[3], Tau_n, ratecheck;
   bool ifchange;
   float Trial[3];
   if (a.friction == 0) {
     if (a.stress_type == 1) {
       float Gt = Gt_func(t, a.smooth_load_T);
-      F.str_init_x[q] = F.T0x[q] + Gt * F.dT0x[q];
-      F.str_init_y[q] = F.T0y[q] + Gt * F.dT0y[q];
-      F.str_init_z[q] = F.T0z[q] + Gt * F.dT0z[q];
+      for (int c = 0; c < 3; c++) tin.si[c] = T0v[c] + Gt * dT0v[c];
+      F.str_init_x[q] = tin.si[0]; F.str_init_y[q] = tin.si[1]; F.str_init_z[q] = tin.si[2];
     }
     float den = DH2 * (Mr[0] * A0P - A0M * Mr[1]);
     for (int c = 0; c < 3; c++) Trial[c] = -(Mr[0] * Mr[1] * dV[c] / DT + Mr[0] * R[1][c] - Mr[1] * R[0][c]) / den * 2.0f;
-    float TL[3] = {Trial[0] / jacvec + F.str_init_x[q], Trial[1] / jacvec + F.str_init_y[q], Trial[2] / jacvec + F.str_init_z[q]};
+    float TL[3] = {Trial[0] / jacvec + tin.si[0], Trial[1] / jacvec + tin.si[1], Trial[2] / jacvec + tin.si[2]};
     float Tn_ = TL[0] * n[0] + TL[1] * n[1] + TL[2] * n[2];
     float Ts[3] = {TL[0] - n[0] * Tn_, TL[1] - n[1] * Tn_, TL[2] - n[2] * Tn_};
     float Ts0 = sqrtf(Ts[0] * Ts[0] + Ts[1] * Ts[1] + Ts[2] * Ts[2]);
     ifchange = false;
     if (Tn_ >= 0.0f) { Tau_n = 0.0f; ifchange = true; } else Tau_n = Tn_;
-    float mu1 = F.str_peak[q], sl = (float)F.slip[q], Dc = F.Dc[q];
+    float sl = (float)slip;
     float fr = sl <= Dc ? mu1 - (mu1 - a.mu_d) * sl / Dc : a.mu_d;
-    float Tau_c = -fr * Tau_n + F.C0[q];
+    float Tau_c = -fr * Tau_n + C0;
     float Tau_s;
     if (Ts0 >= Tau_c) { Tau_s = Tau_c; F.flag_rup[q] = 1; ifchange = true; }
     else { Tau_s = Ts0; F.flag_rup[q] = 0; }
@@ -327,7 +398,7 @@ __global__ void __launch_bounds__(256) fault_pre_kernel(FArgs a) {
     } else {
       for (int c = 0; c < 3; c++) Tau[c] = TL[c];
     }
-    ratecheck = F.hslip[q];
+    ratecheck = hslip;
   } else {
     // rate-and-state with the hard-coded nucleation unless stresses are read
     float y1 = (float)(j - a.NY / 2);
@@ -335,15 +406,10 @@ __global__ void __launch_bounds__(256) fault_pre_kernel(FArgs a) {
     float r = sqrtf(y1 * y1 + z1 * z1) * DH;
     float Gt = Gt_func(t, a.smooth_load_T);
     float Fr = Fr_func(r, 3.0e3f);
-    F.str_init_x[q] = -120e6f;
-    F.str_init_y[q] = -25e6f * Fr * Gt + -75e6f;
-    F.str_init_z[q] = 0.0f;
-    if (a.stress_type == 1) {
-      F.str_init_x[q] = F.T0x[q] + Gt * F.dT0x[q];
-      F.str_init_y[q] = F.T0y[q] + Gt * F.dT0y[q];
-      F.str_init_z[q] = F.T0z[q] + Gt * F.dT0z[q];
-    }
-    float T0[3] = {F.str_init_x[q], F.str_init_y[q], F.str_init_z[q]};
+    float T0[3] = {-120e6f, -25e6f * Fr * Gt + -75e6f, 0.0f};
+    if (a.stress_type == 1)
+      for (int c = 0; c < 3; c++) T0[c] = T0v[c] + Gt * dT0v[c];
+    F.str_init_x[q] = T0[0]; F.str_init_y[q] = T0[1]; F.str_init_z[q] = T0[2];
     double dn[3] = {n[0], n[1], n[2]}, ds1[3] = {s1[0], s1[1], s1[2]}, ds2[3] = {s2[0], s2[1], s2[2]};
     double T0l[3] = {dn[0] * T0[0] + dn[1] * T0[1] + dn[2] * T0[2], ds1[0] * T0[0] + ds1[1] * T0[1] + ds1[2] * T0[2],
                      ds2[0] * T0[0] + ds2[1] * T0[1] + ds2[2] * T0[2]};
@@ -366,11 +432,10 @@ __global__ void __launch_bounds__(256) fault_pre_kernel(FArgs a) {
     Tt[2] = T0l[2] - 2.0 * (M0 * M1 * Rl[2] / dt1 + M0 * R3[1] - M1 * R3[0]) / den;
     double cc = -((double)A0P - (double)A0M) * dt1 * jacvec / ((double)jac_l * rho_l * DH);
     double Vt1 = cc * Tt[1], Vt2 = cc * Tt[2];
-    double st = F.State[q], RS_a = F.a[q];
     double Tau_nd = Tt[0] >= -1e-1 ? -1e-1 : Tt[0];
     // thermal pressurization: the fault's pore pressure makes the normal
     // stress effective for the solve and the strength (trial_ratestate.cu:636-644)
-    if (F.TP_P) Tau_nd += F.TP_P[q];
+    if (F.TP_P) Tau_nd += tp_p;
     double coef = cc * RS_a * fabs(Tau_nd);
     double Vtn = sqrt(Vt1 * Vt1 + Vt2 * Vt2);
     double Ttn = sqrt(Tt[1] * Tt[1] + Tt[2] * Tt[2]);
@@ -398,7 +463,7 @@ __global__ void __launch_bounds__(256) fault_pre_kernel(FArgs a) {
     Cf[7 * n2 + q] = (float)log10(fmax(Rn, 1e-30));
     return;
   }
-  fault_tail(a, F, q, pf, pc, Tau, Tau_n, ifchange, ratecheck, Trial, jacvec, s1, s2);
+  fault_tail(a, F, q, pf, pc, tin, Tau, Tau_n, ifchange, ratecheck, Trial, jacvec, s1, s2);
 }
 
 // Rate-and-state trial after the hand-over from fault_pre_kernel
@@ -451,6 +516,8 @@ __global__ void __launch_bounds__(256) fault_rs_kernel(FArgs a) {
   // total one (trial_ratestate.cu:785-788)
   const double Tau_eff = C[5 * n2 + q], Tt1 = C[6 * n2 + q], Tt2 = C[7 * n2 + q];
   const double Tau_nd = F.TP_P ? Tau_eff - F.TP_P[q] : Tau_eff;
+  unsigned counts[5];
+  for (int c = 0; c < 5; c++) counts[c] = F.newton_stats[c * n2 + q];
   double Ttn = C[8 * n2 + q];
   const float n[3] = {Cf[q], Cf[n2 + q], Cf[2 * n2 + q]};
   const float jacvec = Cf[3 * n2 + q];
@@ -458,11 +525,12 @@ __global__ void __launch_bounds__(256) fault_rs_kernel(FArgs a) {
   const long pf = j1 + (long)k1 * a.ny, pv = pf * 3, pc = a.jpad + j1 + (long)k1 * a.py;
   const float s1[3] = {F.vec_s1[pv], F.vec_s1[pv + 1], F.vec_s1[pv + 2]};
   const float s2[3] = {F.vec_s2[pv], F.vec_s2[pv + 1], F.vec_s2[pv + 2]};
-  F.newton_stats[q] += 1u;  // per-node counters: no contention between nodes
-  F.newton_stats[n2 + q] += (unsigned)iters;
-  F.newton_stats[2 * n2 + q] += fb ? 1u : 0u;
-  F.newton_stats[3 * n2 + q] += x0 != x_plain ? 1u : 0u;  // started from the learned guess
-  F.newton_stats[4 * n2 + q] += consulted ? 1u : 0u;      // its wave evaluated the network
+  const TailIn tin = load_tail(a, F, q, pf, pc);
+  F.newton_stats[q] = counts[0] + 1u;  // per-node counters: no contention between nodes
+  F.newton_stats[n2 + q] = counts[1] + (unsigned)iters;
+  F.newton_stats[2 * n2 + q] = counts[2] + (fb ? 1u : 0u);
+  F.newton_stats[3 * n2 + q] = counts[3] + (x0 != x_plain ? 1u : 0u);  // started from the learned guess
+  F.newton_stats[4 * n2 + q] = counts[4] + (consulted ? 1u : 0u);      // its wave evaluated the network
   const double RS_V0 = 1e-6;
   float V = (float)(2.0 * RS_V0 * exp(-st / RS_a) * sinh(xnew));
   const double Tm = RS_a * xnew * fabs(Tau_eff);
@@ -472,10 +540,10 @@ __global__ void __launch_bounds__(256) fault_rs_kernel(FArgs a) {
   V = fmaxf(V, 1e-30f);
   float Tau[3];
   for (int c = 0; c < 3; c++) Tau[c] = (float)(Tau_nd * (double)n[c] + Ts1 * (double)s1[c] + Ts2 * (double)s2[c]);
-  Tau[0] = F.str_init_x[q];  // trial_ratestate.cu:797
+  Tau[0] = tin.si[0];  // trial_ratestate.cu:797
   const float Tau_n = Tau[0] * n[0] + Tau[1] * n[1] + Tau[2] * n[2];
   const float Trial[3] = {0.0f, 0.0f, 0.0f};
-  fault_tail(a, F, q, pf, pc, Tau, Tau_n, true, V, Trial, jacvec, s1, s2);
+  fault_tail(a, F, q, pf, pc, tin, Tau, Tau_n, true, V, Trial, jacvec, s1, s2);
 }
 
 __device__ __forceinline__ void mv3(const float* A, const float* x, float* y) {
@@ -537,11 +605,10 @@ __device__ __forceinline__ float dxv_off(const FArgs& a, int nn, int c, long pc,
 // (G 0: 0-5, 1: 6-11, 2: 12-15) is a kernel of its own, so that the
 // registers of the split-node stress part do not set the occupancy of the
 // others.
-constexpr int kDerivGroupBase[3] = {0, 6, 12}, kDerivGroupParts[3] = {6, 6, 4};
-template <int G>
+constexpr int kDerivParts = 16;
 __global__ void __launch_bounds__(256) fault_deriv_kernel(FArgs a, int tiles_j, int items) {
   const int item = xcd_remap((int)blockIdx.x, items);
-  const int part = kDerivGroupBase[G] + item % kDerivGroupParts[G], tile = item / kDerivGroupParts[G];
+  const int part = item % kDerivParts, tile = item / kDerivParts;
   int j = (tile % tiles_j) * 64 + threadIdx.x;
   int k = (tile / tiles_j) * 4 + threadIdx.y;
   if (j >= a.nj || k >= a.nk) return;
@@ -559,7 +626,7 @@ __global__ void __launch_bounds__(256) fault_deriv_kernel(FArgs a, int tiles_j, 
   float* slab = a.slabH;
   auto slabx = [&](int i, int c) -> float& { return slab[(long)(i - (i0 - 3)) * 9 * pyz + c * pyz + pc]; };
 
-  if (G == 0) {  // velocity rates at i0-3..-1, +1..+3 (fault_dvelo.cu:153-255)
+  if (part < 6) {  // velocity rates at i0-3..-1, +1..+3 (fault_dvelo.cu:153-255)
     const int i = i0 + (part < 3 ? part - 3 : part - 2);
     {
       // the three axes one after another, each array indexed with constants
@@ -615,7 +682,7 @@ __global__ void __launch_bounds__(256) fault_deriv_kernel(FArgs a, int tiles_j, 
     }
     return;
   }
-  if (G == 1) {  // off-fault stress rates (fault_dstrs_f.cu:1009-1250)
+  if (part < 12) {  // off-fault stress rates (fault_dstrs_f.cu:1009-1250)
     const int nn = part < 9 ? part - 6 : part - 4;
     {
       const int l = nn < 4 ? nn - 3 : nn - 4;
@@ -650,7 +717,7 @@ __global__ void __launch_bounds__(256) fault_deriv_kernel(FArgs a, int tiles_j, 
     }
     return;
   }
-  if (part < 14) {  // G 2: split-node velocity rates of side part-12 (fault_dvelo.cu:260-385)
+  if (part < 14) {  // split-node velocity rates of side part-12 (fault_dvelo.cu:260-385)
     const int m = part - 12;
     const float* TT[3] = {F.T11, F.T12, F.T13};
     float rrj = 1.0f / (F.rho_f[m * nyz + pf] * LMF(a, 9, pc + i0 * mps));
@@ -775,76 +842,76 @@ __global__ void __launch_bounds__(256) fault_post_kernel(FArgs a) {
     int ip = i0 - 3 + pl;
     const long p = pc + ip * wps;
     float damp = a.cerjan ? fminf(a.cj[0][ip], dampj) : 1.0f;
+    float h[9], w0[9], sv[9], tv[9];
+#pragma unroll
     for (int c = 0; c < 9; c++) {
-      long x = c * pyz + p;
-      float h = a.slabH[(long)pl * 9 * pyz + c * pyz + pc];
-      float w = rk_combine(irk, rka, rkb, a.Win[x], h, a.S, a.T, x);
-      a.Wi0[x] = w * damp;
+      const long x = c * pyz + p;
+      h[c] = a.slabH[(long)pl * 9 * pyz + c * pyz + pc];
+      w0[c] = irk == 0 ? a.Win[x] : 0.0f;
+      sv[c] = irk == 1 || irk == 2 ? a.S[x] : 0.0f;
+      tv[c] = irk != 0 ? a.T[x] : 0.0f;
+    }
+#pragma unroll
+    for (int c = 0; c < 9; c++) {
+      const long x = c * pyz + p;
+      a.Wi0[x] = rk_words(irk, rka, rkb, w0[c], h[c], sv[c], tv[c]) * damp;
+      if (irk != 3) a.T[x] = tv[c];
     }
     return;
   }
   float s1[3] = {F.vec_s1[pv], F.vec_s1[pv + 1], F.vec_s1[pv + 2]};
   float s2[3] = {F.vec_s2[pv], F.vec_s2[pv + 1], F.vec_s2[pv + 2]};
   bool uni = F.united[q] != 0;
+  float fw[9][2], fh[9][2], fm[9][2], ft[9][2];
+#pragma unroll
+  for (int c = 0; c < 9; c++)
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+      const long x = c * 2 * nyz + m * nyz + pf;
+      fw[c][m] = F.W[x];
+      fh[c][m] = F.hW[x];
+      fm[c][m] = irk == 1 || irk == 2 ? F.mW[x] : 0.0f;
+      ft[c][m] = irk != 0 ? F.tW[x] : 0.0f;
+    }
+  const FaultMetric met = load_fault_metric(a, pc + i0 * mps);
+  const float T1[3] = {F.T11[3 * nyz + pf], F.T12[3 * nyz + pf], F.T13[3 * nyz + pf]};
+  const float tT[3] = {F.tTs1[q], F.tTs2[q], F.tTn[q]};
+  float Ts[3] = {0.0f, 0.0f, 0.0f};
+  if (irk != 0) { Ts[0] = F.Ts1[q]; Ts[1] = F.Ts2[q]; Ts[2] = F.Tn[q]; }
   if (!uni) {
     float vis = a.viscosity * (float)a.DTd;
-    for (int m = 0; m < 2; m++)
-      for (int c = 0; c < 9; c++) {
-        long x = c * 2 * nyz + m * nyz + pf;
-        float h = F.hW[x];
-        float w0 = F.W[x];
-        if (irk == 0) F.mW[x] = w0;
-        float w = rk_combine(irk, rka, rkb, w0, h, F.mW, F.tW, x);
+#pragma unroll
+    for (int c = 0; c < 9; c++)
+#pragma unroll
+      for (int m = 0; m < 2; m++) {
+        const long x = c * 2 * nyz + m * nyz + pf;
+        const float h = fh[c][m];
+        if (irk == 0) F.mW[x] = fw[c][m];
+        float w = rk_words(irk, rka, rkb, fw[c][m], h, fm[c][m], ft[c][m]);
+        if (irk != 3) F.tW[x] = ft[c][m];
         if (c >= 3) w += vis * h;
         F.W[x] = w;
+        fw[c][m] = w;
       }
   }
   float dV[3];
-  for (int c = 0; c < 3; c++) dV[c] = F.W[c * 2 * nyz + nyz + pf] - F.W[c * 2 * nyz + pf];
+  for (int c = 0; c < 3; c++) dV[c] = fw[c][1] - fw[c][0];
   float vs1 = dV[0] * s1[0] + dV[1] * s1[1] + dV[2] * s1[2];
   float vs2 = dV[0] * s2[0] + dV[1] * s2[1] + dV[2] * s2[2];
   F.hslip[q] = sqrtf(vs2 * vs2 + vs1 * vs1);
   F.Vs1[q] = vs1;
   F.Vs2[q] = vs2;
   float rkb1 = (float)(RB[irk]);
-  if (irk == 0) { F.Ts1[q] = rkb1 * F.tTs1[q]; F.Ts2[q] = rkb1 * F.tTs2[q]; F.Tn[q] = rkb1 * F.tTn[q]; }
-  else { F.Ts1[q] += rkb1 * F.tTs1[q]; F.Ts2[q] += rkb1 * F.tTs2[q]; F.Tn[q] += rkb1 * F.tTn[q]; }
+  if (irk == 0) { F.Ts1[q] = rkb1 * tT[0]; F.Ts2[q] = rkb1 * tT[1]; F.Tn[q] = rkb1 * tT[2]; }
+  else { F.Ts1[q] = Ts[0] + rkb1 * tT[0]; F.Ts2[q] = Ts[1] + rkb1 * tT[1]; F.Tn[q] = Ts[2] + rkb1 * tT[2]; }
   if (uni) return;
   // fault2wave into the stage output at i0
-  const long p = pc + i0 * mps, pw = pc + i0 * wps;
-  float mt[3][3] = {{LMF(a, 0, p), LMF(a, 3, p), LMF(a, 6, p)},
-                    {LMF(a, 1, p), LMF(a, 4, p), LMF(a, 7, p)},
-                    {LMF(a, 2, p), LMF(a, 5, p), LMF(a, 8, p)}};
-  float rj = 1.0f / LMF(a, 9, p);
-  float inv[3][3];
-  inv[0][0] = mt[1][1] * mt[2][2] - mt[2][1] * mt[1][2];
-  inv[0][1] = mt[2][1] * mt[0][2] - mt[0][1] * mt[2][2];
-  inv[0][2] = mt[0][1] * mt[1][2] - mt[0][2] * mt[1][1];
-  inv[1][0] = mt[1][2] * mt[2][0] - mt[1][0] * mt[2][2];
-  inv[1][1] = mt[0][0] * mt[2][2] - mt[2][0] * mt[0][2];
-  inv[1][2] = mt[1][0] * mt[0][2] - mt[0][0] * mt[1][2];
-  inv[2][0] = mt[1][0] * mt[2][1] - mt[1][1] * mt[2][0];
-  inv[2][1] = mt[2][0] * mt[0][1] - mt[0][0] * mt[2][1];
-  inv[2][2] = mt[0][0] * mt[1][1] - mt[0][1] * mt[1][0];
-  float det = 1.0f / (inv[0][0] * mt[0][0] + inv[0][1] * mt[1][0] + inv[0][2] * mt[2][0]);
-  float tr[3][3];
-  tr[0][0] = F.T11[3 * nyz + pf]; tr[1][0] = F.T12[3 * nyz + pf]; tr[2][0] = F.T13[3 * nyz + pf];
-  for (int c = 0; c < 3; c++) {
-    tr[c][1] = (F.W[(3 + c) * 2 * nyz + pf] + F.W[(3 + c) * 2 * nyz + nyz + pf]) * 0.5f;
-    tr[c][2] = (F.W[(6 + c) * 2 * nyz + pf] + F.W[(6 + c) * 2 * nyz + nyz + pf]) * 0.5f;
-  }
-  float sg[3][3];
-  for (int r = 0; r < 3; r++)
-    for (int cc = 0; cc < 3; cc++) sg[r][cc] = (tr[r][0] * inv[0][cc] + tr[r][1] * inv[1][cc] + tr[r][2] * inv[2][cc]) * det * rj;
   float damp = a.cerjan ? fminf(a.cj[0][i0], dampj) : 1.0f;
-  float* W = a.Wi0;
-  for (int c = 0; c < 3; c++) W[c * pyz + pw] = (F.W[c * 2 * nyz + pf] + F.W[c * 2 * nyz + nyz + pf]) * 0.5f * damp;
-  W[3 * pyz + pw] = sg[0][0] * damp;
-  W[4 * pyz + pw] = sg[1][1] * damp;
-  W[5 * pyz + pw] = sg[2][2] * damp;
-  W[6 * pyz + pw] = (sg[0][1] + sg[1][0]) * 0.5f * damp;
-  W[7 * pyz + pw] = (sg[0][2] + sg[2][0]) * 0.5f * damp;
-  W[8 * pyz + pw] = (sg[1][2] + sg[2][1]) * 0.5f * damp;
+  float o[9];
+  fault2wave(met, T1, fw, o);
+  float* W = a.Wi0 + pc + i0 * wps;
+#pragma unroll
+  for (int c = 0; c < 9; c++) W[c * pyz] = o[c] * damp;
 }
 
 // cal_rup_sensor_D_cu / cal_rup_sensor_magn_cu (rup_sensor.cu:7-86).
@@ -1084,13 +1151,8 @@ void launch_fault_deriv(Ctx& c, const float* Win, int fx, int fy, int fz) {
   c.prof.begin(c.stream, PK_FAULT_DERIV);
   const dim3 g = fgrid(c);
   const int tiles = (int)(g.x * g.y);
-  // per-plane velocity parts, per-plane stress parts, split-node parts of each tile
-  hipLaunchKernelGGL(fault_deriv_kernel<0>, dim3(tiles * kDerivGroupParts[0]), dim3(64, 4, 1), 0, c.stream, a, (int)g.x,
-                     tiles * kDerivGroupParts[0]);
-  hipLaunchKernelGGL(fault_deriv_kernel<1>, dim3(tiles * kDerivGroupParts[1]), dim3(64, 4, 1), 0, c.stream, a, (int)g.x,
-                     tiles * kDerivGroupParts[1]);
-  hipLaunchKernelGGL(fault_deriv_kernel<2>, dim3(tiles * kDerivGroupParts[2]), dim3(64, 4, 1), 0, c.stream, a, (int)g.x,
-                     tiles * kDerivGroupParts[2]);
+  hipLaunchKernelGGL(fault_deriv_kernel, dim3(tiles * kDerivParts), dim3(64, 4, 1), 0, c.stream, a, (int)g.x,
+                     tiles * kDerivParts);
   c.prof.end(c.stream);
 }
 
