@@ -296,17 +296,17 @@ __global__ void __launch_bounds__(256) fault_pre_kernel(FArgs a) {
   for (int m = 0; m < 2; m++) {
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      float y[7], v[7];
+      const float* tz = F.W + (6 + c) * 2 * nyz + m * nyz + pf;
+      const float z0 = tz[-3L * ny], z1 = tz[-2L * ny], z2 = tz[-1L * ny], z3 = tz[0], z4 = tz[ny], z5 = tz[2L * ny], z6 = tz[3L * ny];
+      // odd image above the surface row, by selects: as a branch per row
+      // (1, 2, else) the compiler of ROCm 7.2 left the last word of the third
+      // unset
+      const int im = a.freenode && km <= 3 ? km : 0;
+      const float v[7] = {z0, z1, z2, im == 1 ? 0.0f : z3, im == 1 ? -z2 : im == 2 ? 0.0f : z4,
+                          im == 1 ? -z1 : im == 2 ? -z3 : im == 3 ? 0.0f : z5, im == 1 ? -z0 : im == 2 ? -z2 : im == 3 ? -z4 : z6};
+      float y[7];
 #pragma unroll
-      for (int l = -3; l <= 3; l++) {
-        y[l + 3] = F.W[(3 + c) * 2 * nyz + m * nyz + pf + l];
-        v[l + 3] = F.W[(6 + c) * 2 * nyz + m * nyz + pf + (long)l * ny];
-      }
-      if (a.freenode && km <= 3) {  // odd image above the surface row
-        if (km == 1) { v[3] = 0.0f; v[4] = -v[2]; v[5] = -v[1]; v[6] = -v[0]; }
-        else if (km == 2) { v[4] = 0.0f; v[5] = -v[3]; v[6] = -v[2]; }
-        else { v[5] = 0.0f; v[6] = -v[4]; }
-      }
+      for (int l = -3; l <= 3; l++) y[l + 3] = F.W[(3 + c) * 2 * nyz + m * nyz + pf + l];
       const float DyT = (ry % 7 ? d22(&y[3], 1, a.FY) : drp(&y[3], 1, a.FY)) * rDH;
       const float DzT = (rz % 7 ? d22(&v[3], 1, a.FZ) : drp(&v[3], 1, a.FZ)) * rDH;
       const float r = A1 * Tp[m][0][c] + A2 * Tp[m][1][c] + A3 * Tp[m][2][c];
