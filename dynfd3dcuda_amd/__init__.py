@@ -369,11 +369,11 @@ class Solver:
     def profile_aux(self):
         """{kernel class: (ADE-PML (point, face) pairs whose auxiliary value
         one launch reads for the stage, pairs whose auxiliary ODE step it
-        takes)} for the classes with such work."""
+        takes)} for pml_aux and the classes with such work."""
         out = {}
         for name in PROFILE_KERNELS:
             rd, up = ctypes.c_long(), ctypes.c_long()
             self._check(self.lib.cgfdm_profile_aux(self.h, name.encode(), ctypes.byref(rd), ctypes.byref(up)))
-            if rd.value or up.value:
+            if rd.value or up.value or name == "pml_aux":
                 out[name] = (rd.value, up.value)
         return out

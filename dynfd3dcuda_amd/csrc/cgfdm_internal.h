@@ -64,6 +64,7 @@ struct Params {
   int WaveBandIChunk = 0;  // planes per block of the band tiles (0: automatic)
   int WaveTopIChunk = 0;  // planes per block of the free-surface tiles (0: automatic)
   int WaveSurfaceTiles = 1;  // free-surface tiles = the top TK rows, own line-aligned j tiles (0: earlier layout)
+  int WaveUnified = -1;  // 1: one launch of tiles of any kind per stage; 0: one per kind; -1: 1 on small grids
   int WaveBandRound = 0;  // 1: low j band rounded up to whole 64-wide tiles (0: band width exactly)
 
   // derived (set_params.cu:286-295)
@@ -99,6 +100,8 @@ struct Dims {
 // First column of the interior box of the stage kernel (the absorbing band
 // below it is handled by the edge instantiation).
 int interior_lo_j(const Params& p);
+bool wave_unified(const Params& p);
+constexpr double kUnifiedPoints = 12e6;
 
 // Fault state on the device (2-D arrays [nk][nj] unless noted).
 struct FaultDev {
@@ -210,6 +213,7 @@ struct Ctx {
   float* trac_top = nullptr;    // free surface: traction vectors of the six top rows [nx][6][9][ny]
   float* img_top = nullptr;     // free surface: image velocity RHS of the three top rows [3][3][ni][nj]
   int wave_nwork = 0;                  // all work items
+  bool wave_unified = false;        // one launch of tiles of any kind (WaveUnified)
   bool wave_tall = false;           // interior tiles 64 x 16 (WaveTallInterior)
   bool wave_pipe = false;           // pipelined interior kernel (WaveInteriorKernel)
   bool wave_ring = false;           // its LDS plane ring (WaveInteriorKernel 1)

@@ -2,6 +2,7 @@
 // the interior box, absorbing-band and free-surface tiles of one RK stage,
 // the XCD-contiguous block numbering, and the per-stage launch.
 #include "wave_stage_kernels.h"
+#include <cmath>
 
 namespace cgfdm {
 using namespace wave;
@@ -83,9 +84,86 @@ const char* const kProfNames[PK_COUNT] = {"stage_interior", "stage_band", "stage
 // columns between the band and this edge are then plain points, which the
 // band kernel treats like the interior one.
 int interior_lo_j(const Params& p) {
+  if (wave_unified(p)) return 0;  // tiles from the first column on
   const int band = std::max(p.usePML ? p.PML_N : 0, p.useCerjan ? p.DAMP_N : 0);
   if (p.WaveBandRound == 0) return band;
   return (band + TJ - 1) / TJ * TJ;
+}
+
+// Uploads a work list (two int4 per block).
+static int put_work(Ctx& c, const std::vector<int4>& all) {
+  if (c.wave_work) { (void)hipFree(c.wave_work); c.wave_work = nullptr; }
+  if (hipMalloc(&c.wave_work, all.size() * sizeof(int4)) != hipSuccess) return 1;
+  if (hipMemcpy(c.wave_work, all.data(), all.size() * sizeof(int4), hipMemcpyHostToDevice) != hipSuccess) return 1;
+  c.wave_nwork = (int)all.size() / 2;
+  return 0;
+}
+
+// The work list of the unified launch: 64 x 4 tiles over the whole grid, in
+// chunks of planes.
+static int unified_work(Ctx& c) {
+  const Params& p = c.p;
+  const int ni = c.d.ni, nj = c.d.nj, nk = c.d.nk;
+  c.wave_tall = c.wave_pipe = c.wave_ring = c.wave_band_pipe = c.wave_surf_pipe = false;
+  c.pml_fused = true;
+  c.wave_ktop = nk;
+  const long tiles = (long)((nj + TJ - 1) / TJ) * ((nk + TK4 - 1) / TK4);
+  int cus = 0, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    cus = 256;
+  int len = p.WaveBandIChunk;
+  if (len <= 0) {
+    // planes per block: a block takes about its planes and one more for its
+    // start, the launch its blocks spread over the resident ones (two per CU)
+    // and the last of them; shorter chunks for grids that would leave CUs
+    // idle (97 x 125 x 81: 3 planes, 0.42 ms of tiles per step against 0.68
+    // with 20; 151 x 211 x 133: 7 planes, 1.79 against 2.26)
+    double best = 0.0;
+    for (int n = std::min(ni, 2); n <= std::min(ni, 20); n++) {
+      const double t = (n + 1.0) * ((double)tiles * ((ni + n - 1) / n) / (2.0 * cus) + 1.0);
+      if (len <= 0 || t < best) { best = t; len = n; }
+    }
+  }
+  std::vector<int4> all;
+  for (int i0 = 0; i0 < ni; i0 += len)
+    for (int k0 = 0; k0 < nk; k0 += TK4)
+      for (int j0 = 0; j0 < nj; j0 += TJ) {
+        all.push_back(make_int4(j0, k0, i0, std::min(ni, i0 + len)));
+        all.push_back(make_int4(std::min(TJ, nj - j0), std::min((int)TK4, nk - k0), 0, 0));
+      }
+  for (int l = 0; l < 4; l++) c.wave_nkind[l] = 0;
+  c.wave_nkind[1] = (int)all.size() / 2;
+  const long N = c.pml.N;
+  long pairs = 0;
+  for (int f = 0; f < 6; f++)
+    if (c.pml.on[f]) pairs += N * (f < 2 ? (long)nj * nk : f < 4 ? (long)ni * nk : (long)ni * nj);
+  for (int kd = 0; kd < 3; kd++) c.wave_points[kd] = kd == 1 ? (long)ni * nj * nk : 0;
+  for (int kd = 0; kd < 4; kd++) c.aux_read_pairs[kd] = c.aux_update_pairs[kd] = kd == 1 ? pairs : 0;
+  c.pml_nbox = c.pml_blocks = 0;
+  return put_work(c, all);
+}
+
+// True when the two ADE-PML bands of every axis are disjoint (2 N <= the axis
+// length), which the pipelined kernels' one face per axis and point needs.
+static bool bands_disjoint(const Params& p) {
+  if (!p.usePML) return true;
+  return 2 * p.PML_N <= p.NX && 2 * p.PML_N <= p.NY && (p.FreeSurface || 2 * p.PML_N <= p.NZ);
+}
+
+// One launch of tiles of any kind (the FULL form of the pipelined kernel)
+// instead of one per kind: WaveUnified 1, or -1 (default) on grids of at most
+// kUnifiedPoints points without any of the per-kind launch options.  On small
+// grids each launch of one kind leaves most of the chip idle while its longest
+// block runs, and they run one after another: per step 1.26 -> 0.25 ms at
+// 30 x 80 x 50, 1.52 -> 0.41 at 97 x 125 x 81, 1.31 -> 0.65 at 100 x 200 x 100,
+// 3.00 -> 2.34 at 251 x 187 x 143.  At 400 x 300 x 200 both are level (6.5 ms),
+// and the launches of one kind keep their own tile shapes.
+bool wave_unified(const Params& p) {
+  if (p.WaveUnified == 0 || !bands_disjoint(p)) return false;
+  if (p.WaveInteriorKernel != -1 || p.WaveBandKernel != -1 || p.WaveSurfaceKernel != 1 || p.WaveSurfaceTiles != 1 ||
+      p.WaveTallInterior || p.WaveBandRound || !p.PmlAuxFused || p.StageStreams || p.WaveIChunk || p.WaveTopIChunk)
+    return false;
+  return p.WaveUnified > 0 || (double)p.NX * p.NY * p.NZ <= kUnifiedPoints;
 }
 
 // Builds the stage-kernel work lists and allocates the free-surface buffers.  The interior box excludes every face band where a PML profile or
@@ -104,6 +182,8 @@ int upload_wave_work(Ctx& c) {
 
   const Params& p = c.p;
   const int n3[3] = {c.d.ni, c.d.nj, c.d.nk};
+  c.wave_unified = wave_unified(p);
+  if (c.wave_unified) return unified_work(c);
   const bool freenode = p.FreeSurface != 0;
   int lo[3], hi[3];
   for (int ax = 0; ax < 3; ax++) {
@@ -146,10 +226,7 @@ int upload_wave_work(Ctx& c) {
   // WaveBandKernel 1: the pipelined kernel on the band tiles too, which adds
   // the aux terms of one face per axis: used when the two ADE-PML bands of
   // every axis are disjoint (2 N <= the axis length)
-  bool disjoint = true;
-  for (int ax = 0; ax < 3; ax++)
-    if (c.pml.on[2 * ax] && c.pml.on[2 * ax + 1] && 2 * c.pml.N > (ax == 0 ? c.d.ni : ax == 1 ? c.d.nj : c.d.nk))
-      disjoint = false;
+  const bool disjoint = bands_disjoint(p);
   // -1 (automatic): 64 x 4 band tiles beside the 64 x 4 interior tiles of a
   // large grid, 64 x 8 ones on a grid too small for those (400 x 300 x 200:
   // bands 3.28 against 3.35 ms per step)
@@ -354,11 +431,7 @@ int upload_wave_work(Ctx& c) {
     all.insert(all.end(), lists[l].begin(), lists[l].end());
     c.wave_nkind[l] = (int)lists[l].size() / 2;
   }
-  if (c.wave_work) { (void)hipFree(c.wave_work); c.wave_work = nullptr; }
-  if (hipMalloc(&c.wave_work, all.size() * sizeof(int4)) != hipSuccess) return 1;
-  if (hipMemcpy(c.wave_work, all.data(), all.size() * sizeof(int4), hipMemcpyHostToDevice) != hipSuccess) return 1;
-  c.wave_nwork = (int)all.size() / 2;
-  return 0;
+  return put_work(c, all);
 }
 
 void launch_wave_stage(Ctx& c, const StageBufs& b, int irk, int fx, int fy, int fz, bool rhs_only, float* rhs_out) {

@@ -624,10 +624,16 @@ __device__ __forceinline__ float met_raw_get(const uint32_t (&w)[met_raw_n<MT>()
 // two bands of an axis do not overlap), and added after the three axis sums
 // in the general kernel's order; 1/beta and the sponge factor of plane i+1
 // are fetched during plane i.
+//
+// FULL (with BAND and TOP): tiles of any kind in one launch, every auxiliary
+// field of their points advanced here: also those of the free-surface rows
+// and, after the point's stage value is stored, of the edges of the absorbing
+// box, face by face.
 template <int FX, int FY, int FZ, class MT, int TJ_, int NT_, int MINB, bool BAND = false, bool RING = true,
-          bool TOP = false>
+          bool TOP = false, bool FULL = false>
 __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a) {
   static_assert(!TOP || (BAND && TJ_ == 64), "free-surface tiles: band terms, one k row per wavefront");
+  static_assert(!FULL || TOP, "tiles of any kind");
   constexpr int TJ = TJ_, TK = NT_ / TJ_;
   constexpr int LJ = TJ + 4, LK = TK + 4;
   // halo cells of one plane: the 4 k-halo rows over the tile's own columns
@@ -861,7 +867,7 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
       if (pml) {
         if (a.cold.on[0] && i < N) { inx = true; pix = i; }
         else if (a.cold.on[1] && i >= ni - N) { inx = true; pix = i - (ni - N) + xoff1; }
-        const bool fuse = !TOP && a.aux_fused && !a.rhs_only;
+        const bool fuse = (FULL || !TOP) && a.aux_fused && !a.rhs_only;
         const bool need_t = fuse && irk >= 2, need_s = fuse && (irk == 1 || irk == 2);  // stage 1 derives the accumulator
         if (inx) {
           fuse1 = fuse && act && !injl && !inkl;
@@ -914,6 +920,58 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
       auto Dz = [&](int c) {
         return FZ > 0 ? drp5<1>(L[c][lk - 1][lj], L[c][lk][lj], L[c][lk + 1][lj], L[c][lk + 2][lj], L[c][lk + 3][lj])
                       : drp5<-1>(L[c][lk - 3][lj], L[c][lk - 2][lj], L[c][lk - 1][lj], L[c][lk][lj], L[c][lk + 1][lj]);
+      };
+      // one step of the auxiliary ODE of the lane's point on its face along
+      // axis AX (values y, step start s, accumulator t), stored through `on`
+      auto advance = [&](auto AX, auto D, const float(&y)[9], const float(&s)[9], float(&t)[9], auto on) {
+        constexpr int ax = decltype(AX)::value;
+        const float rka = a.rka, rkb = a.rkb;
+        const float e0 = ax == 0 ? xix : ax == 1 ? etx : ztx;
+        const float e1 = ax == 0 ? xiy : ax == 1 ? ety : zty;
+        const float e2 = ax == 0 ? xiz : ax == 1 ? etz : ztz;
+        float d1 = ad_d, ad1 = ad_a;  // of the column's y or z band
+        if (ax == 0) { d1 = uni(cold->pD[0], i); ad1 = -(uni(cold->pA[0], i) + d1); }
+        if (FULL && ax == 2 && injl) { d1 = a.cold.pD[2][k]; ad1 = -(a.cold.pA[2][k] + d1); }  // ad_d is the y band's
+        float dd[9], ah[9], w[9];
+#pragma unroll
+        for (int c = 0; c < 9; c++) dd[c] = rDH * D(c);
+#pragma unroll
+        for (int c = 0; c < 9; c++) ah[c] = ad1 * y[c] + d1 * axis_rhs_c(c, dd, e0, e1, e2, rrho, lam, l2m, mu);
+        if (FULL && ax < 2 && a.freenode && k == nk - 1) {  // the traction-free term (pmlx.cu:185-210)
+          const float c0 = d1 * (ax == 0 ? uni(cold->pB[0], i) : a.cold.pB[1][j]);
+          const float* mat = ax == 0 ? a.cold.mVx : a.cold.mVy;
+          const uint32_t ij = ((uint32_t)(j + 3) + (uint32_t)(i + 3) * (uint32_t)a.ny) * 9;
+          float z1[3];
+#pragma unroll
+          for (int r = 0; r < 3; r++) z1[r] = mat[ij + 3 * r] * dd[0] + mat[ij + 3 * r + 1] * dd[1] + mat[ij + 3 * r + 2] * dd[2];
+#pragma unroll
+          for (int c = 3; c < 9; c++) ah[c] += pml_fs_term(c, z1, ztx, zty, ztz, lam, l2m, mu, c0);
+        }
+        auto st9 = [](const float(&v)[9]) {
+          return [&v](Rsrc r, uint32_t o, uint32_t fb) {
+#pragma unroll
+            for (int c = 0; c < 9; c++) bst<kReuse>(r, o, c * fb, v[c]);
+          };
+        };
+        if (irk == 0) {  // the accumulator is derived in stage 1 (rk_derived_t)
+          on(cold->axS[ax], st9(y));
+#pragma unroll
+          for (int c = 0; c < 9; c++) w[c] = y[c] + rka * ah[c];
+        } else if (irk == 3) {
+#pragma unroll
+          for (int c = 0; c < 9; c++) w[c] = t[c] + rkb * ah[c];
+        } else {
+          if (irk == 1) {
+#pragma unroll
+            for (int c = 0; c < 9; c++) t[c] = rk_derived_t(s[c], y[c]);
+          }
+#pragma unroll
+          for (int c = 0; c < 9; c++) t[c] = t[c] + rkb * ah[c];
+          on(cold->axT[ax], st9(t));
+#pragma unroll
+          for (int c = 0; c < 9; c++) w[c] = s[c] + rka * ah[c];
+        }
+        on(cold->axY[ax], st9(w));
       };
       float h[9];
 #pragma unroll
@@ -977,52 +1035,16 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
 #pragma unroll
             for (int c = 0; c < 9; c++) h[c] += -(injl ? (inx ? ta[c] : sa[c]) : (inx ? sa[c] : ya[c])) * rb3;
           }
-          // the fused auxiliary update (what pml_aux_kernel does for the
-          // point, with the same arithmetic): aux' = -(alpha + d) aux +
-          // d * RHS_axis, RHS_axis from the plain derivative along the face's
-          // axis, advanced with the RK4 stage combine; points on one face only
-          if (!TOP && a.aux_fused && !a.rhs_only) {
-            auto advance = [&](auto D, float e0, float e1, float e2, float d1, float ad1, float* aY, float* aS, float* aT, auto on) {
-              const float rka = a.rka, rkb = a.rkb;
-              float dd[9], ah[9], w[9];
-#pragma unroll
-              for (int c = 0; c < 9; c++) dd[c] = rDH * D(c);
-#pragma unroll
-              for (int c = 0; c < 9; c++) ah[c] = ad1 * ya[c] + d1 * axis_rhs_c(c, dd, e0, e1, e2, rrho, lam, l2m, mu);
-              auto st9 = [](const float(&v)[9]) {
-                return [&v](Rsrc r, uint32_t o, uint32_t fb) {
-#pragma unroll
-                  for (int c = 0; c < 9; c++) bst<kReuse>(r, o, c * fb, v[c]);
-                };
-              };
-              if (irk == 0) {  // the accumulator is derived in stage 1 (rk_derived_t)
-                on(aS, st9(ya));
-#pragma unroll
-                for (int c = 0; c < 9; c++) w[c] = ya[c] + rka * ah[c];
-              } else if (irk == 3) {
-#pragma unroll
-                for (int c = 0; c < 9; c++) w[c] = ta[c] + rkb * ah[c];
-              } else {
-                if (irk == 1) {
-#pragma unroll
-                  for (int c = 0; c < 9; c++) ta[c] = rk_derived_t(sa[c], ya[c]);
-                }
-#pragma unroll
-                for (int c = 0; c < 9; c++) ta[c] = ta[c] + rkb * ah[c];
-                on(aT, st9(ta));
-#pragma unroll
-                for (int c = 0; c < 9; c++) w[c] = sa[c] + rka * ah[c];
-              }
-              on(aY, st9(w));
-            };
+          // the fused auxiliary update of a point on one face (what
+          // pml_aux_kernel does for it, with the same arithmetic): aux' =
+          // -(alpha + d) aux + d * RHS_axis, RHS_axis from the plain
+          // derivative along the face's axis, with the RK4 stage combine
+          if ((FULL || !TOP) && a.aux_fused && !a.rhs_only) {
             if (inx) {
-              if (fuse1) {
-                const float d1 = uni(cold->pD[0], i);
-                advance(Dx, xix, xiy, xiz, d1, -(uni(cold->pA[0], i) + d1), cold->axY[0], cold->axS[0], cold->axT[0], on_x);
-              }
+              if (fuse1) advance(std::integral_constant<int, 0>(), Dx, ya, sa, ta, on_x);
             } else {
-              if (fuse1 && injl) advance(Dy, etx, ety, etz, ad_d, ad_a, cold->axY[1], cold->axS[1], cold->axT[1], on_y);
-              if (fuse1 && inkl) advance(Dz, ztx, zty, ztz, ad_d, ad_a, cold->axY[2], cold->axS[2], cold->axT[2], on_z);
+              if (fuse1 && injl) advance(std::integral_constant<int, 1>(), Dy, ya, sa, ta, on_y);
+              if (fuse1 && inkl) advance(std::integral_constant<int, 2>(), Dz, ya, sa, ta, on_z);
             }
           }
         }
@@ -1058,6 +1080,32 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
           for (int c = 0; c < 9; c++) {
             bst(rt, col4, c * pb, tv[c] + rkb * h[c]);
             bst(ro, col4, c * pb, (sv[c] + rka * h[c]) * damp);
+          }
+        }
+      }
+      if constexpr (FULL) {  // the faces of an edge point, one after another
+        if (pml && a.aux_fused && !a.rhs_only && (inx ? injl || inkl : injl && inkl)) {
+          auto edge = [&](auto AX, auto D, const float(&y)[9], auto on) {
+            constexpr int ax = decltype(AX)::value;
+            float s[9], t[9];
+#pragma unroll
+            for (int c = 0; c < 9; c++) { s[c] = any_value(); t[c] = any_value(); }
+            if (irk >= 2) on(cold->axT[ax], ld9(t));
+            if (irk == 1 || irk == 2) on(cold->axS[ax], ld9(s));
+            advance(AX, D, y, s, t, on);
+          };
+          if (inx) edge(std::integral_constant<int, 0>(), Dx, ya, on_x);
+          if (injl) {
+            float y[9];
+#pragma unroll
+            for (int c = 0; c < 9; c++) y[c] = inx ? sa[c] : ya[c];
+            edge(std::integral_constant<int, 1>(), Dy, y, on_y);
+          }
+          if (inkl) {
+            float y[9];
+#pragma unroll
+            for (int c = 0; c < 9; c++) y[c] = inx && injl ? ta[c] : sa[c];
+            edge(std::integral_constant<int, 2>(), Dz, y, on_z);
           }
         }
       }
@@ -1218,6 +1266,14 @@ __global__ void __launch_bounds__(256) pml_aux_kernel(PmlAuxArgs<MT> a) {
   }
 }
 
+// The two passes of the free-surface image.
+template <int FX, int FY, int FZ, class MT>
+void launch_image(const WaveArgs<MT>& a, const Ctx& c, hipStream_t s) {
+  const long n1 = (long)c.d.nx * 6 * c.d.ny, n2 = (long)c.d.ni * 3 * c.d.nj;
+  hipLaunchKernelGGL(traction_top_kernel<MT>, dim3((unsigned)((n1 + 255) / 256)), dim3(256), 0, s, a, c.d.nx);
+  hipLaunchKernelGGL((image_top_kernel<FX, FY, FZ, MT>), dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0, s, a);
+}
+
 template <int FX, int FY, int FZ, class MT>
 void launch_wave_t(WaveArgs<MT> a, const Ctx& c, hipStream_t s) {
   // work list order: interior, bands (64-wide tiles), bands (32-wide tiles), free-surface tiles
@@ -1241,6 +1297,15 @@ void launch_wave_t(WaveArgs<MT> a, const Ctx& c, hipStream_t s) {
     ss = c.side[1];
     (void)hipStreamWaitEvent(si, c.fence[0], 0);
     (void)hipStreamWaitEvent(ss, c.fence[0], 0);
+  }
+  if (c.wave_unified) {
+    pr.begin(s, PK_STAGE_BAND);
+    if (a.freenode) launch_image<FX, FY, FZ, MT>(a, c, s);
+    a.work = w; a.nwork = n[1];
+    hipLaunchKernelGGL((wave_interior_kernel<FX, FY, FZ, MT, TJ, TJ * TK4, 2, true, false, true, true>), dim3(a.nwork),
+                       dim3(TJ, TK4, 1), 0, s, a);
+    pr.end(s);
+    return;
   }
   if (n[0] > 0) {
     a.work = w; a.nwork = n[0];
@@ -1267,11 +1332,7 @@ void launch_wave_t(WaveArgs<MT> a, const Ctx& c, hipStream_t s) {
   if (n[3] > 0) {
     a.work = w + 2 * o3; a.nwork = n[3];
     pr.begin(ss, PK_STAGE_SURFACE);
-    if (a.freenode) {
-      const long n1 = (long)c.d.nx * 6 * c.d.ny, n2 = (long)c.d.ni * 3 * c.d.nj;
-      hipLaunchKernelGGL(traction_top_kernel<MT>, dim3((unsigned)((n1 + 255) / 256)), dim3(256), 0, ss, a, c.d.nx);
-      hipLaunchKernelGGL((image_top_kernel<FX, FY, FZ, MT>), dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0, ss, a);
-    }
+    if (a.freenode) launch_image<FX, FY, FZ, MT>(a, c, ss);
     if (c.wave_surf_pipe)
       hipLaunchKernelGGL((wave_interior_kernel<FX, FY, FZ, MT, TJ, NTHR, 2, true, true, true>), dim3(a.nwork), dim3(TJ, TK, 1),
                          0, ss, a);
