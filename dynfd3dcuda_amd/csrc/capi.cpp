@@ -202,6 +202,12 @@ struct OutFiles {
   std::vector<int> fv;  // record var ids of the fault file
   int f_init_t0 = -1;
   int wxy[3], wxz[3], wyz[3];
+  RecordDims rd{};
+  uint32_t *dev = nullptr, *host = nullptr;  // a record's words on the device and in pinned host memory
+  ~OutFiles() {
+    if (dev) (void)hipFree(dev);
+    if (host) (void)hipHostFree(host);
+  }
 };
 
 }  // namespace
@@ -892,19 +898,18 @@ int cgfdm_open_outputs(cgfdm_ctx* h) {
     delete o;
     return fail(CGFDM_ENETCDF, err);
   }
+  o->rd = RecordDims{ni, nj, nk, kz, jy, ix, c.p.Rupture ? 1 : 0};
+  const size_t bytes = (size_t)o->rd.words() * sizeof(uint32_t);
+  if (hipMalloc(&o->dev, bytes) != hipSuccess || hipHostMalloc(&o->host, bytes, hipHostMallocDefault) != hipSuccess) {
+    delete o;
+    return fail(CGFDM_EHIP, "no memory for an output record");
+  }
   c.out = o;
   return 0;
 }
 
-// Device-to-host copy that keeps the first failure in *e (the output
-// writer reports it once the records of the call are written).
-static void d2h(void* dst, const void* src, size_t bytes, hipError_t* e) {
-  if (*e == hipSuccess) *e = hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
-}
-
 int cgfdm_write_outputs(cgfdm_ctx* h, int it) {
-  hipError_t herr = hipSuccess;  // first failed copy, reported after the records
-  std::string nonfinite;         // first NaN/Inf of the fault record, reported after it
+  std::string nonfinite;  // first NaN/Inf of the fault record, reported after the records
   if (!h) return fail(CGFDM_EPARAM, "null context");
   Ctx& c = h->c;
   if (!c.out) {
@@ -915,91 +920,37 @@ int cgfdm_write_outputs(cgfdm_ctx* h, int it) {
   if (it % skip) return 0;
   long rec = it / skip;
   NcOut* o = c.out;
-  if (hipError_t e = hipStreamSynchronize(c.stream)) return fail(CGFDM_EHIP, hipGetErrorString(e));
-  const int nj = c.d.nj, nk = c.d.nk, ni = c.d.ni, ny = c.d.ny;
-  const long nxyz = c.d.nxyz, nyz = c.d.nyz, pyz = c.d.pyz;
-  const int py = c.d.py, jpad = c.d.jpad;
-  (void)nxyz; (void)nyz;
-  if (c.p.Rupture) {
-    long n2 = (long)nj * nk;
-    std::vector<float> buf(n2);
-    std::vector<double> db(n2);
-    std::vector<int> ib(n2);
+  const RecordDims& d = o->rd;
+  if (hipError_t e = gather_record(c, d, o->dev, o->host))
+    return fail(CGFDM_EHIP, std::string("output copy failed: ") + hipGetErrorString(e));
+  const int nj = d.nj, nk = d.nk, ni = d.ni;
+  const long n2 = (long)nj * nk;
+  const uint32_t* w = o->host;
+  if (d.fault) {
     const char* names[7] = {"Vs1", "Vs2", "Tn", "Ts1", "Ts2", "slip", "State"};
-    for (int v = 0; v < 7; v++) {
-      FieldRef r = field(c, names[v]);
-      if (r.dtype == 1) {
-        d2h(db.data(), r.ptr, n2 * 8, &herr);
-        for (long q = 0; q < n2; q++) buf[q] = (float)db[q];
-      } else {
-        d2h(buf.data(), r.ptr, n2 * 4, &herr);
-      }
-      o->fault.put_record(o->fv[v], rec, buf.data());
+    for (int v = 0; v < 12; v++, w += n2) {  // Vs1 .. TP_P in the file's order
+      o->fault.put_record(o->fv[v], rec, w);
       // the first non-finite word of the record's fields (reported after the
       // record is written: the file then shows where the run went wrong)
-      if (nonfinite.empty() && herr == hipSuccess)
+      if (v < 7 && nonfinite.empty())
         for (long q = 0; q < n2; q++)
-          if (!std::isfinite(buf[q])) {
+          if ((w[q] & 0x7f800000u) == 0x7f800000u) {
             nonfinite = std::string(names[v]) + " at node j=" + std::to_string(q % nj) + " k=" + std::to_string(q / nj);
             break;
           }
     }
-    d2h(buf.data(), c.f.init_t0, n2 * 4, &herr);
-    o->fault.put_var(o->f_init_t0, buf.data());
-    d2h(ib.data(), c.f.rup_index_y, n2 * 4, &herr);
-    o->fault.put_record(o->fv[7], rec, ib.data());
-    d2h(ib.data(), c.f.rup_index_z, n2 * 4, &herr);
-    o->fault.put_record(o->fv[8], rec, ib.data());
-    d2h(buf.data(), c.f.rup_sensor, n2 * 4, &herr);
-    o->fault.put_record(o->fv[9], rec, buf.data());
-    // thermal pressurization: the rises on the fault (level 0) as the
-    // reference writes them (io_fault.cu:262-266); zeros without it
-    for (int v = 0; v < 2; v++) {
-      const double* src = v ? c.f.TP_P : c.f.TP_T;
-      if (src) {
-        d2h(db.data(), src, n2 * 8, &herr);
-        for (long q = 0; q < n2; q++) buf[q] = (float)db[q];
-      } else {
-        std::fill(buf.begin(), buf.end(), 0.0f);
-      }
-      o->fault.put_record(o->fv[10 + v], rec, buf.data());
-    }
+    o->fault.put_var(o->f_init_t0, w);
+    w += n2;
     o->fault.sync();
   }
-  // slices from the current wavefield
-  auto put_slice = [&](NcFile& f, int* vids, int axis, int idx, int d1n, int d2n) {
-    std::vector<float> buf((size_t)d1n * d2n);
-    std::vector<float> line;
-    for (int comp = 0; comp < 3; comp++) {
-      if (axis == 2) {  // xy: rows of ny for each i
-        line.resize(ny);
-        for (int a = 0; a < d1n; a++) {
-          d2h(line.data(), c.cur + ((long)(a + 3) * 9 + comp) * pyz + jpad + (long)(idx + 3) * py, ny * 4, &herr);
-          std::memcpy(&buf[(long)a * d2n], &line[3], d2n * 4);
-        }
-      } else if (axis == 1) {  // xz
-        std::vector<float> plane(pyz);
-        for (int a = 0; a < d1n; a++) {
-          d2h(plane.data(), c.cur + ((long)(a + 3) * 9 + comp) * pyz, pyz * 4, &herr);
-          for (int b = 0; b < d2n; b++) buf[(long)a * d2n + b] = plane[jpad + (idx + 3) + (long)(b + 3) * py];
-        }
-      } else {  // yz plane at i
-        std::vector<float> plane(pyz);
-        d2h(plane.data(), c.cur + ((long)(idx + 3) * 9 + comp) * pyz, pyz * 4, &herr);
-        for (int a = 0; a < d1n; a++)
-          for (int b = 0; b < d2n; b++) buf[(long)a * d2n + b] = plane[jpad + (b + 3) + (long)(a + 3) * py];
-      }
-      f.put_record(vids[comp], rec, buf.data());
-    }
+  // slices of the current wavefield
+  auto put_slice = [&](NcFile& f, const int* vids, long n) {
+    for (int comp = 0; comp < 3; comp++, w += n) f.put_record(vids[comp], rec, w);
     f.sync();
   };
-  int kz = std::min(std::max(c.p.EXPORT_WAVE_SLICE_Z, 0), nk - 1);
-  int jy = std::min(std::max(c.p.EXPORT_WAVE_SLICE_Y, 0), nj - 1);
-  int ix = std::min(std::max(c.p.EXPORT_WAVE_SLICE_X, 0), ni - 1);
-  put_slice(o->xy, o->wxy, 2, kz, ni, nj);
-  put_slice(o->xz, o->wxz, 1, jy, ni, nk);
-  put_slice(o->yz, o->wyz, 0, ix, nk, nj);
-  if (herr != hipSuccess) return fail(CGFDM_EHIP, std::string("output copy failed: ") + hipGetErrorString(herr));
+  put_slice(o->xy, o->wxy, (long)ni * nj);
+  put_slice(o->xz, o->wxz, (long)ni * nk);
+  put_slice(o->yz, o->wyz, n2);
   if (!nonfinite.empty())
     return fail(CGFDM_ENONFINITE, "non-finite value in fault record " + std::to_string(rec) + " (step " +
                                       std::to_string(it) + "): " + nonfinite + "; the run has become unstable");

@@ -262,6 +262,17 @@ struct Ctx {
 // setup (host, double precision)
 int host_setup(Ctx& c, std::string& err);
 
+// An output record gathered on the device (output_record.hip): the fault
+// fields Vs1 Vs2 Tn Ts1 Ts2 slip State rup_index_y rup_index_z rup_sensor
+// TP_T TP_P init_t0 (none without a fault), then Vx Vy Vz of the slices xy at
+// kz, xz at jy and yz at ix.
+struct RecordDims {
+  int ni, nj, nk, kz, jy, ix, fault;
+  long fault_words() const { return fault ? 13L * nj * nk : 0; }
+  long words() const { return fault_words() + 3L * ((long)ni * nj + (long)ni * nk + (long)nk * nj); }
+};
+hipError_t gather_record(Ctx& c, const RecordDims& d, uint32_t* dev, uint32_t* host);
+
 // kernel launchers (kernels.hip)
 struct StageBufs {
   const float* Win; float* Wout; const float* S; float* T;

@@ -66,6 +66,15 @@ struct Writer {
 
 void swap_copy(const void* src, unsigned char* dst, long n, int ts) {
   const unsigned char* s = (const unsigned char*)src;
+  if (ts == 4) {  // whole words (records are floats and ints): the byte loop ran at 0.3 GB/s
+    for (long q = 0; q < n; q++) {
+      uint32_t w;
+      std::memcpy(&w, s + 4 * q, 4);
+      w = __builtin_bswap32(w);
+      std::memcpy(dst + 4 * q, &w, 4);
+    }
+    return;
+  }
   for (long q = 0; q < n; q++)
     for (int t = 0; t < ts; t++) dst[q * ts + t] = s[q * ts + (ts - 1 - t)];
 }
