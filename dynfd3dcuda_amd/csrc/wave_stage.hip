@@ -176,7 +176,7 @@ int upload_wave_work(Ctx& c) {
   if (c.p.FreeSurface && !c.trac_top) {  // the image stencil reaches six rows down (NZ >= 7)
     if (hipMalloc(&c.trac_top, sizeof(float) * 9 * 6 * (size_t)c.d.nx * c.d.ny) != hipSuccess) return 1;
     c.allocations.push_back(c.trac_top);
-    if (hipMalloc(&c.img_top, sizeof(float) * 9 * (size_t)c.d.ni * c.d.nj) != hipSuccess) return 1;
+    if (hipMalloc(&c.img_top, sizeof(float) * 18 * (size_t)c.d.ni * c.d.nj) != hipSuccess) return 1;
     c.allocations.push_back(c.img_top);
   }
 
@@ -234,14 +234,12 @@ int upload_wave_work(Ctx& c) {
   c.wave_band_pipe = wbk >= 1 && disjoint;
   c.wave_band_tk = c.wave_band_pipe && wbk == 2 ? TK4 : TK;  // 2: 64 x 4 band tiles, two blocks per CU
   // WaveSurfaceKernel 1: the pipelined kernel on the free-surface tiles too
-  // (with the band terms; their auxiliary fields stay with pml_aux_kernel)
+  // (with the band terms and, with PmlAuxFused, the auxiliary fields)
   c.wave_surf_pipe = disjoint && p.WaveSurfaceKernel >= 1;
-  // PmlAuxFused 1: the pipelined band tiles advance the auxiliary fields of
-  // their points on one face only; pml_aux_kernel keeps the edges of the
-  // absorbing box (points on two or three faces, whose words the band tiles
-  // prefetch with the first face's but do not advance) and the free-surface
-  // rows (1600 x 1000 x 500: 138.5 -> 128.6 ms per step; 400 x 300 x 200:
-  // 7.67 -> 6.90 ms; interleaved runs)
+  // PmlAuxFused 1: the pipelined band and free-surface tiles advance their
+  // points' auxiliary fields; pml_aux_kernel runs on the free-surface rows
+  // when those run the general kernel, and on everything with the general
+  // band kernel
   c.pml_fused = c.wave_band_pipe && p.PmlAuxFused != 0;
   const int tki = tall ? 2 * TK : (c.wave_pipe && wik == 2) ? TK6 : (c.wave_pipe && wik == 3) ? TK4 : TK;  // interior tile rows
   c.wave_tki = tki;
@@ -316,9 +314,8 @@ int upload_wave_work(Ctx& c) {
     c.wave_points[kd] += Li * Lj * Lk;
     const long bi = in_bands(0, i0, i1), bj = in_bands(1, a.s + a.o, a.s + a.n), bk = in_bands(2, b.s + b.o, b.s + b.n);
     c.aux_read_pairs[kd] += bi * Lj * Lk + Li * bj * Lk + Li * Lj * bk;
-    // the fused update in the band tiles: points on one face only
-    if (kd == 1 && c.pml_fused)
-      c.aux_update_pairs[kd] += bi * (Lj - bj) * (Lk - bk) + (Li - bi) * bj * (Lk - bk) + (Li - bi) * (Lj - bj) * bk;
+    // the fused update in the band tiles and the pipelined free-surface tiles
+    if (c.pml_fused && (kd == 1 || (kd == 2 && c.wave_surf_pipe))) c.aux_update_pairs[kd] += bi * Lj * Lk + Li * bj * Lk + Li * Lj * bk;
   };
   const auto narrow = [&](const Seg& a) { return !a.in && a.n - a.o <= TJN; };
   // bands of at most TJB columns get tiles exactly TJB wide (with the
@@ -366,23 +363,10 @@ int upload_wave_work(Ctx& c) {
       if (is_top(b))
         for (const Seg& a : sjt) push(3, a, b, i0, std::min(ni, i0 + ich_top));
   // boxes of the auxiliary-update kernel: every absorbing face whole; with
-  // the fused update only the points the band tiles leave to it, the
-  // free-surface rows and the edges of the absorbing box (points on two or
-  // three faces).  In a face's cross-section (u, v) the edges are the
-  // u-band rows for every v, then the v-band columns of the u-middle; the
-  // free-surface rows add the u-middle x v-middle rows from ktop up.
+  // the fused update only the points the tiles leave to it, the rows from
+  // ktop up when their tiles run the general kernel
   {
-    const int N = c.pml.N, nn3[3] = {c.d.ni, c.d.nj, c.d.nk};
-    auto bands = [&](int axis) {
-      std::vector<std::pair<int, int>> v;  // (start, count)
-      if (c.pml.on[2 * axis]) v.push_back({0, N});
-      if (c.pml.on[2 * axis + 1]) v.push_back({nn3[axis] - N, N});
-      return v;
-    };
-    auto middle = [&](int axis) {
-      const int lo = c.pml.on[2 * axis] ? N : 0, hi = c.pml.on[2 * axis + 1] ? nn3[axis] - N : nn3[axis];
-      return std::make_pair(lo, std::max(hi - lo, 0));
-    };
+    const int N = c.pml.N;
     std::vector<int> bx;
     int blocks = 0;
     c.aux_update_pairs[3] = 0;
@@ -394,29 +378,12 @@ int upload_wave_work(Ctx& c) {
       c.aux_update_pairs[3] += (long)nj_ * nk_ * ni_;
     };
     for (int f = 0; f < 6; f++) {
-      if (!c.pml.on[f]) continue;
+      if (!c.pml.on[f] || (c.pml_fused && c.wave_surf_pipe)) continue;
       const int ax = f / 2;
       const int pnj = ax == 1 ? N : c.d.nj, pnk = ax == 2 ? N : c.d.nk, pni = ax == 0 ? N : c.d.ni;
-      if (!c.pml_fused) { add(f, 0, pnj, 0, pnk, 0, pni); continue; }
-      if (ax == 0) {  // u = j, v = k
-        const auto mu = middle(1), mv = middle(2);
-        for (auto b : bands(1)) add(f, b.first, b.second, 0, pnk, 0, pni);
-        for (auto b : bands(2)) add(f, mu.first, mu.second, b.first, b.second, 0, pni);
-        const int s0 = std::max(ktop, mv.first);
-        add(f, mu.first, mu.second, s0, mv.first + mv.second - s0, 0, pni);
-      } else if (ax == 1) {  // u = i, v = k
-        const auto mu = middle(0), mv = middle(2);
-        for (auto b : bands(0)) add(f, 0, pnj, 0, pnk, b.first, b.second);
-        for (auto b : bands(2)) add(f, 0, pnj, b.first, b.second, mu.first, mu.second);
-        const int s0 = std::max(ktop, mv.first);
-        add(f, 0, pnj, s0, mv.first + mv.second - s0, mu.first, mu.second);
-      } else {  // u = i, v = j; the face's own k: free-surface rows inside the band
-        const auto mu = middle(0), mv = middle(1);
-        for (auto b : bands(0)) add(f, 0, pnj, 0, pnk, b.first, b.second);
-        for (auto b : bands(1)) add(f, b.first, b.second, 0, pnk, mu.first, mu.second);
-        const int off = (f & 1) ? c.d.nk - N : 0, s0 = std::max(ktop - off, 0);
-        add(f, mv.first, mv.second, s0, N - s0, mu.first, mu.second);
-      }
+      const int off = f == 5 ? c.d.nk - N : 0;  // first row of the face
+      const int s0 = c.pml_fused ? std::max(ktop - off, 0) : 0;
+      add(f, 0, pnj, s0, pnk - s0, 0, pni);
     }
     c.pml_nbox = (int)bx.size() / kPmlBoxInts;
     c.pml_blocks = blocks;

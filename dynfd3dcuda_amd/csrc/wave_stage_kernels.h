@@ -117,14 +117,9 @@ __device__ __forceinline__ V here(V v) {
   asm volatile("" : "+s"(v));
   return v;
 }
-typedef const __attribute__((address_space(4))) WaveCold* ColdPtr;  // in the kernel arguments
-// A register whose value does not matter: read only where every lane that
-// reads it has loaded it, it needs no zeroing.
-__device__ __forceinline__ float any_value() {
-  float v;
-  asm volatile("" : "=v"(v));
-  return v;
-}
+// A byte offset past the end of every buffer resource: a load there returns 0
+// and a store is dropped, without memory traffic.
+constexpr uint32_t kNoWord = 0xfffffff0u;
 // Word of field c at padded plane x, column jk (plain loads, off the hot path).
 __device__ __forceinline__ float wat(const float* W, int c, int x, uint32_t jk, uint32_t nyz) {
   return W[((size_t)x * 9 + c) * nyz + jk];
@@ -260,6 +255,12 @@ __global__ void __launch_bounds__(256) traction_top_kernel(WaveArgs<MT> a, int n
 // top rows (wave.cu:398-487): DRP derivatives of the traction vectors along
 // each axis, the z stencil zero at the surface and odd-mirrored above it,
 // with the PML 1/beta of each axis; itop[c][row][i][j], row = k - (nk-3).
+// For the top row also what its points need of the velocity maps (traction-
+// free condition, wave.cu:207-232): the dip derivative of the velocity DzV =
+// matVx2Vz DxV + matVy2Vz DyV in planes 9-11, and its two products alone
+// (the source of the x and y faces' auxiliary fields, pmlx.cu:185-210) in
+// planes 12-14 and 15-17.  In the stage tiles, short of registers, the 18
+// map words of a point were a chain of 18 memory round trips per plane.
 template <int FX, int FY, int FZ, class MT>
 __global__ void __launch_bounds__(256) image_top_kernel(WaveArgs<MT> a) {
   const int ni = a.ni, nj = a.nj, nk = a.nk, ny = a.ny;
@@ -304,7 +305,26 @@ __global__ void __launch_bounds__(256) image_top_kernel(WaveArgs<MT> a) {
     }
   }
   const long plane = (long)ni * nj;
-  for (int c = 0; c < 3; c++) a.itop[((long)c * 3 + row) * plane + (long)i * nj + j] = hv[c] * rrhojac;
+  const long ij = (long)i * nj + j;
+  for (int c = 0; c < 3; c++) a.itop[((long)c * 3 + row) * plane + ij] = hv[c] * rrhojac;
+  if (row == 2) {
+    const float* mVx = a.cold.mVx + ((long)(j + 3) + (long)x * ny) * 9;
+    const float* mVy = a.cold.mVy + ((long)(j + 3) + (long)x * ny) * 9;
+    float dxv[3], dyv[3];
+    for (int c = 0; c < 3; c++) {
+      const float* w = a.Win + ((size_t)x * 9 + c) * a.nyz + col;
+      const long st = 9L * a.nyz;
+      dxv[c] = a.rDH * (FX > 0 ? drp5<1>(w[-st], w[0], w[st], w[2 * st], w[3 * st])
+                               : drp5<-1>(w[-3 * st], w[-2 * st], w[-st], w[0], w[st]));
+      dyv[c] = a.rDH * (FY > 0 ? drp5<1>(w[-1], w[0], w[1], w[2], w[3]) : drp5<-1>(w[-3], w[-2], w[-1], w[0], w[1]));
+    }
+    for (int r = 0; r < 3; r++) {
+      a.itop[(9 + r) * plane + ij] = mVx[3 * r] * dxv[0] + mVx[3 * r + 1] * dxv[1] + mVx[3 * r + 2] * dxv[2]
+                                   + mVy[3 * r] * dyv[0] + mVy[3 * r + 1] * dyv[1] + mVy[3 * r + 2] * dyv[2];
+      a.itop[(12 + r) * plane + ij] = mVx[3 * r] * dxv[0] + mVx[3 * r + 1] * dxv[1] + mVx[3 * r + 2] * dxv[2];
+      a.itop[(15 + r) * plane + ij] = mVy[3 * r] * dyv[0] + mVy[3 * r + 1] * dyv[1] + mVy[3 * r + 2] * dyv[2];
+    }
+  }
 }
 
 // Extra auxiliary-field source of the x/y PML faces on the free surface
@@ -604,6 +624,10 @@ __device__ __forceinline__ float met_raw_get(const uint32_t (&w)[met_raw_n<MT>()
   }
 }
 
+// Reads v, so that a load of it is waited for here.
+__device__ __forceinline__ void arrived(float v) { asm volatile("" ::"v"(v)); }
+__device__ __forceinline__ void arrived(uint32_t v) { asm volatile("" ::"v"(v)); }
+
 // Interior stage kernel with every load of plane i+1 issued before plane i
 // is computed: the points of the interior box (no absorbing layer, no free
 // surface), where the general kernel's per-plane metric and RK-register
@@ -625,15 +649,18 @@ __device__ __forceinline__ float met_raw_get(const uint32_t (&w)[met_raw_n<MT>()
 // in the general kernel's order; 1/beta and the sponge factor of plane i+1
 // are fetched during plane i.
 //
-// FULL (with BAND and TOP): tiles of any kind in one launch, every auxiliary
-// field of their points advanced here: also those of the free-surface rows
-// and, after the point's stage value is stored, of the edges of the absorbing
-// box, face by face.
+// With aux_fused a BAND tile also advances the ADE-PML auxiliary fields of
+// its points (what pml_aux_kernel does for them, with the same arithmetic),
+// one face after another for a point on several.  A kernel of its own for the
+// points on several faces read all their words again: 0.55 ms per step at
+// 400 x 300 x 200, for 0.1 ms more in the tiles.
+//
+// TOP: the free-surface rows' terms as well, so that a tile may hold points
+// of any kind.
 template <int FX, int FY, int FZ, class MT, int TJ_, int NT_, int MINB, bool BAND = false, bool RING = true,
-          bool TOP = false, bool FULL = false>
+          bool TOP = false>
 __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a) {
   static_assert(!TOP || (BAND && TJ_ == 64), "free-surface tiles: band terms, one k row per wavefront");
-  static_assert(!FULL || TOP, "tiles of any kind");
   constexpr int TJ = TJ_, TK = NT_ / TJ_;
   constexpr int LJ = TJ + 4, LK = TK + 4;
   // halo cells of one plane: the 4 k-halo rows over the tile's own columns
@@ -641,8 +668,11 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
   // written nor read (the y and z operators reach along one axis only), so
   // each k-halo row costs the cache lines of the tile's own columns alone
   constexpr int NH = 4 * TJ + 4 * TK;
-  constexpr int NHC = (NH + NT_ - 1) / NT_;  // halo cells per thread
-  static_assert(NHC <= 2, "at most two halo cells per thread");
+  // a thread has one halo cell; the few cells of a tile that has more of them
+  // than threads (64 x 4: 16) are split into words, one per thread: as second
+  // cells they took nine registers and nine loads for a sixteenth of the block
+  constexpr int NHX = NH > NT_ ? 9 * (NH - NT_) : 0;
+  static_assert(NHX <= NT_, "at most one word of the further halo cells per thread");
   constexpr int HJL = FY > 0 ? 1 : 3;
   constexpr int HKL = FZ > 0 ? 1 : 3;
   constexpr int QLO = FX > 0 ? -1 : -3;
@@ -664,106 +694,146 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
   const int item = xcd_remap((int)blockIdx.x, a.nwork);
   const int4 wk = a.work[2 * item], we = a.work[2 * item + 1];
   const int j0 = wk.x, k0 = wk.y, ibeg = wk.z, iend = wk.w;
+  typedef const __attribute__((address_space(4))) WaveArgs<MT>* ArgPtr;
+  const ArgPtr kargs = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();  // the argument a
   const int tj = threadIdx.x, tk = threadIdx.y, tid = tj + tk * TJ;
   const int ni = a.ni, nj = a.nj, nk = a.nk;
   const int j = j0 + tj, k = k0 + tk;
+  const int ku = TJ == 64 ? k0 + __builtin_amdgcn_readfirstlane(tk) : k;  // k, uniform where a wavefront is one row
+  // A lane without a point of the tile computes what its cells give and stores
+  // nothing (its stores' offsets are out of range), so that the plane loop
+  // branches on uniform values alone; a wavefront without any has a loop of
+  // its own.
   const bool act = tj >= we.z && tj < we.x && tk >= we.w && tk < we.y;
   const int nxp = ni + 6;
   const uint32_t nyz = a.nyz;
   const uint32_t py = a.py, jpad = a.jpad;
   const uint32_t col = jpad + (uint32_t)(min(max(j, -3), nj + 2) + 3) + (uint32_t)(min(max(k, -3), nk + 2) + 3) * py;
   const uint32_t col4 = col << 2;
-  const uint32_t mcol = col * (uint32_t)sizeof(MT);
+  const uint32_t out4 = act ? col4 : kNoWord;
+  // the metric of a point of the tile in every lane
+  const uint32_t mcol = (jpad + (uint32_t)(j0 + min(max(tj, we.z), we.x - 1) + 3) +
+                         (uint32_t)(k0 + min(max(tk, we.w), we.y - 1) + 3) * py) * (uint32_t)sizeof(MT);
   const uint32_t pb = nyz * 4, mpb = nyz * (uint32_t)sizeof(MT);
   const float* __restrict__ Win = a.Win;
   const int irk = a.irk;
 
-  // this thread's halo cells tid and tid + NT_: the 4 k-halo rows, then the
-  // 4 j-halo cells of each row
-  int hlk[NHC], hlj[NHC];
-  uint32_t hcol4[NHC];
-#pragma unroll
-  for (int e = 0; e < NHC; e++) {
-    const int h = tid + e * NT_;
-    hlk[e] = 0; hlj[e] = 0;
-    uint32_t hcol = col;
-    if (h < NH) {
-      if (h < 4 * TJ) {
-        const int r = h / TJ;
-        hlk[e] = r < HKL ? r : r + TK;
-        hlj[e] = HJL + h % TJ;
-      } else {
-        const int h2 = h - 4 * TJ;
-        hlk[e] = HKL + h2 / 4;
-        const int cc = h2 % 4;
-        hlj[e] = cc < HJL ? cc : cc + TJ;
-      }
-      const int gj = min(max(j0 + hlj[e] - HJL, -3), nj + 2), gk = min(max(k0 + hlk[e] - HKL, -3), nk + 2);
-      hcol = jpad + (uint32_t)(gj + 3) + (uint32_t)(gk + 3) * py;
+  // LDS place and column of halo cell h: the 4 k-halo rows, then the 4 j-halo
+  // cells of each row
+  auto halo_cell = [&](int h, int& l, int& m) -> uint32_t {
+    if (h < 4 * TJ) {
+      const int r = h / TJ;
+      l = r < HKL ? r : r + TK;
+      m = HJL + h % TJ;
+    } else {
+      const int h2 = h - 4 * TJ;
+      const int cc = h2 % 4;
+      l = HKL + h2 / 4;
+      m = cc < HJL ? cc : cc + TJ;
     }
-    hcol4[e] = hcol << 2;
-  }
-  auto load_halo = [&](Rsrc r, float (&v)[NHC][9]) {
-#pragma unroll
-    for (int e = 0; e < NHC; e++)
-      if (e == 0 || tid + e * NT_ < NH) {
-#pragma unroll
-        for (int c = 0; c < 9; c++) v[e][c] = bld(r, hcol4[e], c * pb);
-      }
+    const int gj = min(max(j0 + m - HJL, -3), nj + 2), gk = min(max(k0 + l - HKL, -3), nk + 2);
+    return (jpad + (uint32_t)(gj + 3) + (uint32_t)(gk + 3) * py) << 2;
   };
-  auto store_halo = [&](float (*L)[LK][LJ], const float (&v)[NHC][9]) {
+  // this thread's halo cell tid, and its word of the cells from NT_ on
+  int hlk = 0, hlj = 0, xl = 0;
+  const uint32_t hcol4 = tid < NH ? halo_cell(tid, hlk, hlj) : col4;
+  uint32_t xw4 = kNoWord;
+  if (NHX > 0 && tid < NHX) {
+    int l, m;
+    xw4 = halo_cell(NT_ + tid / 9, l, m) + (uint32_t)(tid % 9) * pb;
+    xl = (tid % 9 * LK + l) * LJ + m;
+  }
+  struct Halo {
+    float c[9], x;
+  };
+  auto load_halo = [&](Rsrc r, Halo& v) {
 #pragma unroll
-    for (int e = 0; e < NHC; e++)
-      if (tid + e * NT_ < NH) {
+    for (int c = 0; c < 9; c++) v.c[c] = bld(r, hcol4, c * pb);
+    if (NHX > 0) v.x = bld(r, xw4, 0);
+  };
+  auto store_halo = [&](float (*L)[LK][LJ], const Halo& v) {
+    if (tid < NH) {
 #pragma unroll
-        for (int c = 0; c < 9; c++) L[c][hlk[e]][hlj[e]] = v[e][c];
-      }
+      for (int c = 0; c < 9; c++) L[c][hlk][hlj] = v.c[c];
+    }
+    if (NHX > 0 && tid < NHX) (&L[0][0][0])[xl] = v.x;
   };
 
-  // BAND: per lane, the sides of the y and z absorbing bands that hold the
-  // point's column (j, k), its 1/beta along them, the sponge factor of the
-  // column, and for a column in one of those bands its auxiliary ODE's
-  // coefficients d/beta and -(alpha + d/beta).  The uniform descriptors are
-  // kernel arguments picked with constant indices, and every auxiliary access
-  // is a buffer access from a uniform plane base.  Through pointers staged in
-  // LDS they were flat accesses, which count as LDS operations too: the
-  // first LDS read of the compute waited for all of them, and the 1/beta of
-  // the next plane for every load ahead of it.  With this, one branch per
-  // stage around the nine fields and the argument reads below, the bands of
-  // 400 x 300 x 200 take 2.85 instead of 3.28 ms per step, of 800 x 1000 x 500
-  // (MetricBF16 2) 16.1 instead of 17.9; on grids of a few million points,
-  // where a plane's instructions are what a block waits for, 15-30% less.
+  // BAND: per lane, the 1/beta of the point's column (j, k) along y and z, the
+  // coefficients d/beta and -(alpha + d/beta) of its auxiliary ODEs there,
+  // the sponge factor of the column, and its words' byte offsets in the first
+  // field of its x, y and z face planes (the high y and z faces follow the
+  // low ones within a plane), kNoWord outside the band.  Whether a wavefront
+  // has a face along x (its plane), y (its columns) or z (its rows) is
+  // uniform, and a face's words are loaded and stored for all of its lanes:
+  // those without one read 0 and store nothing.  Under lane masks the loads
+  // of the different faces met in the same registers, which cost copies
+  // behind waits for the loads in flight.  The uniform descriptors are kernel
+  // arguments and every access a buffer access from a uniform plane base:
+  // through pointers staged in LDS they were flat accesses, which count as
+  // LDS operations too, so that the first LDS read of the compute waited for
+  // all loads in flight.
   const bool pml = BAND && a.pml, cerjan = BAND && a.cerjan;
   float rb2 = 1.0f, rb3 = 1.0f, cjk = 1.0f;
-  float ad_d = 0.0f, ad_a = 0.0f;
+  float dy = 0.0f, ay = 0.0f, dz = 0.0f, az = 0.0f;
   const int N = BAND ? a.cold.N : 0;
-  int sj = -1, sk = -1;  // side (0 low, 1 high) of the y and z band holding the column, -1 outside
-  if constexpr (BAND) {
-    if (act && pml) { rb2 = 1.0f / a.cold.pB[1][j]; rb3 = 1.0f / a.cold.pB[2][k]; }
-    if (act && cerjan) cjk = fminf(a.cold.cj[1][j + 3], a.cold.cj[2][k + 3]);
-    if (act && pml) {
-      if (a.cold.on[2] && j < N) sj = 0;
-      else if (a.cold.on[3] && j >= nj - N) sj = 1;
-      if (a.cold.on[4] && k < N) sk = 0;
-      else if (a.cold.on[5] && k >= nk - N) sk = 1;
-      if (sj >= 0) { ad_d = a.cold.pD[1][j]; ad_a = -(a.cold.pA[1][j] + ad_d); }
-      else if (sk >= 0) { ad_d = a.cold.pD[2][k]; ad_a = -(a.cold.pA[2][k] + ad_d); }
-    }
-  }
-  const bool injl = sj >= 0, inkl = sk >= 0;
-  const ColdPtr kcold = (ColdPtr)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() +
-                                  offsetof(WaveArgs<MT>, cold));
   const uint32_t xpp = (uint32_t)nk * nj, ypp = (uint32_t)nk * N, zpp = (uint32_t)N * nj;  // words of a field of a face plane
   const uint32_t nyf = BAND ? a.cold.on[2] + a.cold.on[3] : 0, nzf = BAND ? a.cold.on[4] + a.cold.on[5] : 0;
-  // byte offset of the lane's word in the first field of its x, y and z face
-  // plane (the high y and z faces follow the low ones within a plane)
-  const uint32_t xo4 = BAND ? (uint32_t)(j + k * nj) << 2 : 0u;
-  const uint32_t yo4 = BAND ? ((sj == 1 ? j - (nj - N) + (a.cold.on[2] ? 9 * ypp : 0u) : j) + (uint32_t)(k * N)) << 2 : 0u;
-  const uint32_t zo4 = BAND ? (j + (sk == 1 ? (k - (nk - N)) * nj + (a.cold.on[4] ? 9 * zpp : 0u) : (uint32_t)(k * nj))) << 2 : 0u;
+  uint32_t xo4 = kNoWord, yo4 = kNoWord, zo4 = kNoWord;
+  bool hasy = false, hasz = false;  // the wavefront has columns in a y band, rows in a z band
+  if constexpr (BAND) {
+    if (pml) {
+      const int ja = j0 + we.z, jb = j0 + we.x;
+      hasy = (a.cold.on[2] && ja < N) || (a.cold.on[3] && jb > nj - N);
+      // rows of this wavefront: one for the 64-wide tiles, else any of the tile's
+      const int ka = TJ == 64 ? ku : k0 + we.w, kb = TJ == 64 ? ka + 1 : k0 + we.y;
+      hasz = (a.cold.on[4] && ka < N) || (a.cold.on[5] && kb > nk - N);
+    }
+    if (act && pml) {
+      rb2 = 1.0f / a.cold.pB[1][j];
+      rb3 = 1.0f / a.cold.pB[2][k];
+      dy = a.cold.pD[1][j];
+      ay = -(a.cold.pA[1][j] + dy);
+      dz = a.cold.pD[2][k];
+      az = -(a.cold.pA[2][k] + dz);
+      xo4 = (uint32_t)(j + k * nj) << 2;
+      if (a.cold.on[2] && j < N) yo4 = (uint32_t)(j + k * N) << 2;
+      else if (a.cold.on[3] && j >= nj - N) yo4 = ((uint32_t)(j - (nj - N) + k * N) + (a.cold.on[2] ? 9 * ypp : 0u)) << 2;
+      if (a.cold.on[4] && k < N) zo4 = (uint32_t)(j + k * nj) << 2;
+      else if (a.cold.on[5] && k >= nk - N) zo4 = ((uint32_t)(j + (k - (nk - N)) * nj) + (a.cold.on[4] ? 9 * zpp : 0u)) << 2;
+    }
+    if (act && cerjan) cjk = fminf(a.cold.cj[1][j + 3], a.cold.cj[2][k + 3]);
+  }
   const int xoff1 = BAND ? (a.cold.on[0] ? N : 0) : 0;  // first plane of the high x face
   // 1/beta of plane i along x and the sponge factor of plane i (uniform)
   auto rb_x = [&](int i) { return pml ? 1.0f / uni(a.cold.pB[0], i) : 1.0f; };
   auto cj_x = [&](int i) { return cerjan ? uni(a.cold.cj[0], i + 3) : 1.0f; };
+
+  if (__builtin_amdgcn_ballot_w64(act) == 0) {  // the cells of the neighbours' stencils alone
+    Halo v;
+    float own[9];
+    auto stage = [&](int plane, int slot) {
+      const Rsrc r = plane_rsrc(Win, plane + 3, 9, nyz);
+#pragma unroll
+      for (int c = 0; c < 9; c++) own[c] = bld(r, col4, c * pb);
+      load_halo(r, v);
+#pragma unroll
+      for (int c = 0; c < 9; c++) lds[slot][c][tk + HKL][tj + HJL] = own[c];
+      store_halo(lds[slot], v);
+    };
+    for (int m = 0; m < LEAD; m++)
+      if (ibeg + m < iend) stage(ibeg + m, m);
+    if (std::is_same<MT, MetBf16Delta>::value && a.pal != nullptr)
+      for (int e = tid; e < a.npal; e += NT_) s_pal[e] = a.pal[e];
+    __syncthreads();
+    int b = 0;
+    for (int i = ibeg; i < iend; ++i) {
+      if (i + LEAD < iend) stage(i + LEAD, b == 0 ? NS - 1 : b - 1);
+      b = b == NS - 1 ? 0 : b + 1;
+      __syncthreads();
+    }
+    return;
+  }
 
   float q[5][9];
 #pragma unroll
@@ -774,7 +844,7 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
   }
   // planes ibeg .. ibeg + LEAD - 1 of the ring: own values from the queue,
   // halos loaded here
-  float hv[NHC][9];
+  Halo hv;
 #pragma unroll
   for (int m = 0; m < LEAD; m++) {
     if (ibeg + m < iend) {  // uniform per block
@@ -796,6 +866,10 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
 
   int b = 0;  // ring slot of plane i; plane i + LEAD goes to the slot before it
   for (int i = ibeg; i < iend; ++i) {
+    // band tiles read the arguments again in every plane: held in scalar
+    // registers across the loop, with the field offsets and the masks of the
+    // bands, they spill to vector lanes (444 v_readlane in the FULL loop)
+    const ArgPtr ap = BAND ? here(kargs) : kargs;
     const bool more = i + 1 < iend;       // uniform per block
     const bool ahead = i + LEAD < iend;   // uniform per block
     const int bw = b == 0 ? NS - 1 : b - 1;
@@ -811,7 +885,7 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
     }
     if (!RING && ahead) load_halo(plane_rsrc(Win, i + 4, 9, nyz), hv);
     uint32_t mwn[NMW];
-    met_raw_load<MT>(plane_rsrc(a.met, min(i + 4, nxp - 1), met_nf<MT>(), nyz), mcol, mpb, mwn, palette, met_skip);
+    met_raw_load<MT>(plane_rsrc(ap->met, min(i + 4, nxp - 1), met_nf<MT>(), nyz), mcol, mpb, mwn, palette, met_skip);
     float rb1n = 1.0f, cjxn = 1.0f;
     if constexpr (BAND) {
       if (more) { rb1n = rb_x(i + 1); cjxn = cj_x(i + 1); }
@@ -819,37 +893,37 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
     // plane i: the step-start (S) and accumulator (T) words of the RK
     // combine; stage 1 derives T from S and the point's stage-0 value
     // unless the point keeps it (rk_combine_b)
-    const bool slab = a.fault && i >= a.ii0 - 3 && i <= a.ii0 + 3 && i != a.ii0;
+    const bool slab = ap->fault && i >= ap->ii0 - 3 && i <= ap->ii0 + 3 && i != ap->ii0;
     const float damp = cerjan ? fminf(cjx, cjk) : 1.0f;
-    const bool keep_t = damp != 1.0f || (a.fault && i == a.ii0);
-    const Rsrc rs = plane_rsrc(a.S, i + 3, 9, nyz), rt = plane_rsrc(a.T, i + 3, 9, nyz);
+    const bool keep_plane = ap->fault && i == ap->ii0;
+    const bool keep_t = damp != 1.0f || keep_plane;
+    const bool keep_any = keep_plane || (cerjan && __builtin_amdgcn_ballot_w64(damp != 1.0f) != 0);  // uniform
+    const bool rk = !ap->rhs_only && !slab;
+    const Rsrc rs = plane_rsrc(ap->S, i + 3, 9, nyz), rt = plane_rsrc(ap->T, i + 3, 9, nyz);
+    // (zeros where the stage has no use for them: left unset, the registers
+    // were carried from plane to plane, with copies behind a wait for the
+    // stores)
     float sv[9], tv[9];
+    if (rk && (irk >= 2 || (irk == 1 && keep_any))) {
 #pragma unroll
-    for (int c = 0; c < 9; c++) { sv[c] = any_value(); tv[c] = any_value(); }
-    if (!a.rhs_only && !slab && irk != 0) {
-      if (irk != 1 || keep_t) {
+      for (int c = 0; c < 9; c++) tv[c] = bld<kStream>(rt, col4, c * pb);
+    } else {
 #pragma unroll
-        for (int c = 0; c < 9; c++) tv[c] = bld<kStream>(rt, col4, c * pb);
-      }
-      if (irk != 3) {
-#pragma unroll
-        for (int c = 0; c < 9; c++) sv[c] = bld<kStream>(rs, col4, c * pb);
-      }
+      for (int c = 0; c < 9; c++) tv[c] = 0.0f;
     }
-    // BAND: the faces whose band holds the point, and the aux words of plane
-    // i (pmlx.cu:126-210 and the y/z variants), all issued with S and T: the
-    // first face's value in ya; for a point on that face alone and the fused
-    // auxiliary update, its step-start (S) and accumulator (T) words in sa
-    // and ta; for a point on two or three faces (an edge of the absorbing
-    // box, whose auxiliary fields pml_aux_kernel advances) the second and
-    // third faces' values in sa and ta instead.  The x band is uniform; a
-    // lane's y or z face is one of two, each under its own mask.
-    float ya[9], sa[9], ta[9];
-    bool inx = false, fuse1 = false;
+    if (rk && (irk == 1 || irk == 2)) {
+#pragma unroll
+      for (int c = 0; c < 9; c++) sv[c] = bld<kStream>(rs, col4, c * pb);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 9; c++) sv[c] = 0.0f;
+    }
+    // BAND: the auxiliary values of plane i on the wavefront's faces
+    // (pmlx.cu:126-210 and the y/z variants), issued with S and T
+    float vx[9], vy[9], vz[9];
+    bool inx = false;  // a plane of an x band
     int pix = 0;
-    // the axes' arrays, read again from the kernel arguments in every plane
-    // (kept in registers across the loop they spill to vector lanes)
-    const ColdPtr cold = here(kcold);
+    const auto cold = &ap->cold;
     // applies f(resource, byte offset, bytes of a field) to the lane's word
     // of its x, y or z face in the axis's array
     auto on_x = [&](float* arr, auto f) { f(aux_rsrc(arr, pix, xpp, 1), xo4, here(4 * xpp)); };
@@ -861,47 +935,23 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
         for (int c = 0; c < 9; c++) v[c] = bld(r, o, c * fb);
       };
     };
-    if constexpr (BAND) {
+    auto st9 = [](const float(&v)[9]) {
+      return [&v](Rsrc r, uint32_t o, uint32_t fb) {
 #pragma unroll
-      for (int c = 0; c < 9; c++) { ya[c] = any_value(); sa[c] = any_value(); ta[c] = any_value(); }
+        for (int c = 0; c < 9; c++) bst<kReuse>(r, o, c * fb, v[c]);
+      };
+    };
+    if constexpr (BAND) {
       if (pml) {
-        if (a.cold.on[0] && i < N) { inx = true; pix = i; }
-        else if (a.cold.on[1] && i >= ni - N) { inx = true; pix = i - (ni - N) + xoff1; }
-        const bool fuse = (FULL || !TOP) && a.aux_fused && !a.rhs_only;
-        const bool need_t = fuse && irk >= 2, need_s = fuse && (irk == 1 || irk == 2);  // stage 1 derives the accumulator
-        if (inx) {
-          fuse1 = fuse && act && !injl && !inkl;
-          if (act) {
-            on_x(cold->axY[0], ld9(ya));
-            if (injl) on_y(cold->axY[1], ld9(sa));
-            else if (inkl) on_z(cold->axY[2], ld9(sa));
-            if (injl && inkl) on_z(cold->axY[2], ld9(ta));
-          }
-          if (fuse1) {
-            if (need_t) on_x(cold->axT[0], ld9(ta));
-            if (need_s) on_x(cold->axS[0], ld9(sa));
-          }
-        } else {
-          fuse1 = fuse && injl != inkl;
-          if (injl) {
-            on_y(cold->axY[1], ld9(ya));
-            if (inkl) on_z(cold->axY[2], ld9(sa));
-            if (fuse1) {
-              if (need_t) on_y(cold->axT[1], ld9(ta));
-              if (need_s) on_y(cold->axS[1], ld9(sa));
-            }
-          } else if (inkl) {
-            on_z(cold->axY[2], ld9(ya));
-            if (fuse1) {
-              if (need_t) on_z(cold->axT[2], ld9(ta));
-              if (need_s) on_z(cold->axS[2], ld9(sa));
-            }
-          }
-        }
+        if (cold->on[0] && i < N) { inx = true; pix = i; }
+        else if (cold->on[1] && i >= ni - N) { inx = true; pix = i - (ni - N) + xoff1; }
+        if (inx) on_x(cold->axY[0], ld9(vx));
+        if (hasy) on_y(cold->axY[1], ld9(vy));
+        if (hasz) on_z(cold->axY[2], ld9(vz));
       }
     }
 
-    if (act) {
+    {
       auto MET = [&](int c) { return met_raw_get<MT>(mw, c, a.mref, palette ? s_pal : nullptr); };
       const float xix = MET(0), xiy = MET(1), xiz = MET(2);
       const float etx = MET(3), ety = MET(4), etz = MET(5);
@@ -909,7 +959,7 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
       const float lam = MET(10), mu = MET(11);
       const float rrho = 1.0f / MET(12);
       const float l2m = lam + 2.0f * mu;
-      const float rDH = a.rDH;
+      const float rDH = ap->rDH;
       const float(*L)[LK][LJ] = lds[b];
       const int lj = tj + HJL, lk = tk + HKL;
       auto Dx = [&](int c) { return drp5<FX>(q[0][c], q[1][c], q[2][c], q[3][c], q[4][c]); };
@@ -921,38 +971,36 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
         return FZ > 0 ? drp5<1>(L[c][lk - 1][lj], L[c][lk][lj], L[c][lk + 1][lj], L[c][lk + 2][lj], L[c][lk + 3][lj])
                       : drp5<-1>(L[c][lk - 3][lj], L[c][lk - 2][lj], L[c][lk - 1][lj], L[c][lk][lj], L[c][lk + 1][lj]);
       };
+      // TOP: the words of the surface rows from image_top_kernel
+      const bool top = TOP && ap->freenode && ku >= nk - 3;  // uniform
+      auto top_word = [&](int p) {  // plane p of the surface words
+        return bld(__builtin_amdgcn_make_buffer_rsrc(ap->itop + ((size_t)p * ni + i) * nj, (short)0, nj * 4, kBufWord3),
+                   (uint32_t)j << 2, 0);
+      };
+      float tv3[3], tz[3];
       // one step of the auxiliary ODE of the lane's point on its face along
-      // axis AX (values y, step start s, accumulator t), stored through `on`
-      auto advance = [&](auto AX, auto D, const float(&y)[9], const float(&s)[9], float(&t)[9], auto on) {
+      // axis AX: aux' = -(alpha + d) aux + d * RHS_axis, RHS_axis from the
+      // plain derivative along the axis, with the RK4 stage combine; y the
+      // values, s and t the step-start and accumulator words
+      auto advance = [&](auto AX, auto D, const float(&y)[9], const float(&s)[9], const float(&t)[9], float d1, float ad1, auto on) {
         constexpr int ax = decltype(AX)::value;
-        const float rka = a.rka, rkb = a.rkb;
+        const float rka = ap->rka, rkb = ap->rkb;
         const float e0 = ax == 0 ? xix : ax == 1 ? etx : ztx;
         const float e1 = ax == 0 ? xiy : ax == 1 ? ety : zty;
         const float e2 = ax == 0 ? xiz : ax == 1 ? etz : ztz;
-        float d1 = ad_d, ad1 = ad_a;  // of the column's y or z band
-        if (ax == 0) { d1 = uni(cold->pD[0], i); ad1 = -(uni(cold->pA[0], i) + d1); }
-        if (FULL && ax == 2 && injl) { d1 = a.cold.pD[2][k]; ad1 = -(a.cold.pA[2][k] + d1); }  // ad_d is the y band's
         float dd[9], ah[9], w[9];
 #pragma unroll
         for (int c = 0; c < 9; c++) dd[c] = rDH * D(c);
 #pragma unroll
         for (int c = 0; c < 9; c++) ah[c] = ad1 * y[c] + d1 * axis_rhs_c(c, dd, e0, e1, e2, rrho, lam, l2m, mu);
-        if (FULL && ax < 2 && a.freenode && k == nk - 1) {  // the traction-free term (pmlx.cu:185-210)
-          const float c0 = d1 * (ax == 0 ? uni(cold->pB[0], i) : a.cold.pB[1][j]);
-          const float* mat = ax == 0 ? a.cold.mVx : a.cold.mVy;
-          const uint32_t ij = ((uint32_t)(j + 3) + (uint32_t)(i + 3) * (uint32_t)a.ny) * 9;
+        if (TOP && ax < 2 && top && ku == nk - 1) {  // the traction-free term (pmlx.cu:185-210)
+          const float c0 = d1 * (ax == 0 ? uni(cold->pB[0], i) : cold->pB[1][min(j, nj - 1)]);
           float z1[3];
 #pragma unroll
-          for (int r = 0; r < 3; r++) z1[r] = mat[ij + 3 * r] * dd[0] + mat[ij + 3 * r + 1] * dd[1] + mat[ij + 3 * r + 2] * dd[2];
+          for (int r = 0; r < 3; r++) z1[r] = top_word(12 + 3 * ax + r);
 #pragma unroll
           for (int c = 3; c < 9; c++) ah[c] += pml_fs_term(c, z1, ztx, zty, ztz, lam, l2m, mu, c0);
         }
-        auto st9 = [](const float(&v)[9]) {
-          return [&v](Rsrc r, uint32_t o, uint32_t fb) {
-#pragma unroll
-            for (int c = 0; c < 9; c++) bst<kReuse>(r, o, c * fb, v[c]);
-          };
-        };
         if (irk == 0) {  // the accumulator is derived in stage 1 (rk_derived_t)
           on(cold->axS[ax], st9(y));
 #pragma unroll
@@ -961,13 +1009,15 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
 #pragma unroll
           for (int c = 0; c < 9; c++) w[c] = t[c] + rkb * ah[c];
         } else {
+          float tn[9];
           if (irk == 1) {
 #pragma unroll
-            for (int c = 0; c < 9; c++) t[c] = rk_derived_t(s[c], y[c]);
-          }
+            for (int c = 0; c < 9; c++) tn[c] = rk_derived_t(s[c], y[c]) + rkb * ah[c];
+          } else {
 #pragma unroll
-          for (int c = 0; c < 9; c++) t[c] = t[c] + rkb * ah[c];
-          on(cold->axT[ax], st9(t));
+            for (int c = 0; c < 9; c++) tn[c] = t[c] + rkb * ah[c];
+          }
+          on(cold->axT[ax], st9(tn));
 #pragma unroll
           for (int c = 0; c < 9; c++) w[c] = s[c] + rka * ah[c];
         }
@@ -981,25 +1031,27 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
         const float s1 = rb1 * rDH, s2 = rb2 * rDH, s3 = rb3 * rDH;
         accum_axis(h, Dx, xix * s1, xiy * s1, xiz * s1, rrho, lam, l2m, mu, true);
         accum_axis(h, Dy, etx * s2, ety * s2, etz * s2, rrho, lam, l2m, mu, true);
-        accum_axis(h, Dz, ztx * s3, zty * s3, ztz * s3, rrho, lam, l2m, mu, !(TOP && a.freenode && k >= nk - 3));
+        if (top) {
+#pragma unroll
+          for (int c = 0; c < 3; c++) tv3[c] = top_word(3 * c + ku - (nk - 3));
+          if (ku == nk - 1) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) tz[c] = top_word(9 + c);
+          }
+        }
+        accum_axis(h, Dz, ztx * s3, zty * s3, ztz * s3, rrho, lam, l2m, mu, !top);
       }
       if constexpr (TOP) {
         // the top three rows under the free surface (wave.cu:207-245), as
         // the general kernel computes them: DzV of the stress rates from the
         // traction-free condition, L22 or L24, and the velocity RHS of the
         // image (image_top_kernel); one k row per wavefront
-        if (a.freenode && k >= nk - 3) {
+        if (top) {
           float dzv[3];
-          if (k == nk - 1) {  // traction-free condition (wave.cu:207-232)
-            const uint32_t ij = ((uint32_t)(j + 3) + (uint32_t)(i + 3) * (uint32_t)a.ny) * 9;
-            const float* mVx = a.cold.mVx;
-            const float* mVy = a.cold.mVy;
-            const float dxv[3] = {rDH * Dx(0), rDH * Dx(1), rDH * Dx(2)}, dyv[3] = {rDH * Dy(0), rDH * Dy(1), rDH * Dy(2)};
+          if (ku == nk - 1) {  // traction-free condition (wave.cu:207-232, image_top_kernel)
 #pragma unroll
-            for (int r = 0; r < 3; r++)
-              dzv[r] = mVx[ij + 3 * r] * dxv[0] + mVx[ij + 3 * r + 1] * dxv[1] + mVx[ij + 3 * r + 2] * dxv[2]
-                     + mVy[ij + 3 * r] * dyv[0] + mVy[ij + 3 * r + 1] * dyv[1] + mVy[ij + 3 * r + 2] * dyv[2];
-          } else if (k == nk - 2) {  // L22 (wave.cu:233-238)
+            for (int c = 0; c < 3; c++) dzv[c] = tz[c];
+          } else if (ku == nk - 2) {  // L22 (wave.cu:233-238)
 #pragma unroll
             for (int c = 0; c < 3; c++) dzv[c] = rDH * (FZ > 0 ? L[c][lk + 1][lj] - L[c][lk][lj] : L[c][lk][lj] - L[c][lk - 1][lj]);
           } else {  // L24 (wave.cu:239-245)
@@ -1015,98 +1067,102 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
           h[6] += (e1 * dzv[0] + e0 * dzv[1]) * mu;
           h[7] += (e2 * dzv[0] + e0 * dzv[2]) * mu;
           h[8] += (e2 * dzv[1] + e1 * dzv[2]) * mu;
-          const long plane = (long)ni * nj, o = ((long)(k - (nk - 3))) * plane + (long)i * nj + j;
 #pragma unroll
-          for (int c = 0; c < 3; c++) h[c] = a.itop[(long)c * 3 * plane + o];
+          for (int c = 0; c < 3; c++) h[c] = tv3[c];
         }
       }
       if constexpr (BAND) {
         if (pml) {
-          // -aux/beta of each face holding the point, x then y then z
+          // -aux/beta of each face, x then y then z (0 for a lane without it)
           if (inx) {
 #pragma unroll
-            for (int c = 0; c < 9; c++) h[c] += -ya[c] * rb1;
+            for (int c = 0; c < 9; c++) h[c] += -vx[c] * rb1;
           }
-          if (injl) {
+          if (hasy) {
 #pragma unroll
-            for (int c = 0; c < 9; c++) h[c] += -(inx ? sa[c] : ya[c]) * rb2;
+            for (int c = 0; c < 9; c++) h[c] += -vy[c] * rb2;
           }
-          if (inkl) {
+          if (hasz) {
 #pragma unroll
-            for (int c = 0; c < 9; c++) h[c] += -(injl ? (inx ? ta[c] : sa[c]) : (inx ? sa[c] : ya[c])) * rb3;
-          }
-          // the fused auxiliary update of a point on one face (what
-          // pml_aux_kernel does for it, with the same arithmetic): aux' =
-          // -(alpha + d) aux + d * RHS_axis, RHS_axis from the plain
-          // derivative along the face's axis, with the RK4 stage combine
-          if ((FULL || !TOP) && a.aux_fused && !a.rhs_only) {
-            if (inx) {
-              if (fuse1) advance(std::integral_constant<int, 0>(), Dx, ya, sa, ta, on_x);
-            } else {
-              if (fuse1 && injl) advance(std::integral_constant<int, 1>(), Dy, ya, sa, ta, on_y);
-              if (fuse1 && inkl) advance(std::integral_constant<int, 2>(), Dz, ya, sa, ta, on_z);
-            }
+            for (int c = 0; c < 9; c++) h[c] += -vz[c] * rb3;
           }
         }
       }
-      if (a.rhs_only) {
+      // Every load of the plane is waited for here: the youngest are needed
+      // now, the others at the plane's end, where a wait for them would be a
+      // wait for the stores below as well (they count together, in order).
+      // The stores drain during the next plane: 41.7 -> 37.5 ms of interior
+      // tiles per step at 800 x 1000 x 500, 2.18 -> 1.76 ms of tiles at
+      // 251 x 187 x 143.
 #pragma unroll
-        for (int c = 0; c < 9; c++) bst(plane_rsrc(a.rhs, i + 3, 9, nyz), col4, c * pb, h[c]);
+      for (int c = 0; c < 9; c++) arrived(nq[c]), arrived(hv.c[c]), arrived(sv[c]), arrived(tv[c]);
+      if (NHX > 0) arrived(hv.x);
+#pragma unroll
+      for (int m = 0; m < NMW; m++) arrived(mwn[m]);
+      // the first face's step-start and accumulator words, in flight during
+      // the RK combine (they take the registers of the stencil's operands)
+      const bool fuse = BAND && pml && ap->aux_fused && !ap->rhs_only;
+      float as[9], at[9];
+      auto ld_st = [&](auto AX, auto on) {
+        constexpr int ax = decltype(AX)::value;
+        if (irk >= 2) on(cold->axT[ax], ld9(at));
+        if (irk == 1 || irk == 2) on(cold->axS[ax], ld9(as));
+      };
+      constexpr std::integral_constant<int, 0> X{};
+      constexpr std::integral_constant<int, 1> Y{};
+      constexpr std::integral_constant<int, 2> Z{};
+      if (!TOP && fuse) {
+        if (inx) ld_st(X, on_x);
+        else if (hasy) ld_st(Y, on_y);
+        else if (hasz) ld_st(Z, on_z);
+      }
+      if (ap->rhs_only) {
+#pragma unroll
+        for (int c = 0; c < 9; c++) bst(plane_rsrc(ap->rhs, i + 3, 9, nyz), out4, c * pb, h[c]);
       } else if (slab) {
-        const Rsrc r = plane_rsrc(a.slabH, i - (a.ii0 - 3), 9, nyz);
+        const Rsrc r = plane_rsrc(ap->slabH, i - (ap->ii0 - 3), 9, nyz);
 #pragma unroll
-        for (int c = 0; c < 9; c++) bst(r, col4, c * pb, h[c]);
+        for (int c = 0; c < 9; c++) bst(r, out4, c * pb, h[c]);
       } else {
         // RK_Syn (rk4.cu:20-33); the damping factor is 1 in the interior
-        const Rsrc ro = plane_rsrc(a.Wout, i + 3, 9, nyz);
-        const float rka = a.rka, rkb = a.rkb;
+        const Rsrc ro = plane_rsrc(ap->Wout, i + 3, 9, nyz);
+        const float rka = ap->rka, rkb = ap->rkb;
         // one branch per stage around its nine fields, not one per field
         if (irk == 0) {
-          if (keep_t) {
+          if (keep_any) {
+            const uint32_t t4 = keep_t ? out4 : kNoWord;
 #pragma unroll
-            for (int c = 0; c < 9; c++) bst(rt, col4, c * pb, q[CTR][c] + rkb * h[c]);
+            for (int c = 0; c < 9; c++) bst(rt, t4, c * pb, q[CTR][c] + rkb * h[c]);
           }
 #pragma unroll
-          for (int c = 0; c < 9; c++) bst(ro, col4, c * pb, (q[CTR][c] + rka * h[c]) * damp);
+          for (int c = 0; c < 9; c++) bst(ro, out4, c * pb, (q[CTR][c] + rka * h[c]) * damp);
         } else if (irk == 3) {
 #pragma unroll
-          for (int c = 0; c < 9; c++) bst(ro, col4, c * pb, (tv[c] + rkb * h[c]) * damp);
+          for (int c = 0; c < 9; c++) bst(ro, out4, c * pb, (tv[c] + rkb * h[c]) * damp);
         } else {
-          if (irk == 1 && !keep_t) {
+          float tb[9];
 #pragma unroll
-            for (int c = 0; c < 9; c++) tv[c] = rk_derived_t(sv[c], q[CTR][c]);
-          }
+          for (int c = 0; c < 9; c++) tb[c] = irk == 2 || keep_t ? tv[c] : rk_derived_t(sv[c], q[CTR][c]);
 #pragma unroll
           for (int c = 0; c < 9; c++) {
-            bst(rt, col4, c * pb, tv[c] + rkb * h[c]);
-            bst(ro, col4, c * pb, (sv[c] + rka * h[c]) * damp);
+            bst(rt, out4, c * pb, tb[c] + rkb * h[c]);
+            bst(ro, out4, c * pb, (sv[c] + rka * h[c]) * damp);
           }
         }
       }
-      if constexpr (FULL) {  // the faces of an edge point, one after another
-        if (pml && a.aux_fused && !a.rhs_only && (inx ? injl || inkl : injl && inkl)) {
-          auto edge = [&](auto AX, auto D, const float(&y)[9], auto on) {
-            constexpr int ax = decltype(AX)::value;
-            float s[9], t[9];
-#pragma unroll
-            for (int c = 0; c < 9; c++) { s[c] = any_value(); t[c] = any_value(); }
-            if (irk >= 2) on(cold->axT[ax], ld9(t));
-            if (irk == 1 || irk == 2) on(cold->axS[ax], ld9(s));
-            advance(AX, D, y, s, t, on);
-          };
-          if (inx) edge(std::integral_constant<int, 0>(), Dx, ya, on_x);
-          if (injl) {
-            float y[9];
-#pragma unroll
-            for (int c = 0; c < 9; c++) y[c] = inx ? sa[c] : ya[c];
-            edge(std::integral_constant<int, 1>(), Dy, y, on_y);
-          }
-          if (inkl) {
-            float y[9];
-#pragma unroll
-            for (int c = 0; c < 9; c++) y[c] = inx && injl ? ta[c] : sa[c];
-            edge(std::integral_constant<int, 2>(), Dz, y, on_z);
-          }
+      if (fuse) {
+        if (inx) {
+          if (TOP) ld_st(X, on_x);
+          const float d1 = uni(cold->pD[0], i);
+          advance(X, Dx, vx, as, at, d1, -(uni(cold->pA[0], i) + d1), on_x);
+        }
+        if (hasy) {
+          if (TOP || inx) ld_st(Y, on_y);
+          advance(Y, Dy, vy, as, at, dy, ay, on_y);
+        }
+        if (hasz) {
+          if (TOP || inx || hasy) ld_st(Z, on_z);
+          advance(Z, Dz, vz, as, at, dz, az, on_z);
         }
       }
     }
@@ -1302,7 +1358,7 @@ void launch_wave_t(WaveArgs<MT> a, const Ctx& c, hipStream_t s) {
     pr.begin(s, PK_STAGE_BAND);
     if (a.freenode) launch_image<FX, FY, FZ, MT>(a, c, s);
     a.work = w; a.nwork = n[1];
-    hipLaunchKernelGGL((wave_interior_kernel<FX, FY, FZ, MT, TJ, TJ * TK4, 2, true, false, true, true>), dim3(a.nwork),
+    hipLaunchKernelGGL((wave_interior_kernel<FX, FY, FZ, MT, TJ, TJ * TK4, 2, true, false, true>), dim3(a.nwork),
                        dim3(TJ, TK4, 1), 0, s, a);
     pr.end(s);
     return;
