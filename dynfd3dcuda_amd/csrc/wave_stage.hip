@@ -99,15 +99,19 @@ static int put_work(Ctx& c, const std::vector<int4>& all) {
   return 0;
 }
 
-// The work list of the unified launch: 64 x 4 tiles over the whole grid, in
-// chunks of planes.
+// The work list of the unified launch: 32 x 8 tiles over the whole grid, in
+// chunks of planes.  A wavefront's time is the same for a full and for a
+// partial tile, and most grids leave less of a 32-wide tile empty than of a
+// 64-wide one (ms of tiles per step, 64 x 4 -> 32 x 8: 100 x 200 x 100
+// 0.52 -> 0.45, 151 x 211 x 133 1.60 -> 1.42, 200 x 160 x 120 1.30 -> 1.13;
+// where 64 x 4 fits better, 97 x 125 x 81, level: 0.37).
 static int unified_work(Ctx& c) {
   const Params& p = c.p;
   const int ni = c.d.ni, nj = c.d.nj, nk = c.d.nk;
   c.wave_tall = c.wave_pipe = c.wave_ring = c.wave_band_pipe = c.wave_surf_pipe = false;
   c.pml_fused = true;
   c.wave_ktop = nk;
-  const long tiles = (long)((nj + TJ - 1) / TJ) * ((nk + TK4 - 1) / TK4);
+  const long tiles = (long)((nj + TJN - 1) / TJN) * ((nk + TKN - 1) / TKN);
   int cus = 0, dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     cus = 256;
@@ -116,8 +120,8 @@ static int unified_work(Ctx& c) {
     // planes per block: a block takes about its planes and one more for its
     // start, the launch its blocks spread over the resident ones (two per CU)
     // and the last of them; shorter chunks for grids that would leave CUs
-    // idle (97 x 125 x 81: 3 planes, 0.42 ms of tiles per step against 0.68
-    // with 20; 151 x 211 x 133: 7 planes, 1.79 against 2.26)
+    // idle (151 x 211 x 133: 1.41 ms of tiles per step against 1.62 with 20
+    // planes; 200 x 160 x 120: 1.13 against 1.35)
     double best = 0.0;
     for (int n = std::min(ni, 2); n <= std::min(ni, 20); n++) {
       const double t = (n + 1.0) * ((double)tiles * ((ni + n - 1) / n) / (2.0 * cus) + 1.0);
@@ -126,10 +130,10 @@ static int unified_work(Ctx& c) {
   }
   std::vector<int4> all;
   for (int i0 = 0; i0 < ni; i0 += len)
-    for (int k0 = 0; k0 < nk; k0 += TK4)
-      for (int j0 = 0; j0 < nj; j0 += TJ) {
+    for (int k0 = 0; k0 < nk; k0 += TKN)
+      for (int j0 = 0; j0 < nj; j0 += TJN) {
         all.push_back(make_int4(j0, k0, i0, std::min(ni, i0 + len)));
-        all.push_back(make_int4(std::min(TJ, nj - j0), std::min((int)TK4, nk - k0), 0, 0));
+        all.push_back(make_int4(std::min((int)TJN, nj - j0), std::min((int)TKN, nk - k0), 0, 0));
       }
   for (int l = 0; l < 4; l++) c.wave_nkind[l] = 0;
   c.wave_nkind[1] = (int)all.size() / 2;
@@ -156,8 +160,9 @@ static bool bands_disjoint(const Params& p) {
 // grids each launch of one kind leaves most of the chip idle while its longest
 // block runs, and they run one after another: per step 1.26 -> 0.25 ms at
 // 30 x 80 x 50, 1.52 -> 0.41 at 97 x 125 x 81, 1.31 -> 0.65 at 100 x 200 x 100,
-// 3.00 -> 2.34 at 251 x 187 x 143.  At 400 x 300 x 200 both are level (6.5 ms),
-// and the launches of one kind keep their own tile shapes.
+// 3.00 -> 2.34 at 251 x 187 x 143.  At 400 x 300 x 200 both are level (6.2 ms
+// each, now that the tiles wait less), and the launches of one kind keep their
+// own tile shapes.
 bool wave_unified(const Params& p) {
   if (p.WaveUnified == 0 || !bands_disjoint(p)) return false;
   if (p.WaveInteriorKernel != -1 || p.WaveBandKernel != -1 || p.WaveSurfaceKernel != 1 || p.WaveSurfaceTiles != 1 ||

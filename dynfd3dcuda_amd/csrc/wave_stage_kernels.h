@@ -304,25 +304,24 @@ __global__ void __launch_bounds__(256) image_top_kernel(WaveArgs<MT> a) {
       hv[c] += d * rb[ax];
     }
   }
-  const long plane = (long)ni * nj;
-  const long ij = (long)i * nj + j;
-  for (int c = 0; c < 3; c++) a.itop[((long)c * 3 + row) * plane + ij] = hv[c] * rrhojac;
+  float* w = a.itop + (size_t)i * 18 * nj + j;
+  for (int c = 0; c < 3; c++) w[(size_t)(c * 3 + row) * nj] = hv[c] * rrhojac;
   if (row == 2) {
     const float* mVx = a.cold.mVx + ((long)(j + 3) + (long)x * ny) * 9;
     const float* mVy = a.cold.mVy + ((long)(j + 3) + (long)x * ny) * 9;
     float dxv[3], dyv[3];
     for (int c = 0; c < 3; c++) {
-      const float* w = a.Win + ((size_t)x * 9 + c) * a.nyz + col;
+      const float* v = a.Win + ((size_t)x * 9 + c) * a.nyz + col;
       const long st = 9L * a.nyz;
-      dxv[c] = a.rDH * (FX > 0 ? drp5<1>(w[-st], w[0], w[st], w[2 * st], w[3 * st])
-                               : drp5<-1>(w[-3 * st], w[-2 * st], w[-st], w[0], w[st]));
-      dyv[c] = a.rDH * (FY > 0 ? drp5<1>(w[-1], w[0], w[1], w[2], w[3]) : drp5<-1>(w[-3], w[-2], w[-1], w[0], w[1]));
+      dxv[c] = a.rDH * (FX > 0 ? drp5<1>(v[-st], v[0], v[st], v[2 * st], v[3 * st])
+                               : drp5<-1>(v[-3 * st], v[-2 * st], v[-st], v[0], v[st]));
+      dyv[c] = a.rDH * (FY > 0 ? drp5<1>(v[-1], v[0], v[1], v[2], v[3]) : drp5<-1>(v[-3], v[-2], v[-1], v[0], v[1]));
     }
     for (int r = 0; r < 3; r++) {
-      a.itop[(9 + r) * plane + ij] = mVx[3 * r] * dxv[0] + mVx[3 * r + 1] * dxv[1] + mVx[3 * r + 2] * dxv[2]
-                                   + mVy[3 * r] * dyv[0] + mVy[3 * r + 1] * dyv[1] + mVy[3 * r + 2] * dyv[2];
-      a.itop[(12 + r) * plane + ij] = mVx[3 * r] * dxv[0] + mVx[3 * r + 1] * dxv[1] + mVx[3 * r + 2] * dxv[2];
-      a.itop[(15 + r) * plane + ij] = mVy[3 * r] * dyv[0] + mVy[3 * r + 1] * dyv[1] + mVy[3 * r + 2] * dyv[2];
+      w[(size_t)(9 + r) * nj] = mVx[3 * r] * dxv[0] + mVx[3 * r + 1] * dxv[1] + mVx[3 * r + 2] * dxv[2]
+                               + mVy[3 * r] * dyv[0] + mVy[3 * r + 1] * dyv[1] + mVy[3 * r + 2] * dyv[2];
+      w[(size_t)(12 + r) * nj] = mVx[3 * r] * dxv[0] + mVx[3 * r + 1] * dxv[1] + mVx[3 * r + 2] * dxv[2];
+      w[(size_t)(15 + r) * nj] = mVy[3 * r] * dyv[0] + mVy[3 * r + 1] * dyv[1] + mVy[3 * r + 2] * dyv[2];
     }
   }
 }
@@ -501,9 +500,9 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
         h[7] += (e2 * dzv[0] + e0 * dzv[2]) * mu;
         h[8] += (e2 * dzv[1] + e1 * dzv[2]) * mu;
         {  // the image velocity RHS (image_top_kernel)
-          const long plane = (long)ni * nj, o = ((long)(k - (nk - 3))) * plane + (long)i * nj + j;
+          const float* w = a.itop + ((size_t)i * 18 + (k - (nk - 3))) * nj + j;
 #pragma unroll
-          for (int c = 0; c < 3; c++) h[c] = a.itop[(long)c * 3 * plane + o];
+          for (int c = 0; c < 3; c++) h[c] = w[(size_t)c * 3 * nj];
         }
       }
 
@@ -660,8 +659,9 @@ __device__ __forceinline__ void arrived(uint32_t v) { asm volatile("" ::"v"(v));
 template <int FX, int FY, int FZ, class MT, int TJ_, int NT_, int MINB, bool BAND = false, bool RING = true,
           bool TOP = false>
 __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a) {
-  static_assert(!TOP || (BAND && TJ_ == 64), "free-surface tiles: band terms, one k row per wavefront");
+  static_assert(!TOP || (BAND && 64 % TJ_ == 0), "free-surface tiles: band terms, whole k rows per wavefront");
   constexpr int TJ = TJ_, TK = NT_ / TJ_;
+  constexpr int WR = 64 % TJ_ == 0 ? 64 / TJ_ : TK;  // k rows of a wavefront (of the tile if they do not divide)
   constexpr int LJ = TJ + 4, LK = TK + 4;
   // halo cells of one plane: the 4 k-halo rows over the tile's own columns
   // and 4 j-halo cells per row; the corners of the LDS tile are neither
@@ -699,7 +699,7 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
   const int tj = threadIdx.x, tk = threadIdx.y, tid = tj + tk * TJ;
   const int ni = a.ni, nj = a.nj, nk = a.nk;
   const int j = j0 + tj, k = k0 + tk;
-  const int ku = TJ == 64 ? k0 + __builtin_amdgcn_readfirstlane(tk) : k;  // k, uniform where a wavefront is one row
+  const int ku = k0 + (WR < TK ? __builtin_amdgcn_readfirstlane(tk) : 0);  // first of the wavefront's rows, uniform
   // A lane without a point of the tile computes what its cells give and stores
   // nothing (its stores' offsets are out of range), so that the plane loop
   // branches on uniform values alone; a wavefront without any has a loop of
@@ -785,9 +785,7 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
     if (pml) {
       const int ja = j0 + we.z, jb = j0 + we.x;
       hasy = (a.cold.on[2] && ja < N) || (a.cold.on[3] && jb > nj - N);
-      // rows of this wavefront: one for the 64-wide tiles, else any of the tile's
-      const int ka = TJ == 64 ? ku : k0 + we.w, kb = TJ == 64 ? ka + 1 : k0 + we.y;
-      hasz = (a.cold.on[4] && ka < N) || (a.cold.on[5] && kb > nk - N);
+      hasz = (a.cold.on[4] && ku < N) || (a.cold.on[5] && ku + WR > nk - N);
     }
     if (act && pml) {
       rb2 = 1.0f / a.cold.pB[1][j];
@@ -971,13 +969,15 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
         return FZ > 0 ? drp5<1>(L[c][lk - 1][lj], L[c][lk][lj], L[c][lk + 1][lj], L[c][lk + 2][lj], L[c][lk + 3][lj])
                       : drp5<-1>(L[c][lk - 3][lj], L[c][lk - 2][lj], L[c][lk - 1][lj], L[c][lk][lj], L[c][lk + 1][lj]);
       };
-      // TOP: the words of the surface rows from image_top_kernel
-      const bool top = TOP && ap->freenode && ku >= nk - 3;  // uniform
-      auto top_word = [&](int p) {  // plane p of the surface words
-        return bld(__builtin_amdgcn_make_buffer_rsrc(ap->itop + ((size_t)p * ni + i) * nj, (short)0, nj * 4, kBufWord3),
-                   (uint32_t)j << 2, 0);
+      // TOP: whether the wavefront has surface rows (uniform), the lane's
+      // surface row, and word p of its surface words (image_top_kernel)
+      const bool top = TOP && ap->freenode && ku + WR > nk - 3;
+      const bool last = top && ku + WR > nk - 1;
+      const int row = (WR == 1 ? ku : k) - (nk - 3);
+      auto top_word = [&](int p, bool mine) {
+        return bld(__builtin_amdgcn_make_buffer_rsrc(ap->itop + (size_t)i * 18 * nj, (short)0, 18 * nj * 4, kBufWord3),
+                   mine ? (uint32_t)(p * nj + j) << 2 : kNoWord, 0);
       };
-      float tv3[3], tz[3];
       // one step of the auxiliary ODE of the lane's point on its face along
       // axis AX: aux' = -(alpha + d) aux + d * RHS_axis, RHS_axis from the
       // plain derivative along the axis, with the RK4 stage combine; y the
@@ -993,13 +993,16 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
         for (int c = 0; c < 9; c++) dd[c] = rDH * D(c);
 #pragma unroll
         for (int c = 0; c < 9; c++) ah[c] = ad1 * y[c] + d1 * axis_rhs_c(c, dd, e0, e1, e2, rrho, lam, l2m, mu);
-        if (TOP && ax < 2 && top && ku == nk - 1) {  // the traction-free term (pmlx.cu:185-210)
+        if (TOP && ax < 2 && last) {  // the traction-free term (pmlx.cu:185-210)
           const float c0 = d1 * (ax == 0 ? uni(cold->pB[0], i) : cold->pB[1][min(j, nj - 1)]);
           float z1[3];
 #pragma unroll
-          for (int r = 0; r < 3; r++) z1[r] = top_word(12 + 3 * ax + r);
+          for (int r = 0; r < 3; r++) z1[r] = top_word(12 + 3 * ax + r, row == 2);
 #pragma unroll
-          for (int c = 3; c < 9; c++) ah[c] += pml_fs_term(c, z1, ztx, zty, ztz, lam, l2m, mu, c0);
+          for (int c = 3; c < 9; c++) {
+            const float v = ah[c] + pml_fs_term(c, z1, ztx, zty, ztz, lam, l2m, mu, c0);
+            ah[c] = row == 2 ? v : ah[c];
+          }
         }
         if (irk == 0) {  // the accumulator is derived in stage 1 (rk_derived_t)
           on(cold->axS[ax], st9(y));
@@ -1031,44 +1034,46 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
         const float s1 = rb1 * rDH, s2 = rb2 * rDH, s3 = rb3 * rDH;
         accum_axis(h, Dx, xix * s1, xiy * s1, xiz * s1, rrho, lam, l2m, mu, true);
         accum_axis(h, Dy, etx * s2, ety * s2, etz * s2, rrho, lam, l2m, mu, true);
-        if (top) {
+        if (!top) {
+          accum_axis(h, Dz, ztx * s3, zty * s3, ztz * s3, rrho, lam, l2m, mu, true);
+        } else {
+          // the top three rows under the free surface (wave.cu:207-245), as
+          // the general kernel computes them: DzV of the stress rates from the
+          // traction-free condition, L22 or L24, and the velocity RHS of the
+          // image.  A wavefront's rows that are no surface rows keep the
+          // general sums; by selects, since its rows may be of any of the four
+          // kinds.
+          float hs[6], tz[3], hv3[3];
+          const bool mine = row >= 0 && row < 3;
 #pragma unroll
-          for (int c = 0; c < 3; c++) tv3[c] = top_word(3 * c + ku - (nk - 3));
-          if (ku == nk - 1) {
+          for (int c = 0; c < 6; c++) hs[c] = h[3 + c];
+          accum_axis(h, Dz, ztx * s3, zty * s3, ztz * s3, rrho, lam, l2m, mu, WR > 1);
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int c = 0; c < 3; c++) tz[c] = top_word(9 + c);
-          }
-        }
-        accum_axis(h, Dz, ztx * s3, zty * s3, ztz * s3, rrho, lam, l2m, mu, !top);
-      }
-      if constexpr (TOP) {
-        // the top three rows under the free surface (wave.cu:207-245), as
-        // the general kernel computes them: DzV of the stress rates from the
-        // traction-free condition, L22 or L24, and the velocity RHS of the
-        // image (image_top_kernel); one k row per wavefront
-        if (top) {
+          for (int c = 0; c < 3; c++) tz[c] = top_word(9 + c, row == 2);
           float dzv[3];
-          if (ku == nk - 1) {  // traction-free condition (wave.cu:207-232, image_top_kernel)
 #pragma unroll
-            for (int c = 0; c < 3; c++) dzv[c] = tz[c];
-          } else if (ku == nk - 2) {  // L22 (wave.cu:233-238)
-#pragma unroll
-            for (int c = 0; c < 3; c++) dzv[c] = rDH * (FZ > 0 ? L[c][lk + 1][lj] - L[c][lk][lj] : L[c][lk][lj] - L[c][lk - 1][lj]);
-          } else {  // L24 (wave.cu:239-245)
-#pragma unroll
-            for (int c = 0; c < 3; c++)
-              dzv[c] = rDH * (FZ > 0 ? -C24_1 * L[c][lk][lj] + C24_2 * L[c][lk + 1][lj] - C24_3 * L[c][lk + 2][lj]
-                                     : C24_3 * L[c][lk - 2][lj] - C24_2 * L[c][lk - 1][lj] + C24_1 * L[c][lk][lj]);
+          for (int c = 0; c < 3; c++) {
+            const float l22 = rDH * (FZ > 0 ? L[c][lk + 1][lj] - L[c][lk][lj] : L[c][lk][lj] - L[c][lk - 1][lj]);
+            const float l24 = rDH * (FZ > 0 ? -C24_1 * L[c][lk][lj] + C24_2 * L[c][lk + 1][lj] - C24_3 * L[c][lk + 2][lj]
+                                            : C24_3 * L[c][lk - 2][lj] - C24_2 * L[c][lk - 1][lj] + C24_1 * L[c][lk][lj]);
+            dzv[c] = row == 2 ? tz[c] : row == 1 ? l22 : l24;
           }
           const float e0 = ztx * rb3, e1 = zty * rb3, e2 = ztz * rb3;
-          h[3] += (l2m * e0 * dzv[0] + lam * e1 * dzv[1] + lam * e2 * dzv[2]);
-          h[4] += (lam * e0 * dzv[0] + l2m * e1 * dzv[1] + lam * e2 * dzv[2]);
-          h[5] += (lam * e0 * dzv[0] + lam * e1 * dzv[1] + l2m * e2 * dzv[2]);
-          h[6] += (e1 * dzv[0] + e0 * dzv[1]) * mu;
-          h[7] += (e2 * dzv[0] + e0 * dzv[2]) * mu;
-          h[8] += (e2 * dzv[1] + e1 * dzv[2]) * mu;
+          hs[0] += (l2m * e0 * dzv[0] + lam * e1 * dzv[1] + lam * e2 * dzv[2]);
+          hs[1] += (lam * e0 * dzv[0] + l2m * e1 * dzv[1] + lam * e2 * dzv[2]);
+          hs[2] += (lam * e0 * dzv[0] + lam * e1 * dzv[1] + l2m * e2 * dzv[2]);
+          hs[3] += (e1 * dzv[0] + e0 * dzv[1]) * mu;
+          hs[4] += (e2 * dzv[0] + e0 * dzv[2]) * mu;
+          hs[5] += (e2 * dzv[1] + e1 * dzv[2]) * mu;
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int c = 0; c < 3; c++) h[c] = tv3[c];
+          for (int c = 0; c < 3; c++) hv3[c] = top_word(3 * c + row, mine);
+#pragma unroll
+          for (int c = 0; c < 9; c++) {
+            const float v = c < 3 ? hv3[c % 3] : hs[(c + 3) % 6];
+            h[c] = mine || WR == 1 ? v : h[c];
+          }
         }
       }
       if constexpr (BAND) {
@@ -1358,8 +1363,8 @@ void launch_wave_t(WaveArgs<MT> a, const Ctx& c, hipStream_t s) {
     pr.begin(s, PK_STAGE_BAND);
     if (a.freenode) launch_image<FX, FY, FZ, MT>(a, c, s);
     a.work = w; a.nwork = n[1];
-    hipLaunchKernelGGL((wave_interior_kernel<FX, FY, FZ, MT, TJ, TJ * TK4, 2, true, false, true>), dim3(a.nwork),
-                       dim3(TJ, TK4, 1), 0, s, a);
+    hipLaunchKernelGGL((wave_interior_kernel<FX, FY, FZ, MT, TJN, NTHRN, 2, true, false, true>), dim3(a.nwork),
+                       dim3(TJN, TKN, 1), 0, s, a);
     pr.end(s);
     return;
   }
