@@ -73,105 +73,229 @@ struct GradArgs {
   const int* idx;       // sample order, or null for 0..count-1
   long first, count;    // samples idx[first .. first+count)
   float gscale;         // 2 / count
-  float lscale;         // loss weight of one squared error
-  float* grad;          // [kMlpParams], accumulated
-  float* loss;          // accumulated
+  float* part;          // [gridDim.x][kGradRow] sums of each block
 };
 
-// Gradient of the loss over a batch.  A block is one wavefront; lane l owns
-// hidden unit l of both layers for the accumulation (W1[l][:], b1[l],
-// W2[l][:], b2[l], w3[l]) and lane 0 also b3.  Per chunk of 64 samples every
-// lane runs forward and backward for its own sample in registers, and the
-// per-sample outer products are summed through LDS.
-__global__ void __launch_bounds__(64) mlp_grad_kernel(GradArgs a) {
-  __shared__ float bufA[64][65];  // per-sample rows: h2, then dz2 ... (padded: conflict-free row writes)
-  __shared__ float bufB[64][65];  // h1, then dz1
-  __shared__ float xs[64][4];
-  __shared__ float dos[64];
+constexpr int kGradWaves = 4;          // wavefronts of a gradient block
+constexpr int kGradBlocks = 256;       // blocks at most: one per CU
+constexpr int kGradRow = kMlpParams + 1;  // gradient, then the sum of squared errors
+
+// Blocks of the gradient kernel for a batch of count samples.
+inline int grad_blocks(long count) {
+  return (int)std::min<long>((count + 16 * kGradWaves - 1) / (16 * kGradWaves), kGradBlocks);
+}
+
+// Gradient of the loss over a batch, on the matrix cores: a wavefront takes
+// 16 samples at a time and keeps its sums of all parameters in registers.
+// With g = lane / 16 and c = lane % 16, the matrix instructions hand out their
+// result as D[4 g + r][c] and take operand element r of k-slot g, so a result
+// is the next product's operand as it stands when the contracted index is its
+// row.  The hidden layers are therefore computed in both orientations, rows
+// of units ("u", unit 16 t + 4 g + r of sample c) and rows of samples ("s",
+// sample 4 g + r at unit 16 t + c), and nothing goes through LDS:
+//   z2 (u and s)   bf16 products, FP32 sums, as in the forward pass
+//   dW2 = dz2 h1^T   samples contracted: s operands, FP32 products
+//   dz1 = W2^T dz2   hidden units contracted: u operand, FP32 products
+// 128 FP32 and 32 bf16 matrix instructions per 16 samples.  The blocks' sums
+// go to rows of a buffer that a second kernel adds up.  A scalar form (a lane
+// per sample, products summed through LDS, every block adding its 4555 words
+// to the same addresses) took 570 us at 60000 samples and 2.0 ms at 500000;
+// this one 34 and 184 us, of which the FP32 matrix instructions are about a
+// third (one wavefront per SIMD: 447 registers), and the sum kernel 4 us.
+__global__ void __launch_bounds__(64 * kGradWaves, 1) mlp_grad_kernel(GradArgs a) {
+  __shared__ __align__(16) float sW1[kMlpH][kMlpIn], sb1[kMlpH], sb2[kMlpH], sw3[kMlpH];
+  __shared__ float sum[kGradWaves][kGradRow];
   const MlpDev* __restrict__ m = a.m;
-  const int l = threadIdx.x;
-  float gW2[kMlpH], gW1[4] = {0, 0, 0, 0}, gb1 = 0, gb2 = 0, gw3 = 0, gb3 = 0, lsum = 0;
-  for (int i = 0; i < kMlpH; i++) gW2[i] = 0.0f;
-  const long nchunk = (a.count + 63) / 64;
-  for (long ch = blockIdx.x; ch < nchunk; ch += gridDim.x) {
-    const long r = ch * 64 + l;
-    const bool ok = r < a.count;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
+  for (int t = tid; t < kMlpH * kMlpIn; t += 64 * kGradWaves) sW1[t / kMlpIn][t % kMlpIn] = m->W1[t / kMlpIn][t % kMlpIn];
+  if (tid < kMlpH) {
+    sb1[tid] = m->b1[tid];
+    sb2[tid] = m->b2[tid];
+    sw3[tid] = m->w3[tid];
+  }
+  __syncthreads();
+  bf16x4 w2[4][4];      // [t][k][r]: W2[16 t + c][16 k + 4 g + r]
+  float w2t[4][4][4];   // [k][t][r]: W2[16 k + 4 g + r][16 t + c]
+#pragma unroll
+  for (int t = 0; t < 4; t++)
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint16_t* q = &m->W2[16 * t + c][16 * k + 4 * g];
+      w2[t][k] = bf16x4{(short)q[0], (short)q[1], (short)q[2], (short)q[3]};
+#pragma unroll
+      for (int r = 0; r < 4; r++) w2t[k][t][r] = bf2f(m->W2[16 * k + 4 * g + r][16 * t + c]);
+    }
+  f32x4 gW2[4][4];  // hidden unit 16 [.] + 4 g + r, first-layer unit 16 [.] + c
+  float gW1[4][kMlpIn], gb1[4], gb2[4], gw3[4], gb3 = 0.0f, lsum = 0.0f;
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    gb1[t] = gb2[t] = gw3[t] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      gW2[t][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      gW1[t][k] = 0.0f;
+    }
+  }
+  const long ntile = (a.count + 15) / 16;
+  for (long tile = (long)blockIdx.x * kGradWaves + w; tile < ntile; tile += (long)gridDim.x * kGradWaves) {
+    const long q = tile * 16 + c;
+    const bool ok = q < a.count;
     long s = 0;
-    if (ok) s = a.idx ? (long)a.idx[a.first + r] : a.first + r;
-    float x[4];
-    for (int i = 0; i < 4; i++) x[i] = ok ? (a.feat[4 * s + i] - m->xmean[i]) * m->xscale[i] : 0.0f;
-    float h1[kMlpH];
+    if (ok) s = a.idx ? (long)a.idx[a.first + q] : a.first + q;
+    float x[kMlpIn], xs[kMlpIn][4];  // standardised features of sample c, and of samples 4 g + r
 #pragma unroll
-    for (int h = 0; h < kMlpH; h++) h1[h] = mlp_h1(m, h, x);
-    float o = m->b3;
-    float h2[kMlpH];
+    for (int i = 0; i < kMlpIn; i++) {
+      x[i] = ok ? (a.feat[4 * s + i] - m->xmean[i]) * m->xscale[i] : 0.0f;
 #pragma unroll
-    for (int h = 0; h < kMlpH; h++) {
-      float z = 0.0f;
-#pragma unroll
-      for (int i = 0; i < kMlpH; i++) z += bf2f(m->W2[h][i]) * h1[i];
-      h2[h] = fmaxf(z + m->b2[h], 0.0f);
-      o += m->w3[h] * h2[h];
+      for (int r = 0; r < 4; r++) xs[i][r] = __shfl(x[i], 4 * g + r);
     }
     const float tn = ok ? (a.target[s] - m->ymean) / m->yscale : 0.0f;
-    const float e = ok ? o - tn : 0.0f;
-    lsum += e * e;
+    bf16x4 h1u[4];
+    float h1s[4][4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int u = 16 * t + 4 * g + r, v = 16 * t + c;
+        float zu = sb1[u], zs = sb1[v];
+#pragma unroll
+        for (int i = 0; i < kMlpIn; i++) {
+          zu = fmaf(sW1[u][i], x[i], zu);
+          zs = fmaf(sW1[v][i], xs[i][r], zs);
+        }
+        h1u[t][r] = (short)f2bf(fmaxf(zu, 0.0f));
+        h1s[t][r] = bf2f(f2bf(fmaxf(zs, 0.0f)));
+      }
+    }
+    f32x4 zu[4], zs[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      zu[t] = zs[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        zu[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w2[t][k], h1u[k], zu[t], 0, 0, 0);
+        zs[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(h1u[k], w2[t][k], zs[t], 0, 0, 0);
+      }
+    }
+    float o = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int u = 16 * t + 4 * g + r;
+        zu[t][r] = fmaxf(zu[t][r] + sb2[u], 0.0f);
+        o += sw3[u] * zu[t][r];
+      }
+    o += __shfl_xor(o, 16);
+    o += __shfl_xor(o, 32);
+    const float e = ok ? o + m->b3 - tn : 0.0f;
     const float dout = a.gscale * e;
-    for (int i = 0; i < 4; i++) xs[l][i] = x[i];
-    dos[l] = dout;
+    lsum += e * e;
+    gb3 += dout;
+    float ds[4];
 #pragma unroll
-    for (int h = 0; h < kMlpH; h++) {
-      bufA[l][h] = h2[h];
-      bufB[l][h] = h1[h];
+    for (int r = 0; r < 4; r++) ds[r] = __shfl(dout, 4 * g + r);
+    // dz2 in both orientations (in place of the layer's values)
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const float b2 = sb2[16 * t + c], w3 = sw3[16 * t + c];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        zu[t][r] = zu[t][r] > 0.0f ? dout * sw3[16 * t + 4 * g + r] : 0.0f;
+        const float h2 = fmaxf(zs[t][r] + b2, 0.0f);
+        gw3[t] += ds[r] * h2;
+        zs[t][r] = h2 > 0.0f ? ds[r] * w3 : 0.0f;
+        gb2[t] += zs[t][r];
+      }
     }
-    __syncthreads();
-    for (int q = 0; q < 64; q++) {  // w3, b3
-      gw3 += dos[q] * bufA[q][l];
-      gb3 += dos[q];
-    }
-    __syncthreads();
-    // dz2 of this lane's sample
-    float dz2[kMlpH];
 #pragma unroll
-    for (int h = 0; h < kMlpH; h++) dz2[h] = h2[h] > 0.0f ? dout * m->w3[h] : 0.0f;
+    for (int r = 0; r < 4; r++)
 #pragma unroll
-    for (int h = 0; h < kMlpH; h++) bufA[l][h] = dz2[h];
-    __syncthreads();
-    for (int q = 0; q < 64; q++) {  // W2 row l, b2[l]
-      const float d = bufA[q][l];
-      gb2 += d;
+      for (int t = 0; t < 4; t++)
 #pragma unroll
-      for (int i = 0; i < kMlpH; i++) gW2[i] += d * bufB[q][i];
-    }
-    __syncthreads();
-    // dz1 of this lane's sample: (W2^T dz2) masked by the first layer's ReLU
-    float d1[kMlpH];
+        for (int k = 0; k < 4; k++) gW2[t][k] = __builtin_amdgcn_mfma_f32_16x16x4f32(zs[t][r], h1s[k][r], gW2[t][k], 0, 0, 0);
+    f32x4 d1[4];
 #pragma unroll
-    for (int i = 0; i < kMlpH; i++) d1[i] = 0.0f;
+    for (int t = 0; t < 4; t++) d1[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int h = 0; h < kMlpH; h++)
+    for (int k = 0; k < 4; k++)
 #pragma unroll
-      for (int i = 0; i < kMlpH; i++) d1[i] += bf2f(m->W2[h][i]) * dz2[h];
+      for (int r = 0; r < 4; r++)
 #pragma unroll
-    for (int i = 0; i < kMlpH; i++) bufB[l][i] = h1[i] > 0.0f ? d1[i] : 0.0f;
-    __syncthreads();
-    for (int q = 0; q < 64; q++) {  // W1 row l, b1[l]
-      const float d = bufB[q][l];
-      gb1 += d;
-      for (int i = 0; i < 4; i++) gW1[i] += d * xs[q][i];
-    }
-    __syncthreads();
+        for (int t = 0; t < 4; t++) d1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(zu[k][r], w2t[k][t][r], d1[t], 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const float d = h1s[t][r] > 0.0f ? d1[t][r] : 0.0f;
+        gb1[t] += d;
+#pragma unroll
+        for (int i = 0; i < kMlpIn; i++) gW1[t][i] += d * xs[i][r];
+      }
   }
-  float* g = a.grad;
-  for (int i = 0; i < 4; i++) atomicAdd(&g[kOffW1 + l * kMlpIn + i], gW1[i]);
-  atomicAdd(&g[kOffB1 + l], gb1);
+  // this wavefront's sums, then the block's
+  auto over_g = [](float v) {
+    v += __shfl_xor(v, 16);
+    return v + __shfl_xor(v, 32);
+  };
+  auto over_c = [](float v) {
+    for (int k = 1; k < 16; k *= 2) v += __shfl_xor(v, k);
+    return v;
+  };
+  float* row = sum[w];
 #pragma unroll
-  for (int i = 0; i < kMlpH; i++) atomicAdd(&g[kOffW2 + l * kMlpH + i], gW2[i]);
-  atomicAdd(&g[kOffB2 + l], gb2);
-  atomicAdd(&g[kOffW3 + l], gw3);
-  if (l == 0) atomicAdd(&g[kOffB3], gb3);
-  for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
-  if (l == 0) atomicAdd(a.loss, lsum * a.lscale);
+  for (int t = 0; t < 4; t++) {
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) row[kOffW2 + (16 * t + 4 * g + r) * kMlpH + 16 * k + c] = gW2[t][k][r];
+    const int u = 16 * t + c;
+    const float b1 = over_g(gb1[t]), b2 = over_g(gb2[t]), w3 = over_g(gw3[t]);
+    float w1[kMlpIn];
+#pragma unroll
+    for (int i = 0; i < kMlpIn; i++) w1[i] = over_g(gW1[t][i]);
+    if (g == 0) {
+      row[kOffB1 + u] = b1;
+      row[kOffB2 + u] = b2;
+      row[kOffW3 + u] = w3;
+#pragma unroll
+      for (int i = 0; i < kMlpIn; i++) row[kOffW1 + u * kMlpIn + i] = w1[i];
+    }
+  }
+  gb3 = over_c(gb3);
+  lsum = over_c(lsum);
+  if (lane < kOffW1) row[lane] = 0.0f;
+  if (lane == 0) {
+    row[kOffB3] = gb3;
+    row[kMlpParams] = lsum;
+  }
+  __syncthreads();
+  for (int p = tid; p < kGradRow; p += 64 * kGradWaves) {
+    float v = sum[0][p];
+    for (int k = 1; k < kGradWaves; k++) v += sum[k][p];
+    a.part[(size_t)blockIdx.x * kGradRow + p] = v;
+  }
+}
+
+// Sums the blocks' rows: grad set, the loss (lscale times the squared errors)
+// added to.  32 parameters x 8 row groups per block.
+__global__ void __launch_bounds__(256) mlp_grad_sum_kernel(const float* __restrict__ part, int nrow,
+                                                           float* __restrict__ grad, float* __restrict__ loss,
+                                                           float lscale) {
+  __shared__ float s[8][33];
+  const int c = threadIdx.x & 31, q = threadIdx.x >> 5, p = blockIdx.x * 32 + c;
+  float v = 0.0f;
+  if (p < kGradRow) {
+#pragma unroll 8
+    for (int r = q; r < nrow; r += 8) v += part[(size_t)r * kGradRow + p];
+  }
+  s[q][c] = v;
+  __syncthreads();
+  if (q == 0 && p < kGradRow) {
+    for (int k = 1; k < 8; k++) v += s[k][c];
+    if (p < kMlpParams) grad[p] = v;
+    else loss[0] += v * lscale;
+  }
 }
 
 __global__ void __launch_bounds__(256) mlp_fill_kernel(float* __restrict__ p, int n) {
@@ -229,17 +353,18 @@ void pack_on(hipStream_t s, const float* P, MlpDev* m) {
   hipLaunchKernelGGL(mlp_pack_kernel, dim3(16), dim3(256), 0, s, P, m);
 }
 
+// grad: kMlpParams words and, behind them, the rows of the blocks' sums
+size_t grad_words(long count) { return kMlpParams + (size_t)grad_blocks(count) * kGradRow; }
+
 void grad_on(hipStream_t s, const MlpDev* m, const float* feat, const float* target, const int* idx, long first,
              long count, float lscale, float* grad, float* loss) {
   GradArgs a;
   a.m = m; a.feat = feat; a.target = target; a.idx = idx; a.first = first; a.count = count;
   a.gscale = 2.0f / (float)count;
-  a.lscale = lscale;
-  a.grad = grad; a.loss = loss;
-  const long nchunk = (count + 63) / 64;
-  const int grid = (int)std::min<long>(nchunk, 2048);
-  hipLaunchKernelGGL(mlp_fill_kernel, dim3((kMlpParams + 255) / 256), dim3(256), 0, s, grad, kMlpParams);
-  hipLaunchKernelGGL(mlp_grad_kernel, dim3(grid), dim3(64), 0, s, a);
+  a.part = grad + kMlpParams;
+  const int grid = grad_blocks(count);
+  if (grid > 0) hipLaunchKernelGGL(mlp_grad_kernel, dim3(grid), dim3(64 * kGradWaves), 0, s, a);
+  hipLaunchKernelGGL(mlp_grad_sum_kernel, dim3((kGradRow + 31) / 32), dim3(256), 0, s, a.part, grid, grad, loss, lscale);
 }
 
 }  // namespace
@@ -313,7 +438,7 @@ int mlp_grad_host(const float* blob, const float* feat, const float* target, lon
   MlpDev* m = bm.alloc<MlpDev>(1);
   float* f = bf.alloc<float>(4 * n);
   float* t = bt.alloc<float>(n);
-  float* g = bg.alloc<float>(kMlpParams);
+  float* g = bg.alloc<float>(grad_words(n));
   float* l = bl.alloc<float>(1);
   if (!st.s || !P || !m || !f || !t || !g || !l) { err = "hipMalloc failed"; return 1; }
   if (hip_ok(hipMemcpyAsync(P, blob, kMlpParams * sizeof(float), hipMemcpyHostToDevice, st.s), "copy", err) ||
@@ -337,7 +462,7 @@ int mlp_train_host(float* blob, const float* feat, const float* target, long n, 
   MlpDev* m = bm.alloc<MlpDev>(1);
   float* f = bf.alloc<float>(4 * n);
   float* t = bt.alloc<float>(n);
-  float* g = bg.alloc<float>(kMlpParams);
+  float* g = bg.alloc<float>(grad_words(std::min<long>(batch, n)));
   float* l = bl.alloc<float>(epochs);
   float* m1 = bm1.alloc<float>(kMlpParams);
   float* m2 = bm2.alloc<float>(kMlpParams);
