@@ -99,6 +99,15 @@ static int put_work(Ctx& c, const std::vector<int4>& all) {
   return 0;
 }
 
+// Compute units of the current device.
+static int cu_count() {
+  int cus = 0, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus <= 0)
+    cus = 256;
+  return cus;
+}
+
 // The work list of the unified launch: 32 x 8 tiles over the whole grid, in
 // chunks of planes.  A wavefront's time is the same for a full and for a
 // partial tile, and most grids leave less of a 32-wide tile empty than of a
@@ -112,9 +121,7 @@ static int unified_work(Ctx& c) {
   c.pml_fused = true;
   c.wave_ktop = nk;
   const long tiles = (long)((nj + TJN - 1) / TJN) * ((nk + TKN - 1) / TKN);
-  int cus = 0, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    cus = 256;
+  const int cus = cu_count();
   int len = p.WaveBandIChunk;
   if (len <= 0) {
     // planes per block: a block takes about its planes and one more for its
@@ -216,11 +223,9 @@ int upload_wave_work(Ctx& c) {
   // leave the last ones ragged: 1600 x 1000 x 500, 88 k blocks: 90-95 ms of
   // interior per step against 96-101 for 1; 400 x 300 x 200, 2 k blocks:
   // 2.67 against 2.49 ms), else 1
+  const int cus = cu_count();
   int wik = p.WaveInteriorKernel;
   if (wik < 0) {
-    int cus = 0, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      cus = 256;
     const long ej = std::max(0, n3[1] - lo[1] - hi[1]), ek = std::max(0, n3[2] - lo[2] - hi[2]);
     const long span = std::max(0, n3[0] - lo[0] - hi[0]);
     const long blocks4 = (ej / TJ) * (ek / TK4) * ((span + 31) / 32);
@@ -289,7 +294,22 @@ int upload_wave_work(Ctx& c) {
   // (1600 x 1000 x 500: 97.7 ms of interior per step against 106.2 for the
   // ~300-plane chunks of a 4096-block target and 104.5 for 16 planes;
   // 400 x 300 x 200: 2.44 against 2.70 ms for ~8 planes).
+  // With one block per CU and few rounds of blocks (the ring kernel) the
+  // launch takes its rounds times the planes of a block and about two more
+  // for its start, and the last round may be nearly empty: the length that
+  // takes the least (400 x 300 x 200, 84 tiles of 360 planes: 120 planes in
+  // one round, 2.16 ms of interior per step; 2.37 with 32, 2.92 with 90).
+  auto rounds_chunk = [&](int span, long ntiles) {
+    int len = std::max(span, 1);
+    long best = 0;
+    for (int n = std::min(len, 8); n <= std::max(span, 1); n++) {
+      const long t = (n + 2) * ((ntiles * ((span + n - 1) / n) + cus - 1) / cus);
+      if (best == 0 || t < best) { best = t; len = n; }
+    }
+    return len;
+  };
   const int ich_in = p.WaveIChunk > 0 ? p.WaveIChunk
+                     : c.wave_ring   ? rounds_chunk(ib - ia, tiles_in)
                      : c.wave_pipe   ? std::min(std::max(ib - ia, 1), 32)
                                      : chunk(ib - ia, tiles_in, tall ? 2048 : 4096, 4);
   // band tiles stream 20 planes (1600 x 1000 x 500: 23.4 ms per step against
