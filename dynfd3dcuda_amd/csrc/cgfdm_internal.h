@@ -64,7 +64,7 @@ struct Params {
   int WaveBandIChunk = 0;  // planes per block of the band tiles (0: automatic)
   int WaveTopIChunk = 0;  // planes per block of the free-surface tiles (0: automatic)
   int WaveSurfaceTiles = 1;  // free-surface tiles = the top TK rows, own line-aligned j tiles (0: earlier layout)
-  int WaveUnified = -1;  // 1: one launch of tiles of any kind per stage; 0: one per kind; -1: 1 on small grids
+  int WaveUnified = -1;  // 1: one launch of tiles of any kind per stage, 2: one beside the interior's; 0: one per kind; -1: 1 or 2
   int WaveBandRound = 0;  // 1: low j band rounded up to whole 64-wide tiles (0: band width exactly)
 
   // derived (set_params.cu:286-295)
@@ -101,7 +101,7 @@ struct Dims {
 // below it is handled by the edge instantiation).
 int interior_lo_j(const Params& p);
 bool wave_unified(const Params& p);
-constexpr double kUnifiedPoints = 12e6;
+constexpr double kBoxPoints = 4e6, kPerKindPoints = 200e6;
 
 // Fault state on the device (2-D arrays [nk][nj] unless noted).
 struct FaultDev {

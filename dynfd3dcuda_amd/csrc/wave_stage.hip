@@ -108,8 +108,36 @@ static int cu_count() {
   return cus;
 }
 
-// The work list of the unified launch: 32 x 8 tiles over the whole grid, in
-// chunks of planes.  A wavefront's time is the same for a full and for a
+// The interior kernel (WaveInteriorKernel, see upload_wave_work): -1 (default)
+// picks 3 when the interior launch holds at least 16 rounds of resident 64 x 4
+// blocks (three per CU; fewer rounds leave the last ones ragged:
+// 1600 x 1000 x 500, 88 k blocks: 90-95 ms of interior per step against
+// 96-101 for 1; 400 x 300 x 200, 2 k blocks: 2.50 against 2.16 ms), else 1.
+// cols: 64-wide tiles along j, rows along k, planes along i.
+static int interior_kernel(const Params& p, long cols, long rows, long planes, int cus) {
+  if (p.WaveInteriorKernel >= 0) return p.WaveInteriorKernel;
+  return cols * (rows / TK4) * ((planes + 31) / 32) >= 16L * 3 * cus ? 3 : 1;
+}
+
+// Planes per block of a launch with one block per CU and few rounds of blocks
+// (the ring kernel): it takes its rounds times the planes of a block and about
+// two more for its start, and the last round may be nearly empty, so the
+// length that takes the least (400 x 300 x 200, 84 tiles of 360 planes: 120
+// planes in one round, 2.16 ms of interior per step; 2.37 with 32, 2.92 with
+// 90).
+static int rounds_chunk(int span, long ntiles, int cus) {
+  int len = std::max(span, 1);
+  long best = 0;
+  for (int n = std::min(len, 8); n <= std::max(span, 1); n++) {
+    const long t = (n + 2) * ((ntiles * ((span + n - 1) / n) + cus - 1) / cus);
+    if (best == 0 || t < best) { best = t; len = n; }
+  }
+  return len;
+}
+
+// The work list of the unified launch: 32 x 8 tiles over the whole grid, or
+// over all of it but the interior box, in chunks of planes; before it the
+// box's tiles.  A wavefront's time is the same for a full and for a
 // partial tile, and most grids leave less of a 32-wide tile empty than of a
 // 64-wide one (ms of tiles per step, 64 x 4 -> 32 x 8: 100 x 200 x 100
 // 0.52 -> 0.45, 151 x 211 x 133 1.60 -> 1.42, 200 x 160 x 120 1.30 -> 1.13;
@@ -120,8 +148,49 @@ static int unified_work(Ctx& c) {
   c.wave_tall = c.wave_pipe = c.wave_ring = c.wave_band_pipe = c.wave_surf_pipe = false;
   c.pml_fused = true;
   c.wave_ktop = nk;
-  const long tiles = (long)((nj + TJN - 1) / TJN) * ((nk + TKN - 1) / TKN);
   const int cus = cu_count();
+  // the interior box [i0, i1) x [j0, j1) x [k0, k1) in whole 64 x 8 tiles on
+  // the 32 x 8 tiles' lattice (a lattice from the low bands' edges has larger
+  // boxes, but partial tiles at all four sides: 512 x 384 x 256 11.7 against
+  // 10.5 ms per step, 251 x 187 x 143 2.32 against 2.05)
+  int i0 = 0, i1 = 0, j0 = 0, j1 = 0, k0 = 0, k1 = 0;
+  if (p.WaveUnified == 2 || (p.WaveUnified < 0 && (double)p.NX * p.NY * p.NZ > kBoxPoints)) {
+    int lo[3], hi[3];
+    for (int ax = 0; ax < 3; ax++) {
+      const int damp = p.useCerjan ? p.DAMP_N : 0;
+      lo[ax] = std::max(c.pml.on[2 * ax] ? c.pml.N : 0, damp);
+      hi[ax] = ax == 2 && p.FreeSurface ? 3 : std::max(c.pml.on[2 * ax + 1] ? c.pml.N : 0, damp);
+    }
+    i0 = std::min(lo[0], ni);
+    i1 = std::max(i0, ni - hi[0]);
+    j0 = (lo[1] + TJN - 1) / TJN * TJN;
+    j1 = j0 + std::max(0, nj - hi[1] - j0) / TJ * TJ;
+    k0 = (lo[2] + TKN - 1) / TKN * TKN;
+    k1 = k0 + std::max(0, nk - hi[2] - k0) / TKN * TKN;
+    if (i1 == i0 || j1 == j0 || k1 == k0) i1 = i0;
+  }
+  const long span = i1 - i0;
+  std::vector<int4> box;
+  if (span > 0) {
+    c.wave_pipe = true;
+    c.wave_ring = interior_kernel(p, (j1 - j0) / TJ, k1 - k0, span, cus) == 1;
+    c.wave_tki = c.wave_ring ? (int)TK : (int)TK4;
+    const int len = c.wave_ring ? rounds_chunk((int)span, (long)(j1 - j0) / TJ * ((k1 - k0) / TK), cus) : std::min((int)span, 32);
+    for (int i = i0; i < i1; i += len)
+      for (int k = k0; k < k1; k += c.wave_tki)
+        for (int j = j0; j < j1; j += TJ) {
+          box.push_back(make_int4(j, k, i, std::min(i1, i + len)));
+          box.push_back(make_int4(TJ, c.wave_tki, 0, 0));
+        }
+  }
+  // the other tiles: all of them on the planes outside the box, those around
+  // it on its planes
+  const long tiles = (long)((nj + TJN - 1) / TJN) * ((nk + TKN - 1) / TKN);
+  const long around = tiles - (long)(j1 - j0) / TJN * ((k1 - k0) / TKN);
+  auto blocks = [&](int n) {
+    auto cut = [&](long planes) { return (planes + n - 1) / n; };
+    return span > 0 ? tiles * (cut(i0) + cut(ni - i1)) + around * cut(span) : tiles * cut(ni);
+  };
   int len = p.WaveBandIChunk;
   if (len <= 0) {
     // planes per block: a block takes about its planes and one more for its
@@ -131,27 +200,42 @@ static int unified_work(Ctx& c) {
     // planes; 200 x 160 x 120: 1.13 against 1.35)
     double best = 0.0;
     for (int n = std::min(ni, 2); n <= std::min(ni, 20); n++) {
-      const double t = (n + 1.0) * ((double)tiles * ((ni + n - 1) / n) / (2.0 * cus) + 1.0);
+      const double t = (n + 1.0) * ((double)blocks(n) / (2.0 * cus) + 1.0);
       if (len <= 0 || t < best) { best = t; len = n; }
     }
   }
-  std::vector<int4> all;
-  for (int i0 = 0; i0 < ni; i0 += len)
-    for (int k0 = 0; k0 < nk; k0 += TKN)
-      for (int j0 = 0; j0 < nj; j0 += TJN) {
-        all.push_back(make_int4(j0, k0, i0, std::min(ni, i0 + len)));
-        all.push_back(make_int4(std::min((int)TJN, nj - j0), std::min((int)TKN, nk - k0), 0, 0));
-      }
+  std::vector<int4> rest;
+  auto add = [&](int a, int b, bool whole) {
+    for (int i = a; i < b; i += len)
+      for (int k = 0; k < nk; k += TKN)
+        for (int j = 0; j < nj; j += TJN) {
+          if (!whole && j >= j0 && j < j1 && k >= k0 && k < k1) continue;
+          rest.push_back(make_int4(j, k, i, std::min(b, i + len)));
+          rest.push_back(make_int4(std::min((int)TJN, nj - j), std::min((int)TKN, nk - k), 0, 0));
+        }
+  };
+  if (span > 0) {
+    add(0, i0, true);
+    add(i0, i1, false);
+    add(i1, ni, true);
+  } else {
+    add(0, ni, true);
+  }
   for (int l = 0; l < 4; l++) c.wave_nkind[l] = 0;
-  c.wave_nkind[1] = (int)all.size() / 2;
+  c.wave_nkind[0] = (int)box.size() / 2;
+  c.wave_nkind[1] = (int)rest.size() / 2;
   const long N = c.pml.N;
   long pairs = 0;
   for (int f = 0; f < 6; f++)
     if (c.pml.on[f]) pairs += N * (f < 2 ? (long)nj * nk : f < 4 ? (long)ni * nk : (long)ni * nj);
-  for (int kd = 0; kd < 3; kd++) c.wave_points[kd] = kd == 1 ? (long)ni * nj * nk : 0;
+  const long inside = span * (j1 - j0) * (k1 - k0);
+  c.wave_points[0] = inside;
+  c.wave_points[1] = (long)ni * nj * nk - inside;
+  c.wave_points[2] = 0;
   for (int kd = 0; kd < 4; kd++) c.aux_read_pairs[kd] = c.aux_update_pairs[kd] = kd == 1 ? pairs : 0;
   c.pml_nbox = c.pml_blocks = 0;
-  return put_work(c, all);
+  box.insert(box.end(), rest.begin(), rest.end());
+  return put_work(c, box);
 }
 
 // True when the two ADE-PML bands of every axis are disjoint (2 N <= the axis
@@ -161,21 +245,29 @@ static bool bands_disjoint(const Params& p) {
   return 2 * p.PML_N <= p.NX && 2 * p.PML_N <= p.NY && (p.FreeSurface || 2 * p.PML_N <= p.NZ);
 }
 
-// One launch of tiles of any kind (the FULL form of the pipelined kernel)
-// instead of one per kind: WaveUnified 1, or -1 (default) on grids of at most
-// kUnifiedPoints points without any of the per-kind launch options.  On small
-// grids each launch of one kind leaves most of the chip idle while its longest
-// block runs, and they run one after another: per step 1.26 -> 0.25 ms at
-// 30 x 80 x 50, 1.52 -> 0.41 at 97 x 125 x 81, 1.31 -> 0.65 at 100 x 200 x 100,
-// 3.00 -> 2.34 at 251 x 187 x 143.  At 400 x 300 x 200 both are level (6.2 ms
-// each, now that the tiles wait less), and the launches of one kind keep their
-// own tile shapes.
+// One launch of tiles of any kind instead of one per kind, and beside it, with
+// a box, the interior kernel on the interior tiles: WaveUnified 1 (without the
+// box) or 2 (with it), or -1 (default) without any of the per-kind launch
+// options: 1 up to kBoxPoints points, 2 up to kPerKindPoints, one launch per
+// kind above.  Each launch ends with CUs idle while its last blocks run, and
+// the launches of a stage run one after another, so small grids take one;
+// the box's kernel streams interior points at twice the rate, which pays
+// for a second launch, and the many blocks of a large grid make the tiles of
+// each kind's own shape the better choice.  ms per step with one launch, with
+// the box, and per kind:
+//   97 x 125 x 81    0.36   0.43   1.52
+//   200 x 160 x 120  1.32   1.31
+//   251 x 187 x 143  2.15   2.05   2.83
+//   400 x 300 x 200  6.20   5.91   6.00
+//   512 x 384 x 256  11.1   10.5   12.2
+//   640 x 512 x 400         25.1   27.3
+//   800 x 1000 x 500 71.8   57.1   55.8
 bool wave_unified(const Params& p) {
   if (p.WaveUnified == 0 || !bands_disjoint(p)) return false;
   if (p.WaveInteriorKernel != -1 || p.WaveBandKernel != -1 || p.WaveSurfaceKernel != 1 || p.WaveSurfaceTiles != 1 ||
       p.WaveTallInterior || p.WaveBandRound || !p.PmlAuxFused || p.StageStreams || p.WaveIChunk || p.WaveTopIChunk)
     return false;
-  return p.WaveUnified > 0 || (double)p.NX * p.NY * p.NZ <= kUnifiedPoints;
+  return p.WaveUnified > 0 || (double)p.NX * p.NY * p.NZ <= kPerKindPoints;
 }
 
 // Builds the stage-kernel work lists and allocates the free-surface buffers.  The interior box excludes every face band where a PML profile or
@@ -218,19 +310,9 @@ int upload_wave_work(Ctx& c) {
   // CU), 2 the pipelined kernel on 64 x 6 tiles (384 threads, two blocks per
   // CU), 3 on 64 x 4 tiles (256 threads, three blocks per CU), 4 on 64 x 8
   // tiles with an LDS double buffer instead of the ring
-  // WaveInteriorKernel -1 (default) picks 3 when the interior launch holds
-  // at least 16 rounds of resident 64 x 4 blocks (three per CU; fewer rounds
-  // leave the last ones ragged: 1600 x 1000 x 500, 88 k blocks: 90-95 ms of
-  // interior per step against 96-101 for 1; 400 x 300 x 200, 2 k blocks:
-  // 2.67 against 2.49 ms), else 1
   const int cus = cu_count();
-  int wik = p.WaveInteriorKernel;
-  if (wik < 0) {
-    const long ej = std::max(0, n3[1] - lo[1] - hi[1]), ek = std::max(0, n3[2] - lo[2] - hi[2]);
-    const long span = std::max(0, n3[0] - lo[0] - hi[0]);
-    const long blocks4 = (ej / TJ) * (ek / TK4) * ((span + 31) / 32);
-    wik = blocks4 >= 16L * 3 * cus ? 3 : 1;
-  }
+  const int wik = interior_kernel(p, std::max(0, n3[1] - lo[1] - hi[1]) / TJ, std::max(0, n3[2] - lo[2] - hi[2]),
+                                  std::max(0, n3[0] - lo[0] - hi[0]), cus);
   c.wave_pipe = !tall && wik >= 1;
   c.wave_ring = wik == 1;
   // WaveBandKernel 1: the pipelined kernel on the band tiles too, which adds
@@ -294,22 +376,8 @@ int upload_wave_work(Ctx& c) {
   // (1600 x 1000 x 500: 97.7 ms of interior per step against 106.2 for the
   // ~300-plane chunks of a 4096-block target and 104.5 for 16 planes;
   // 400 x 300 x 200: 2.44 against 2.70 ms for ~8 planes).
-  // With one block per CU and few rounds of blocks (the ring kernel) the
-  // launch takes its rounds times the planes of a block and about two more
-  // for its start, and the last round may be nearly empty: the length that
-  // takes the least (400 x 300 x 200, 84 tiles of 360 planes: 120 planes in
-  // one round, 2.16 ms of interior per step; 2.37 with 32, 2.92 with 90).
-  auto rounds_chunk = [&](int span, long ntiles) {
-    int len = std::max(span, 1);
-    long best = 0;
-    for (int n = std::min(len, 8); n <= std::max(span, 1); n++) {
-      const long t = (n + 2) * ((ntiles * ((span + n - 1) / n) + cus - 1) / cus);
-      if (best == 0 || t < best) { best = t; len = n; }
-    }
-    return len;
-  };
   const int ich_in = p.WaveIChunk > 0 ? p.WaveIChunk
-                     : c.wave_ring   ? rounds_chunk(ib - ia, tiles_in)
+                     : c.wave_ring   ? rounds_chunk(ib - ia, tiles_in, cus)
                      : c.wave_pipe   ? std::min(std::max(ib - ia, 1), 32)
                                      : chunk(ib - ia, tiles_in, tall ? 2048 : 4096, 4);
   // band tiles stream 20 planes (1600 x 1000 x 500: 23.4 ms per step against

@@ -1359,15 +1359,6 @@ void launch_wave_t(WaveArgs<MT> a, const Ctx& c, hipStream_t s) {
     (void)hipStreamWaitEvent(si, c.fence[0], 0);
     (void)hipStreamWaitEvent(ss, c.fence[0], 0);
   }
-  if (c.wave_unified) {
-    pr.begin(s, PK_STAGE_BAND);
-    if (a.freenode) launch_image<FX, FY, FZ, MT>(a, c, s);
-    a.work = w; a.nwork = n[1];
-    hipLaunchKernelGGL((wave_interior_kernel<FX, FY, FZ, MT, TJN, NTHRN, 2, true, false, true>), dim3(a.nwork),
-                       dim3(TJN, TKN, 1), 0, s, a);
-    pr.end(s);
-    return;
-  }
   if (n[0] > 0) {
     a.work = w; a.nwork = n[0];
     pr.begin(si, PK_STAGE_INTERIOR);
@@ -1389,6 +1380,15 @@ void launch_wave_t(WaveArgs<MT> a, const Ctx& c, hipStream_t s) {
     else
       hipLaunchKernelGGL((wave_stage_kernel<FX, FY, FZ, MT, 0>), dim3(a.nwork), dim3(TJ, TK, 1), 0, si, a);
     pr.end(si);
+  }
+  if (c.wave_unified) {
+    pr.begin(s, PK_STAGE_BAND);
+    if (a.freenode) launch_image<FX, FY, FZ, MT>(a, c, s);
+    a.work = w + 2 * o1; a.nwork = n[1];
+    hipLaunchKernelGGL((wave_interior_kernel<FX, FY, FZ, MT, TJN, NTHRN, 2, true, false, true>), dim3(a.nwork),
+                       dim3(TJN, TKN, 1), 0, s, a);
+    pr.end(s);
+    return;
   }
   if (n[3] > 0) {
     a.work = w + 2 * o3; a.nwork = n[3];

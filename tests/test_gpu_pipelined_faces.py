@@ -36,3 +36,30 @@ def test_same_as_general_kernels(opts, nz):
         x = a.get(n)
         assert np.abs(x).max() > 0, n
         np.testing.assert_array_equal(x, b.get(n), err_msg=n)
+
+
+@pytest.mark.parametrize("dims", [(20, 112, 24), (41, 113, 27), (37, 241, 45), (19, 96, 40)])
+@pytest.mark.parametrize("opts", [{}, {"useCerjan": 1}, {"FreeSurface": 0}, {"MetricBF16": 1}, {"usePML": 0}],
+                         ids=["pml", "sponge", "no_surface", "bf16", "plain"])
+def test_interior_box_beside_unified_tiles(opts, dims):
+    """The interior kernel on the whole 64 x 8 tiles of the interior, one
+    launch of 32 x 8 tiles around them: boxes of one tile, of several, and
+    none at all (the last size)."""
+    case = cases.volume_case(curved=True, NX=dims[0], NY=dims[1], NZ=dims[2], PML_N=8, **opts)
+    a = dyn.Solver(dict(case["params"], WaveUnified=2))
+    b = dyn.Solver(dict(case["params"], **GENERAL))
+    for s in (a, b):
+        cases.apply_to_solver(case, s)
+        s.setup()
+        d = s.dims()
+        s.put("W", cases.random_wavefield(d["nx"], d["ny"], d["nz"], seed=12))
+        s.run(0, 8)
+    a.profile(True)
+    a.run(8, 1)
+    b.run(8, 1)
+    edge = case["params"]["PML_N"] if opts.get("usePML", 1) else 0
+    lo = (edge + 31) // 32 * 32
+    assert (a.profile_report()["stage_interior"][1] > 0) == ((dims[1] - edge - lo) // 64 >= 1)
+    for n in ["W"] + (["PMLx1", "PMLx2", "PMLy1", "PMLy2", "PMLz1"] if case["params"]["usePML"] else []):
+        assert np.abs(a.get(n)).max() > 0, n
+        np.testing.assert_array_equal(a.get(n), b.get(n), err_msg=n)
