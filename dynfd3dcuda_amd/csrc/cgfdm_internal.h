@@ -210,7 +210,6 @@ struct Ctx {
   float *matVx2Vz = nullptr, *matVy2Vz = nullptr;  // [nx][ny][9]
   float *cj[3] = {nullptr, nullptr, nullptr};      // Cerjan 1-D profiles (nx, ny, nz incl. ghosts)
   void* wave_work = nullptr;    // stage-kernel work list (two int4 per block)
-  float* trac_top = nullptr;    // free surface: traction vectors of the six top rows [nx][6][9][ny]
   float* img_top = nullptr;     // free surface: words of the top rows (image_top_kernel) [18][ni][nj]
   int wave_nwork = 0;                  // all work items
   bool wave_unified = false;        // one launch of tiles of any kind (WaveUnified)

@@ -16,7 +16,6 @@ WaveArgs<MT> make_args(Ctx& c, const StageBufs& b, int irk, bool rhs_only, float
   a.met = (const MT*)c.met;
   a.slabH = c.slabH;
   a.rhs = rhs_out;
-  a.ttop = c.trac_top;
   a.itop = c.img_top;
   WaveCold& w = a.cold;
   for (int x = 0; x < 3; x++) { w.pA[x] = c.pml.A[x]; w.pB[x] = c.pml.B[x]; w.pD[x] = c.pml.D[x]; w.cj[x] = c.cj[x]; }
@@ -277,9 +276,7 @@ bool wave_unified(const Params& p) {
 // 256 CUs stay balanced), then the edge items; each list is chunk-major so that
 // one XCD's contiguous share covers neighbouring tiles.
 int upload_wave_work(Ctx& c) {
-  if (c.p.FreeSurface && !c.trac_top) {  // the image stencil reaches six rows down (NZ >= 7)
-    if (hipMalloc(&c.trac_top, sizeof(float) * 9 * 6 * (size_t)c.d.nx * c.d.ny) != hipSuccess) return 1;
-    c.allocations.push_back(c.trac_top);
+  if (c.p.FreeSurface && !c.img_top) {  // the image stencil reaches six rows down (NZ >= 7)
     if (hipMalloc(&c.img_top, sizeof(float) * 18 * (size_t)c.d.ni * c.d.nj) != hipSuccess) return 1;
     c.allocations.push_back(c.img_top);
   }

@@ -202,7 +202,6 @@ struct WaveArgs {
   const MT* __restrict__ met;
   float* __restrict__ slabH;
   float* __restrict__ rhs;
-  float* ttop;  // traction vectors of the six top rows (free surface)
   float* itop;  // image velocity RHS of the three top rows (free surface)
   WaveCold cold;  // absorbing layers and free-surface maps, indexed with constants only
   const int4* __restrict__ work;  // two int4 per block: (j0, k0, first plane, end plane), (j lanes, k rows, first active j lane, first active k row)
@@ -221,46 +220,38 @@ struct WaveArgs {
   int aux_fused;  // BAND tiles advance their points' ADE-PML auxiliary fields themselves
 };
 
-// Free surface, first pass: the conservative traction vectors
-// J (grad xi_ax . sigma) (wave.cu:398-440) of the six rows nk-6..nk-1 that
-// the image stencil reaches, for every padded plane and column, from the
-// stage input: ttop[x][r][3 ax + c][jj], r = row - (nk-6), jj the padded
-// column.  One thread per point.
+// The conservative traction vector J (grad xi_ax . sigma) (wave.cu:398-440) of
+// a point, from the stage input.
 template <class MT>
-__global__ void __launch_bounds__(256) traction_top_kernel(WaveArgs<MT> a, int nx) {
-  const int ny = a.ny;
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)nx * 6 * ny) return;
-  const int jj = (int)(idx % ny);
-  const int r = (int)((idx / ny) % 6);
-  const int x = (int)(idx / ((long)ny * 6));
+__device__ __forceinline__ void trac_vec(const WaveArgs<MT>& a, int ax, int x, uint32_t q, float (&o)[3]) {
   const uint32_t nyz = a.nyz;
-  const uint32_t q = (uint32_t)a.jpad + (uint32_t)jj + (uint32_t)(a.nk - 6 + r + 3) * (uint32_t)a.py;
   const float* W = a.Win;
   const MT* M = a.met;
   const float J = mat_(M, 9, x, q, nyz, a.mref);
   const float txx = wat(W, 3, x, q, nyz), tyy = wat(W, 4, x, q, nyz), tzz = wat(W, 5, x, q, nyz);
   const float txy = wat(W, 6, x, q, nyz), txz = wat(W, 7, x, q, nyz), tyz = wat(W, 8, x, q, nyz);
-  float* o = a.ttop + ((long)x * 6 + r) * 9 * ny + jj;
-#pragma unroll
-  for (int ax = 0; ax < 3; ax++) {
-    const float e0 = mat_(M, 3 * ax, x, q, nyz, a.mref), e1 = mat_(M, 3 * ax + 1, x, q, nyz, a.mref), e2 = mat_(M, 3 * ax + 2, x, q, nyz, a.mref);
-    o[(3 * ax + 0) * ny] = (e0 * txx + e1 * txy + e2 * txz) * J;
-    o[(3 * ax + 1) * ny] = (e0 * txy + e1 * tyy + e2 * tyz) * J;
-    o[(3 * ax + 2) * ny] = (e0 * txz + e1 * tyz + e2 * tzz) * J;
-  }
+  const float e0 = mat_(M, 3 * ax, x, q, nyz, a.mref), e1 = mat_(M, 3 * ax + 1, x, q, nyz, a.mref), e2 = mat_(M, 3 * ax + 2, x, q, nyz, a.mref);
+  o[0] = (e0 * txx + e1 * txy + e2 * txz) * J;
+  o[1] = (e0 * txy + e1 * tyy + e2 * tyz) * J;
+  o[2] = (e0 * txz + e1 * tyz + e2 * tzz) * J;
 }
 
-// Free surface, second pass: the traction-image velocity RHS of the three
-// top rows (wave.cu:398-487): DRP derivatives of the traction vectors along
-// each axis, the z stencil zero at the surface and odd-mirrored above it,
-// with the PML 1/beta of each axis; itop[c][row][i][j], row = k - (nk-3).
-// For the top row also what its points need of the velocity maps (traction-
-// free condition, wave.cu:207-232): the dip derivative of the velocity DzV =
-// matVx2Vz DxV + matVy2Vz DyV in planes 9-11, and its two products alone
-// (the source of the x and y faces' auxiliary fields, pmlx.cu:185-210) in
-// planes 12-14 and 15-17.  In the stage tiles, short of registers, the 18
-// map words of a point were a chain of 18 memory round trips per plane.
+// Free surface: the traction-image velocity RHS of the three top rows
+// (wave.cu:398-487): DRP derivatives of the traction vectors along each axis,
+// the z stencil zero at the surface and odd-mirrored above it, with the PML
+// 1/beta of each axis, in planes 3 c + row of itop ([i][18][nj]), row = k -
+// (nk-3).  For the top row also what its points need of the velocity maps
+// (traction-free condition, wave.cu:207-232): the dip derivative of the
+// velocity DzV = matVx2Vz DxV + matVy2Vz DyV in planes 9-11, and its two
+// products alone (the source of the x and y faces' auxiliary fields,
+// pmlx.cu:185-210) in planes 12-14 and 15-17.  In the stage tiles, short of
+// registers, the 18 map words of a point were a chain of 18 memory round
+// trips per plane.
+// A point's 15 traction vectors are computed where they are used, all loads at
+// once: bound by latency, and as a pass of its own, which wrote them for this
+// one to read, it cost a launch per stage and a second round trip (ms of tiles
+// and image per step at 30 x 80 x 50 0.135 -> 0.124, 100 x 200 x 100 0.449 ->
+// 0.436; surface tiles and image at 800 x 1000 x 500 2.07 -> 1.98).
 template <int FX, int FY, int FZ, class MT>
 __global__ void __launch_bounds__(256) image_top_kernel(WaveArgs<MT> a) {
   const int ni = a.ni, nj = a.nj, nk = a.nk, ny = a.ny;
@@ -272,6 +263,7 @@ __global__ void __launch_bounds__(256) image_top_kernel(WaveArgs<MT> a) {
   const int k = nk - 3 + row, ik = 2 - row, x = i + 3;
   const uint32_t col = (uint32_t)a.jpad + (uint32_t)(j + 3) + (uint32_t)(k + 3) * (uint32_t)a.py;
   const MT* M = a.met;
+  const uint32_t py = (uint32_t)a.py;
   const float rrhojac = 1.0f / (mat_(M, 12, x, col, a.nyz, a.mref) * mat_(M, 9, x, col, a.nyz, a.mref));
   float rb[3] = {1.0f, 1.0f, 1.0f};
   if (a.pml) {
@@ -280,16 +272,18 @@ __global__ void __launch_bounds__(256) image_top_kernel(WaveArgs<MT> a) {
     rb[2] = 1.0f / a.cold.pB[2][k];
   }
   const int fl[3] = {FX, FY, FZ};
-  const int r0 = k - (nk - 6);  // 3, 4, 5
   float hv[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
   for (int ax = 0; ax < 3; ax++) {
     float v[3][7];
+#pragma unroll
     for (int l = 0; l < 7; l++) {
       const int xq = ax == 0 ? x + l - 3 : x;
-      const int r = ax == 2 ? min(r0 + l - 3, 5) : r0;  // rows above the surface: replaced below
-      const int jq = j + 3 + (ax == 1 ? l - 3 : 0);
-      const float* t = a.ttop + ((long)xq * 6 + r) * 9 * ny + (long)(3 * ax) * ny + jq;
-      for (int c = 0; c < 3; c++) v[c][l] = t[(long)c * ny];
+      const int up = ax == 2 ? min(l - 3, 2 - row) : 0;  // rows above the surface: replaced below
+      float o[3];
+      trac_vec(a, ax, xq, col + (uint32_t)(ax == 1 ? l - 3 : 0) + (uint32_t)up * py, o);
+#pragma unroll
+      for (int c = 0; c < 3; c++) v[c][l] = o[c];
     }
     if (ax == 2) {
       for (int c = 0; c < 3; c++) {
@@ -1327,12 +1321,11 @@ __global__ void __launch_bounds__(256) pml_aux_kernel(PmlAuxArgs<MT> a) {
   }
 }
 
-// The two passes of the free-surface image.
+// The free-surface image.
 template <int FX, int FY, int FZ, class MT>
 void launch_image(const WaveArgs<MT>& a, const Ctx& c, hipStream_t s) {
-  const long n1 = (long)c.d.nx * 6 * c.d.ny, n2 = (long)c.d.ni * 3 * c.d.nj;
-  hipLaunchKernelGGL(traction_top_kernel<MT>, dim3((unsigned)((n1 + 255) / 256)), dim3(256), 0, s, a, c.d.nx);
-  hipLaunchKernelGGL((image_top_kernel<FX, FY, FZ, MT>), dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0, s, a);
+  const long n = (long)c.d.ni * 3 * c.d.nj;
+  hipLaunchKernelGGL((image_top_kernel<FX, FY, FZ, MT>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
 }
 
 template <int FX, int FY, int FZ, class MT>
