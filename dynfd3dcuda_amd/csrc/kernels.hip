@@ -914,7 +914,6 @@ __global__ void __launch_bounds__(256) fault_post_kernel(FArgs a) {
   for (int c = 0; c < 9; c++) W[c * pyz] = o[c] * damp;
 }
 
-// cal_rup_sensor_D_cu / cal_rup_sensor_magn_cu (rup_sensor.cu:7-86).
 // Thermal pressurization (thermpress_cu, thermpress.cu:22-233), once per
 // step before the stages: per fault node, the temperature and pore-pressure
 // rises on TP_n points x = i dh normal to the fault (mirror symmetric at
@@ -965,35 +964,42 @@ __global__ void __launch_bounds__(256) thermpress_kernel(FaultDev F, int nj, int
   }
 }
 
-__global__ void rup_sensor_d_kernel(FaultDev F, int nj, int nk, int g0, int g1, int g2, int g3) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;
-  int k = blockIdx.y * blockDim.y + threadIdx.y;
+// cal_rup_sensor_D_cu / cal_rup_sensor_magn_cu (rup_sensor.cu:7-86).  The
+// magnitude takes the D words of the four neighbours: those of this call where
+// the neighbour gets any (inside the rectangle and split), computed here again
+// from its own neighbours' Ts1, else the words that the field holds.  One
+// launch instead of two per step; all loads before the store.
+__global__ void __launch_bounds__(256) rup_sensor_kernel(FaultDev F, int nj, int nk, int g0, int g1, int g2, int g3) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  const int k = blockIdx.y * blockDim.y + threadIdx.y;
   if (j >= nj || k >= nk) return;
-  int gj1 = j + 1, gk1 = k + 1;
-  if (!(gj1 >= g0 + 3 && gj1 <= g1 - 3 && gk1 >= g2 + 3 && gk1 <= g3 - 3)) return;
-  long q = j + (long)nj * k;
-  if (F.united[q]) return;
+  auto inside = [&](int j, int k) {
+    return j + 1 >= g0 + 3 && j + 1 <= g1 - 3 && k + 1 >= g2 + 3 && k + 1 <= g3 - 3;
+  };
+  if (!inside(j, k)) return;
+  const long q = j + (long)nj * k;
   const float* p = F.Ts1;
-  F.rsD_y[q] = 0.25f * (-p[q + 1] + 2.0f * p[q] - p[q - 1]);
-  F.rsD_z[q] = 0.25f * (-p[q + nj] + 2.0f * p[q] - p[q - nj]);
-}
-__global__ void rup_sensor_m_kernel(FaultDev F, int nj, int nk, int g0, int g1, int g2, int g3) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;
-  int k = blockIdx.y * blockDim.y + threadIdx.y;
-  if (j >= nj || k >= nk) return;
-  int gj1 = j + 1, gk1 = k + 1;
-  if (!(gj1 >= g0 + 3 && gj1 <= g1 - 3 && gk1 >= g2 + 3 && gk1 <= g3 - 3)) return;
-  long q = j + (long)nj * k;
-  const float* Dy = F.rsD_y;
-  const float* Dz = F.rsD_z;
-  float D1 = Dy[q] - Dy[q + 1], D2 = Dy[q] - Dy[q - 1];
+  auto d_y = [&](long x) { return 0.25f * (-p[x + 1] + 2.0f * p[x] - p[x - 1]); };
+  auto d_z = [&](long x) { return 0.25f * (-p[x + nj] + 2.0f * p[x] - p[x - nj]); };
+  auto D_y = [&](int dj, int dk) {
+    const long x = q + dj + (long)nj * dk;
+    const bool on = inside(j + dj, k + dk) && j + dj >= 0 && j + dj < nj && k + dk >= 0 && k + dk < nk;
+    return on && !F.united[x] ? d_y(x) : F.rsD_y[x];
+  };
+  const bool uni = F.united[q] != 0;
+  const float Dy = uni ? F.rsD_y[q] : d_y(q), Dz = uni ? F.rsD_z[q] : d_z(q);
+  const float jp = D_y(1, 0), jm = D_y(-1, 0), kp = D_y(0, 1), km = D_y(0, -1);
+  float D1 = Dy - jp, D2 = Dy - jm;
   float mg = 0.5f * (D1 * D1 + D2 * D2);
-  D1 = Dz[q] - Dy[q + nj];  // rup_sensor.cu:75-76 pairs Dz with Dy
-  D2 = Dz[q] - Dy[q - nj];
+  D1 = Dz - kp;  // rup_sensor.cu:75-76 pairs Dz with Dy
+  D2 = Dz - km;
   mg += 0.5f * (D1 * D1 + D2 * D2);
-  float p0 = F.Ts1[q] * F.Ts1[q];
-  F.rup_sensor[q] = mg / (p0 + 1e-16f) + 1e-16f;
-  if (F.united[q]) F.rup_sensor[q] = 0;
+  const float p0 = p[q] * p[q];
+  if (!uni) {
+    F.rsD_y[q] = Dy;
+    F.rsD_z[q] = Dz;
+  }
+  F.rup_sensor[q] = uni ? 0.0f : mg / (p0 + 1e-16f) + 1e-16f;
 }
 
 // smooth_gauss_volume0 (smooth.cu:15-62): mirror the split nodes, the
@@ -1176,8 +1182,7 @@ void launch_rup_sensor(Ctx& c) {
   dim3 g((c.d.nj + 63) / 64, (c.d.nk + 3) / 4, 1);
   const int* G = c.p.Fault_grid;
   c.prof.begin(c.stream, PK_RUP_SENSOR);
-  hipLaunchKernelGGL(rup_sensor_d_kernel, g, dim3(64, 4, 1), 0, c.stream, c.f, c.d.nj, c.d.nk, G[0], G[1], G[2], G[3]);
-  hipLaunchKernelGGL(rup_sensor_m_kernel, g, dim3(64, 4, 1), 0, c.stream, c.f, c.d.nj, c.d.nk, G[0], G[1], G[2], G[3]);
+  hipLaunchKernelGGL(rup_sensor_kernel, g, dim3(64, 4, 1), 0, c.stream, c.f, c.d.nj, c.d.nk, G[0], G[1], G[2], G[3]);
   c.prof.end(c.stream);
 }
 
