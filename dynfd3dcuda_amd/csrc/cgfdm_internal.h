@@ -57,14 +57,14 @@ struct Params {
   int WaveBandKernel = -1;  // absorbing-band tiles: 0 general kernel; pipelined kernel: 1 64 x 8 tiles, 2 64 x 4 tiles;
                             // -1: 2 with 64 x 4 interior tiles, else 1
   int WaveSurfaceKernel = 1;  // free-surface tiles: 0 general kernel; 1 pipelined kernel
-  int PmlAuxFused = 1;     // 1: the pipelined band tiles advance the ADE-PML auxiliary fields of their
-                           // points on one face; 0: a kernel of its own advances every band point's
+  int PmlAuxFused = 1;     // 1: the pipelined band and surface tiles advance the ADE-PML auxiliary fields of
+                           // their points; 0: a kernel of its own advances every band point's
   int WaveBufferSkew = 16384;  // words (a multiple of 32) by which buffer q of S, A, B, T starts q times
                                // further into its allocation
   int WaveBandIChunk = 0;  // planes per block of the band tiles (0: automatic)
   int WaveTopIChunk = 0;  // planes per block of the free-surface tiles (0: automatic)
   int WaveSurfaceTiles = 1;  // free-surface tiles = the top TK rows, own line-aligned j tiles (0: earlier layout)
-  int WaveUnified = -1;  // 1: one launch of tiles of any kind per stage, 2: one beside the interior's; 0: one per kind; -1: 1 or 2
+  int WaveUnified = -1;  // 1: one launch of tiles of any kind per stage, 2: one beside the interior's; 0: one per kind; -1: by points
   int WaveBandRound = 0;  // 1: low j band rounded up to whole 64-wide tiles (0: band width exactly)
 
   // derived (set_params.cu:286-295)
@@ -101,6 +101,9 @@ struct Dims {
 // below it is handled by the edge instantiation).
 int interior_lo_j(const Params& p);
 bool wave_unified(const Params& p);
+// Grids up to kBoxPoints points: one launch of tiles of any kind per stage; up
+// to kPerKindPoints: the interior box beside it; above: a launch per kind (the
+// figures are at wave_unified).
 constexpr double kBoxPoints = 4e6, kPerKindPoints = 200e6;
 
 // Fault state on the device (2-D arrays [nk][nj] unless noted).
@@ -210,7 +213,7 @@ struct Ctx {
   float *matVx2Vz = nullptr, *matVy2Vz = nullptr;  // [nx][ny][9]
   float *cj[3] = {nullptr, nullptr, nullptr};      // Cerjan 1-D profiles (nx, ny, nz incl. ghosts)
   void* wave_work = nullptr;    // stage-kernel work list (two int4 per block)
-  float* img_top = nullptr;     // free surface: words of the top rows (image_top_kernel) [18][ni][nj]
+  float* img_top = nullptr;     // free surface: words of the top rows (image_top_kernel) [ni][18][nj]
   int wave_nwork = 0;                  // all work items
   bool wave_unified = false;        // one launch of tiles of any kind (WaveUnified)
   bool wave_tall = false;           // interior tiles 64 x 16 (WaveTallInterior)

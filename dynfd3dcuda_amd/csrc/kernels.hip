@@ -601,10 +601,7 @@ __device__ __forceinline__ float dxv_off(const FArgs& a, int nn, int c, long pc,
 // rates of sides 0 and 1, 14-15 their stress rates.  The parts of one
 // 64 x 4 tile of fault nodes are consecutive work items, kept on one XCD:
 // they read the same slab planes around the tile, which then come from that
-// XCD's L2 instead of being fetched once per part.  Each group of parts
-// (G 0: 0-5, 1: 6-11, 2: 12-15) is a kernel of its own, so that the
-// registers of the split-node stress part do not set the occupancy of the
-// others.
+// XCD's L2 instead of being fetched once per part.
 constexpr int kDerivParts = 16;
 __global__ void __launch_bounds__(256) fault_deriv_kernel(FArgs a, int tiles_j, int items) {
   const int item = xcd_remap((int)blockIdx.x, items);

@@ -269,12 +269,12 @@ bool wave_unified(const Params& p) {
   return p.WaveUnified > 0 || (double)p.NX * p.NY * p.NZ <= kPerKindPoints;
 }
 
-// Builds the stage-kernel work lists and allocates the free-surface buffers.  The interior box excludes every face band where a PML profile or
-// the Cerjan sponge is non-trivial and the three free-surface rows; its
-// tiles start at the box edge so that no interior tile straddles a band.
-// Interior items come first (chunks sized for about 4096 blocks in total, so
-// 256 CUs stay balanced), then the edge items; each list is chunk-major so that
-// one XCD's contiguous share covers neighbouring tiles.
+// Builds the stage-kernel work lists and allocates the free-surface buffer.
+// With one launch per kind the interior box excludes every face band where a
+// PML profile or the Cerjan sponge is non-trivial and the three free-surface
+// rows; its tiles start at the box edge so that no interior tile straddles a
+// band.  Interior items come first, then the edge items; each list is
+// chunk-major so that one XCD's contiguous share covers neighbouring tiles.
 int upload_wave_work(Ctx& c) {
   if (c.p.FreeSurface && !c.img_top) {  // the image stencil reaches six rows down (NZ >= 7)
     if (hipMalloc(&c.img_top, sizeof(float) * 18 * (size_t)c.d.ni * c.d.nj) != hipSuccess) return 1;

@@ -202,7 +202,7 @@ struct WaveArgs {
   const MT* __restrict__ met;
   float* __restrict__ slabH;
   float* __restrict__ rhs;
-  float* itop;  // image velocity RHS of the three top rows (free surface)
+  float* itop;  // what the surface rows need of the free-surface image, [ni][18][nj] (image_top_kernel)
   WaveCold cold;  // absorbing layers and free-surface maps, indexed with constants only
   const int4* __restrict__ work;  // two int4 per block: (j0, k0, first plane, end plane), (j lanes, k rows, first active j lane, first active k row)
   unsigned nyz;                   // words of one field of one plane (py*nz, padded rows)
@@ -1438,8 +1438,8 @@ void launch_wave_t(WaveArgs<MT> a, const Ctx& c, hipStream_t s) {
     for (int ax = 0; ax < 3; ax++) p.np[ax] = c.pml.parts(ax);
     p.mat[0] = c.matVx2Vz; p.mat[1] = c.matVy2Vz;
     for (int f = 0; f < 6; f++) { p.Y[f] = c.pml.Y[f]; p.S[f] = c.pml.S[f]; p.T[f] = c.pml.T[f]; }
-    // the boxes (upload_wave_cold): every face whole, or with the fused
-    // update the free-surface rows and the edges of the absorbing box
+    // the boxes (upload_wave_work): every face whole, or with the fused
+    // update the free-surface rows when their tiles run the general kernel
     p.boxes = c.pml_boxes;
     p.nbox = c.pml_nbox;
     const int blocks = c.pml_blocks;
