@@ -14,11 +14,11 @@
 
 Kernel classes: stage_interior / stage_band / stage_surface (the
 instantiations of the wave stage kernel and of the pipelined stage kernel,
-whose BAND instantiations are band tiles; stage_surface includes the two
-free-surface precompute passes), pml_aux, fault_pre, fault_rs, fault_deriv,
-fault_post, rup_sensor, thermpress, setup_metric (the setup's metric
-pass), setup_other (its other passes); everything else is listed under its
-own name.
+whose BAND instantiations are band tiles; tiles of any kind count as band
+tiles; stage_surface includes the free-surface image), pml_aux, fault_pre,
+fault_rs, fault_deriv, fault_post, rup_sensor, thermpress, setup_metric (the
+setup's metric pass), setup_other (its other passes); everything else is
+listed under its own name.
 """
 import argparse
 import collections
@@ -43,13 +43,13 @@ def kernel_class(name):
     m = re.search(r"wave_interior_kernel<([^>]*)>", name)
     if m:  # the pipelined kernel: FX, FY, FZ, metric type, tile width, threads, waves per SIMD[, BAND, RING, TOP]
         args = [x.strip() for x in m.group(1).split(",")]
-        if len(args) > 9 and args[9] == "true":
-            return "stage_surface"
+        if len(args) > 9 and args[9] == "true":  # 32-wide: the tiles of any kind, which the solver's profile calls stage_band
+            return "stage_band" if args[4] == "32" else "stage_surface"
         return "stage_band" if len(args) > 7 and args[7] == "true" else "stage_interior"
     if "wave_interior_kernel" in name:
         return "stage_interior"
-    if "traction_top_kernel" in name or "image_top_kernel" in name:
-        return "stage_surface"  # the free-surface precompute passes
+    if "image_top_kernel" in name:
+        return "stage_surface"  # the free-surface image
     for k in ("pml_aux_kernel", "fault_pre_kernel", "fault_rs_kernel", "fault_deriv_kernel", "fault_post_kernel"):
         if k in name:
             return k[: -len("_kernel")]
