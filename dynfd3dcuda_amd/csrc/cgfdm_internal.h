@@ -97,6 +97,12 @@ struct Dims {
   long pyz;
 };
 
+// Index of the point nearest to x on an axis of n points.  A tile's lanes may
+// lie past either end (the first tile of the free-surface rows starts up to
+// 31 columns below the grid), and what such a lane reads without a mask it
+// reads here.
+constexpr int nearest_point(int x, int n) { return x < 0 ? 0 : x < n ? x : n - 1; }
+
 // First column of the interior box of the stage kernel (the absorbing band
 // below it is handled by the edge instantiation).
 int interior_lo_j(const Params& p);
@@ -301,5 +307,11 @@ int mlp_train_host(float* blob, const float* feat, const float* target, long n, 
                    unsigned seed, float* loss_hist, std::string& err);
 void launch_fill(Ctx& c, float* p, long n, float v);
 int upload_wave_work(Ctx& c);  // nonzero on a HIP error
+
+// The stage kernels' work list (two int4 per block) for a device of cus
+// compute units, with the tables of it that c keeps, and in boxes those of the
+// auxiliary-update kernel.  No HIP call: c needs its parameters, dimensions
+// and absorbing faces only.
+std::vector<int4> wave_work_list(Ctx& c, int cus, std::vector<int>& boxes);
 
 }  // namespace cgfdm

@@ -141,13 +141,12 @@ static int rounds_chunk(int span, long ntiles, int cus) {
 // 64-wide one (ms of tiles per step, 64 x 4 -> 32 x 8: 100 x 200 x 100
 // 0.52 -> 0.45, 151 x 211 x 133 1.60 -> 1.42, 200 x 160 x 120 1.30 -> 1.13;
 // where 64 x 4 fits better, 97 x 125 x 81, level: 0.37).
-static int unified_work(Ctx& c) {
+static std::vector<int4> unified_work(Ctx& c, int cus) {
   const Params& p = c.p;
   const int ni = c.d.ni, nj = c.d.nj, nk = c.d.nk;
   c.wave_tall = c.wave_pipe = c.wave_ring = c.wave_band_pipe = c.wave_surf_pipe = false;
   c.pml_fused = true;
   c.wave_ktop = nk;
-  const int cus = cu_count();
   // the interior box [i0, i1) x [j0, j1) x [k0, k1) in whole 64 x 8 tiles on
   // the 32 x 8 tiles' lattice (a lattice from the low bands' edges has larger
   // boxes, but partial tiles at all four sides: 512 x 384 x 256 11.7 against
@@ -234,7 +233,7 @@ static int unified_work(Ctx& c) {
   for (int kd = 0; kd < 4; kd++) c.aux_read_pairs[kd] = c.aux_update_pairs[kd] = kd == 1 ? pairs : 0;
   c.pml_nbox = c.pml_blocks = 0;
   box.insert(box.end(), rest.begin(), rest.end());
-  return put_work(c, box);
+  return box;
 }
 
 // True when the two ADE-PML bands of every axis are disjoint (2 N <= the axis
@@ -269,22 +268,17 @@ bool wave_unified(const Params& p) {
   return p.WaveUnified > 0 || (double)p.NX * p.NY * p.NZ <= kPerKindPoints;
 }
 
-// Builds the stage-kernel work lists and allocates the free-surface buffer.
 // With one launch per kind the interior box excludes every face band where a
 // PML profile or the Cerjan sponge is non-trivial and the three free-surface
 // rows; its tiles start at the box edge so that no interior tile straddles a
 // band.  Interior items come first, then the edge items; each list is
 // chunk-major so that one XCD's contiguous share covers neighbouring tiles.
-int upload_wave_work(Ctx& c) {
-  if (c.p.FreeSurface && !c.img_top) {  // the image stencil reaches six rows down (NZ >= 7)
-    if (hipMalloc(&c.img_top, sizeof(float) * 18 * (size_t)c.d.ni * c.d.nj) != hipSuccess) return 1;
-    c.allocations.push_back(c.img_top);
-  }
-
+std::vector<int4> wave_work_list(Ctx& c, int cus, std::vector<int>& boxes) {
+  boxes.clear();
   const Params& p = c.p;
   const int n3[3] = {c.d.ni, c.d.nj, c.d.nk};
   c.wave_unified = wave_unified(p);
-  if (c.wave_unified) return unified_work(c);
+  if (c.wave_unified) return unified_work(c, cus);
   const bool freenode = p.FreeSurface != 0;
   int lo[3], hi[3];
   for (int ax = 0; ax < 3; ax++) {
@@ -307,7 +301,6 @@ int upload_wave_work(Ctx& c) {
   // CU), 2 the pipelined kernel on 64 x 6 tiles (384 threads, two blocks per
   // CU), 3 on 64 x 4 tiles (256 threads, three blocks per CU), 4 on 64 x 8
   // tiles with an LDS double buffer instead of the ring
-  const int cus = cu_count();
   const int wik = interior_kernel(p, std::max(0, n3[1] - lo[1] - hi[1]) / TJ, std::max(0, n3[2] - lo[2] - hi[2]),
                                   std::max(0, n3[0] - lo[0] - hi[0]), cus);
   c.wave_pipe = !tall && wik >= 1;
@@ -457,7 +450,7 @@ int upload_wave_work(Ctx& c) {
   // ktop up when their tiles run the general kernel
   {
     const int N = c.pml.N;
-    std::vector<int> bx;
+    std::vector<int>& bx = boxes;
     int blocks = 0;
     c.aux_update_pairs[3] = 0;
     // box in face-local (j, k, i) coordinates
@@ -477,16 +470,28 @@ int upload_wave_work(Ctx& c) {
     }
     c.pml_nbox = (int)bx.size() / kPmlBoxInts;
     c.pml_blocks = blocks;
-    if (c.pml_boxes) { (void)hipFree(c.pml_boxes); c.pml_boxes = nullptr; }
-    if (!bx.empty()) {
-      if (hipMalloc(&c.pml_boxes, bx.size() * sizeof(int)) != hipSuccess) return 1;
-      if (hipMemcpy(c.pml_boxes, bx.data(), bx.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) return 1;
-    }
   }
   std::vector<int4> all;
   for (int l = 0; l < 4; l++) {
     all.insert(all.end(), lists[l].begin(), lists[l].end());
     c.wave_nkind[l] = (int)lists[l].size() / 2;
+  }
+  return all;
+}
+
+// Builds and uploads the stage-kernel work lists and allocates the
+// free-surface buffer.
+int upload_wave_work(Ctx& c) {
+  if (c.p.FreeSurface && !c.img_top) {  // the image stencil reaches six rows down (NZ >= 7)
+    if (hipMalloc(&c.img_top, sizeof(float) * 18 * (size_t)c.d.ni * c.d.nj) != hipSuccess) return 1;
+    c.allocations.push_back(c.img_top);
+  }
+  std::vector<int> boxes;
+  const std::vector<int4> all = wave_work_list(c, cu_count(), boxes);
+  if (c.pml_boxes) { (void)hipFree(c.pml_boxes); c.pml_boxes = nullptr; }
+  if (!boxes.empty()) {
+    if (hipMalloc(&c.pml_boxes, boxes.size() * sizeof(int)) != hipSuccess) return 1;
+    if (hipMemcpy(c.pml_boxes, boxes.data(), boxes.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) return 1;
   }
   return put_work(c, all);
 }

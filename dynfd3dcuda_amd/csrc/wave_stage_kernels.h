@@ -988,7 +988,7 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
 #pragma unroll
         for (int c = 0; c < 9; c++) ah[c] = ad1 * y[c] + d1 * axis_rhs_c(c, dd, e0, e1, e2, rrho, lam, l2m, mu);
         if (TOP && ax < 2 && last) {  // the traction-free term (pmlx.cu:185-210)
-          const float c0 = d1 * (ax == 0 ? uni(cold->pB[0], i) : cold->pB[1][min(j, nj - 1)]);
+          const float c0 = d1 * (ax == 0 ? uni(cold->pB[0], i) : cold->pB[1][nearest_point(j, nj)]);
           float z1[3];
 #pragma unroll
           for (int r = 0; r < 3; r++) z1[r] = top_word(12 + 3 * ax + r, row == 2);
