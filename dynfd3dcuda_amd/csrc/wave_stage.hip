@@ -89,6 +89,33 @@ int interior_lo_j(const Params& p) {
   return (band + TJ - 1) / TJ * TJ;
 }
 
+// Clears the counts of points and (point, face) pairs of the work lists.
+static void clear_counts(Ctx& c) {
+  for (int kd = 0; kd < 3; kd++) c.wave_points[kd] = 0;
+  for (int kd = 0; kd < 4; kd++) c.aux_read_pairs[kd] = c.aux_update_pairs[kd] = 0;
+}
+
+// Adds the points of a block, planes [i0, i1) of columns [j0, j1) and rows
+// [k0, k1), to the counts of kind kd; update: it advances their auxiliary
+// fields.  Every list counts what it pushes, so that a tile missed or listed
+// twice shows in the sums.
+static void count_block(Ctx& c, int kd, int i0, int i1, int j0, int j1, int k0, int k1, bool update) {
+  // points of [lo, hi) along axis ax inside that axis's absorbing bands
+  auto in_bands = [&](int ax, int lo, int hi) {
+    const int N = c.pml.N, nn = ax == 0 ? c.d.ni : ax == 1 ? c.d.nj : c.d.nk;
+    const int a0 = 0, a1 = c.pml.on[2 * ax] ? std::min(N, nn) : 0;
+    const int b0 = c.pml.on[2 * ax + 1] ? std::max(nn - N, 0) : nn, b1 = nn;
+    auto len = [&](int x0, int x1) { return std::max(0, std::min(x1, hi) - std::max(x0, lo)); };
+    return len(a0, a1) + len(b0, b1) - len(std::max(a0, b0), std::min(a1, b1));
+  };
+  const long Li = i1 - i0, Lj = j1 - j0, Lk = k1 - k0;
+  const long bi = in_bands(0, i0, i1), bj = in_bands(1, j0, j1), bk = in_bands(2, k0, k1);
+  const long pairs = bi * Lj * Lk + Li * bj * Lk + Li * Lj * bk;
+  c.wave_points[kd] += Li * Lj * Lk;
+  c.aux_read_pairs[kd] += pairs;
+  if (update) c.aux_update_pairs[kd] += pairs;
+}
+
 // Uploads a work list (two int4 per block).
 static int put_work(Ctx& c, const std::vector<int4>& all) {
   if (c.wave_work) { (void)hipFree(c.wave_work); c.wave_work = nullptr; }
@@ -179,6 +206,7 @@ static std::vector<int4> unified_work(Ctx& c, int cus) {
         for (int j = j0; j < j1; j += TJ) {
           box.push_back(make_int4(j, k, i, std::min(i1, i + len)));
           box.push_back(make_int4(TJ, c.wave_tki, 0, 0));
+          count_block(c, 0, i, std::min(i1, i + len), j, j + TJ, k, k + c.wave_tki, false);
         }
   }
   // the other tiles: all of them on the planes outside the box, those around
@@ -208,8 +236,10 @@ static std::vector<int4> unified_work(Ctx& c, int cus) {
       for (int k = 0; k < nk; k += TKN)
         for (int j = 0; j < nj; j += TJN) {
           if (!whole && j >= j0 && j < j1 && k >= k0 && k < k1) continue;
-          rest.push_back(make_int4(j, k, i, std::min(b, i + len)));
-          rest.push_back(make_int4(std::min((int)TJN, nj - j), std::min((int)TKN, nk - k), 0, 0));
+          const int ie = std::min(b, i + len), w = std::min((int)TJN, nj - j), h = std::min((int)TKN, nk - k);
+          rest.push_back(make_int4(j, k, i, ie));
+          rest.push_back(make_int4(w, h, 0, 0));
+          count_block(c, 1, i, ie, j, j + w, k, k + h, true);
         }
   };
   if (span > 0) {
@@ -222,15 +252,6 @@ static std::vector<int4> unified_work(Ctx& c, int cus) {
   for (int l = 0; l < 4; l++) c.wave_nkind[l] = 0;
   c.wave_nkind[0] = (int)box.size() / 2;
   c.wave_nkind[1] = (int)rest.size() / 2;
-  const long N = c.pml.N;
-  long pairs = 0;
-  for (int f = 0; f < 6; f++)
-    if (c.pml.on[f]) pairs += N * (f < 2 ? (long)nj * nk : f < 4 ? (long)ni * nk : (long)ni * nj);
-  const long inside = span * (j1 - j0) * (k1 - k0);
-  c.wave_points[0] = inside;
-  c.wave_points[1] = (long)ni * nj * nk - inside;
-  c.wave_points[2] = 0;
-  for (int kd = 0; kd < 4; kd++) c.aux_read_pairs[kd] = c.aux_update_pairs[kd] = kd == 1 ? pairs : 0;
   c.pml_nbox = c.pml_blocks = 0;
   box.insert(box.end(), rest.begin(), rest.end());
   return box;
@@ -275,6 +296,7 @@ bool wave_unified(const Params& p) {
 // chunk-major so that one XCD's contiguous share covers neighbouring tiles.
 std::vector<int4> wave_work_list(Ctx& c, int cus, std::vector<int>& boxes) {
   boxes.clear();
+  clear_counts(c);
   const Params& p = c.p;
   const int n3[3] = {c.d.ni, c.d.nj, c.d.nk};
   c.wave_unified = wave_unified(p);
@@ -379,26 +401,12 @@ std::vector<int4> wave_work_list(Ctx& c, int cus, std::vector<int>& boxes) {
   // of at most 32 columns along j (32 x 16 tiles, half the idle lanes),
   // 3 tiles holding free-surface rows
   std::vector<int4> lists[4];
-  for (int kd = 0; kd < 3; kd++) c.wave_points[kd] = 0;
-  for (int kd = 0; kd < 3; kd++) c.aux_read_pairs[kd] = c.aux_update_pairs[kd] = 0;
-  // points of [lo, hi) along axis ax inside that axis's absorbing bands
-  auto in_bands = [&](int ax, int lo, int hi) {
-    const int N = c.pml.N, nn = n3[ax];
-    const int a0 = 0, a1 = c.pml.on[2 * ax] ? std::min(N, nn) : 0;
-    const int b0 = c.pml.on[2 * ax + 1] ? std::max(nn - N, 0) : nn, b1 = nn;
-    auto len = [&](int x0, int x1) { return std::max(0, std::min(x1, hi) - std::max(x0, lo)); };
-    return len(a0, a1) + len(b0, b1) - len(std::max(a0, b0), std::min(a1, b1));
-  };
   auto push = [&](int list, const Seg& a, const Seg& b, int i0, int i1) {
     lists[list].push_back(make_int4(a.s, b.s, i0, i1));
     lists[list].push_back(make_int4(a.n, b.n, a.o, b.o));
     const int kd = list == 0 ? 0 : list == 3 ? 2 : 1;
-    const long Li = i1 - i0, Lj = a.n - a.o, Lk = b.n - b.o;
-    c.wave_points[kd] += Li * Lj * Lk;
-    const long bi = in_bands(0, i0, i1), bj = in_bands(1, a.s + a.o, a.s + a.n), bk = in_bands(2, b.s + b.o, b.s + b.n);
-    c.aux_read_pairs[kd] += bi * Lj * Lk + Li * bj * Lk + Li * Lj * bk;
     // the fused update in the band tiles and the pipelined free-surface tiles
-    if (c.pml_fused && (kd == 1 || (kd == 2 && c.wave_surf_pipe))) c.aux_update_pairs[kd] += bi * Lj * Lk + Li * bj * Lk + Li * Lj * bk;
+    count_block(c, kd, i0, i1, a.s + a.o, a.s + a.n, b.s + b.o, b.s + b.n, c.pml_fused && (kd == 1 || (kd == 2 && c.wave_surf_pipe)));
   };
   const auto narrow = [&](const Seg& a) { return !a.in && a.n - a.o <= TJN; };
   // bands of at most TJB columns get tiles exactly TJB wide (with the
@@ -452,7 +460,6 @@ std::vector<int4> wave_work_list(Ctx& c, int cus, std::vector<int>& boxes) {
     const int N = c.pml.N;
     std::vector<int>& bx = boxes;
     int blocks = 0;
-    c.aux_update_pairs[3] = 0;
     // box in face-local (j, k, i) coordinates
     auto add = [&](int f, int j0, int nj_, int k0, int nk_, int i0, int ni_) {
       if (nj_ <= 0 || nk_ <= 0 || ni_ <= 0) return;

@@ -67,3 +67,56 @@ def test_lanes_beside_the_grid_read_profiles_inside_them(tool, layer, opts):
             low = min(low, it[1])
     edge = max(layer, p.get("DAMP_N", 0) if p.get("useCerjan") else 0)
     assert low == (0 if r["unified"] else edge - 32 * ((edge + 31) // 32))
+
+
+LAYOUTS = [{"WaveUnified": 0}, {"WaveUnified": 0, "WaveInteriorKernel": 3}, {"WaveUnified": 0, "WaveSurfaceKernel": 0},
+           {"WaveUnified": 0, "WaveSurfaceTiles": 0}, {"WaveUnified": 0, "PmlAuxFused": 0}, {"WaveUnified": 0, "WaveBandRound": 1},
+           {"WaveUnified": 1}, {"WaveUnified": 1, "WaveBandIChunk": 3}, {"WaveUnified": 2}]
+
+
+@pytest.mark.parametrize("dims", [(44, 150, 52), (41, 181, 61), (45, 240, 47)], ids=["44x150x52", "41x181x61", "45x240x47"])
+@pytest.mark.parametrize("free", [1, 0], ids=["surface", "no_surface"])
+@pytest.mark.parametrize("layout", LAYOUTS, ids=lambda v: "-".join(f"{k}{x}" for k, x in v.items()))
+def test_every_point_and_face_once(tool, layout, free, dims):
+    """Every point is in one block's tile, every (point, absorbing face) pair
+    is read by one block and advanced by one block or box, no interior block
+    holds an absorbing point or a surface row, and the counts that the solver
+    reports are those of the blocks in the list."""
+    N = 12
+    r = work(tool, **dict(dict(zip(("NX", "NY", "NZ"), dims), PML_N=N, FreeSurface=free), **layout))
+    ni, nj, nk = dims
+    faces = np.zeros(dims, int)  # absorbing faces of each point
+    for ax, n in enumerate(dims):
+        edge = np.zeros(n, int)
+        edge[:N] += 1
+        if ax < 2 or not free:
+            edge[n - N:] += 1
+        faces += edge.reshape([-1 if a == ax else 1 for a in range(3)])
+    seen, updated = np.zeros(dims, int), np.zeros(dims, int)
+    points, read, update = [0, 0, 0], [0, 0, 0, 0], [0, 0, 0, 0]
+    for kind, j, k, i0, i1, jn, kn, jo, ko in r["item"]:
+        w, h = lanes(r, (kind,))
+        assert 0 <= jo < jn <= w and 0 <= ko < kn <= h and i0 < i1
+        at = (slice(i0, i1), slice(j + jo, j + jn), slice(k + ko, k + kn))
+        assert i0 >= 0 and i1 <= ni and at[1].start >= 0 and at[1].stop <= nj and at[2].start >= 0 and at[2].stop <= nk
+        seen[at] += 1
+        group = 0 if kind == 0 else 2 if kind == 3 else 1
+        pairs = int(faces[at].sum())
+        points[group] += seen[at].size
+        read[group] += pairs
+        if group == 0:
+            assert pairs == 0 and not (free and at[2].stop > nk - 3)
+        elif r["fused"] and (group == 1 or r["surf_pipe"]):
+            update[group] += pairs
+            updated[at] += faces[at]
+    for f, j, nj_, k, nk_, i, ni_, _ in r["box"]:
+        off = [0, 0, 0]  # the face's first point
+        if f & 1:
+            off[f // 2] = dims[f // 2] - N
+        at = tuple(slice(o + x, o + x + n) for o, x, n in zip(off, (i, j, k), (ni_, nj_, nk_)))
+        updated[at] += 1
+        update[3] += ni_ * nj_ * nk_
+    assert (seen == 1).all() and np.array_equal(updated, faces)
+    assert r["points"] == points and r["read"] == read and r["update"] == update
+    if layout["WaveUnified"] == 2:
+        assert points[0] > 0
