@@ -268,7 +268,8 @@ static bool bands_disjoint(const Params& p) {
 // a box, the interior kernel on the interior tiles: WaveUnified 1 (without the
 // box) or 2 (with it), or -1 (default) without any of the per-kind launch
 // options: 1 up to kBoxPoints points, 2 up to kPerKindPoints, one launch per
-// kind above.  Each launch ends with CUs idle while its last blocks run, and
+// kind above.  WaveInteriorKernel 1 or 3 with WaveUnified 2 names the box's
+// kernel.  Each launch ends with CUs idle while its last blocks run, and
 // the launches of a stage run one after another, so small grids take one;
 // the box's kernel streams interior points at twice the rate, which pays
 // for a second launch, and the many blocks of a large grid make the tiles of
@@ -283,7 +284,8 @@ static bool bands_disjoint(const Params& p) {
 //   800 x 1000 x 500 71.8   57.1   55.8
 bool wave_unified(const Params& p) {
   if (p.WaveUnified == 0 || !bands_disjoint(p)) return false;
-  if (p.WaveInteriorKernel != -1 || p.WaveBandKernel != -1 || p.WaveSurfaceKernel != 1 || p.WaveSurfaceTiles != 1 ||
+  const bool box_kernel = p.WaveUnified == 2 && (p.WaveInteriorKernel == 1 || p.WaveInteriorKernel == 3);
+  if ((p.WaveInteriorKernel != -1 && !box_kernel) || p.WaveBandKernel != -1 || p.WaveSurfaceKernel != 1 || p.WaveSurfaceTiles != 1 ||
       p.WaveTallInterior || p.WaveBandRound || !p.PmlAuxFused || p.StageStreams || p.WaveIChunk || p.WaveTopIChunk)
     return false;
   return p.WaveUnified > 0 || (double)p.NX * p.NY * p.NZ <= kPerKindPoints;

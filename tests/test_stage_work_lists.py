@@ -120,3 +120,15 @@ def test_every_point_and_face_once(tool, layout, free, dims):
     assert r["points"] == points and r["read"] == read and r["update"] == update
     if layout["WaveUnified"] == 2:
         assert points[0] > 0
+
+
+@pytest.mark.parametrize("opts,rows", [(dict(NX=600, NY=640, NZ=500), 4), (dict(NX=400, NY=300, NZ=200), 8),
+                                       (dict(NX=44, NY=150, NZ=52, WaveUnified=2, WaveInteriorKernel=3), 4),
+                                       (dict(NX=600, NY=640, NZ=500, WaveUnified=2, WaveInteriorKernel=1), 8)],
+                         ids=["automatic_large", "automatic", "64x4", "64x8_ring"])
+def test_kernel_of_the_interior_box(tool, opts, rows):
+    """The box beside the tiles of any kind runs in 64 x 4 tiles when it holds
+    many of them or when asked to, else in the ring kernel's 64 x 8 tiles."""
+    r = work(tool, **opts)
+    assert r["unified"] and r["points"][0] > 0
+    assert {it[6] for it in r["item"] if it[0] == 0} == {rows} and r["ring"] == (rows == 8)
