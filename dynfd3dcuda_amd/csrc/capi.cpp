@@ -338,6 +338,9 @@ int cgfdm_setup(cgfdm_ctx* h) {
     int code = rc == 5 ? CGFDM_ECFL : rc == 4 ? CGFDM_ENETCDF : rc == 2 ? CGFDM_EFILE : rc == 6 ? CGFDM_EHIP : CGFDM_EPARAM;
     return fail(code, err);
   }
+  // what the work lists took of WaveUnified, for cgfdm_get_param: a request
+  // that the other options or the grid do not allow is not kept silently
+  c.p.WaveUnified = !c.wave_unified ? 0 : c.wave_nkind[0] > 0 ? 2 : 1;
   if (hipStreamCreateWithFlags(&c.own_stream, hipStreamNonBlocking) != hipSuccess)
     return fail(CGFDM_EHIP, "stream creation failed");
   c.stream = c.own_stream;

@@ -58,3 +58,19 @@ def test_box_same_rupture(kind, metric, kernel):
     for n in ("W", "FW", "Vs1", "Vs2", "Ts1", "Ts2", "Tn", "slip", "State", "slabH", "rup_sensor", "PMLx1", "PMLx2", "PMLy1",
               "PMLy2", "PMLz1"):
         np.testing.assert_array_equal(a.get(n), b.get(n), err_msg=n)
+
+
+@pytest.mark.parametrize("opts,used", [
+    ({}, 1), ({"WaveUnified": 2}, 1), ({"WaveUnified": 2, "NY": 112}, 2), ({"WaveUnified": 2, "NY": 112, "WaveInteriorKernel": 3}, 2),
+    ({"WaveUnified": 0}, 0), ({"WaveUnified": 1, "WaveInteriorKernel": 3}, 0), ({"WaveUnified": 1, "StageStreams": 1}, 0),
+    ({"WaveUnified": 2, "WaveTopIChunk": 4}, 0), ({"WaveUnified": 1, "PML_N": 11}, 0), ({"WaveUnified": 1, "WaveBandIChunk": 5}, 1)],
+    ids=["default", "no_box", "box", "box_64x4", "off", "other_kernel", "streams", "surface_chunk", "bands_overlap", "chunk"])
+def test_setup_reports_the_layout_in_use(opts, used):
+    """A WaveUnified that cannot be honoured reads back as what runs."""
+    case = cases.volume_case(curved=False, **dict(dict(NX=20, NY=40, NZ=24, PML_N=8), **opts))
+    s = dyn.Solver(case["params"])
+    assert s.get_param("WaveUnified") == opts.get("WaveUnified", -1)
+    s.setup()
+    assert s.get_param("WaveUnified") == used
+    s.run(0, 1)
+    s.close()
