@@ -523,23 +523,38 @@ int cgfdm_fault_smooth(cgfdm_ctx* h) {
   return check_hip("fault smoothing launch");
 }
 
+// Between the caller's [field][plane][words] and the device's
+// [plane][field][words], planes swap_stride words apart: a field's planes at a
+// time gathered on the device into a buffer (or scattered from it) that one
+// copy brings over.  What is left is the copy of pageable memory: a y face of
+// 400 x 300 x 200 (54 MB) takes 2.1 ms to put and 5.8 to get; swapped on the
+// host, with the words between the face's planes brought over as well, 35 and
+// 33 ms.
+static hipError_t swap_copy(Ctx& c, const FieldRef& r, char* host, bool to_dev) {
+  const long np = r.swap_n, row = (long)(r.count / 9) / np;
+  const long step = std::min(np, std::max(1L, (1L << 22) / row));  // planes of a piece: 16 MB at most, or one plane
+  float* buf = nullptr;
+  if (hipError_t e = hipMalloc(&buf, step * row * sizeof(float))) return e;
+  hipError_t e = hipSuccess;
+  for (int f = 0; f < 9 && !e; f++)
+    for (long i = 0; i < np && !e; i += step) {
+      const long n = std::min(step, np - i);
+      const size_t bytes = n * row * sizeof(float);
+      char* h = host + (f * np + i) * row * sizeof(float);
+      float* d = (float*)r.ptr + i * (long)r.swap_stride + f * row;
+      if (to_dev) e = hipMemcpyAsync(buf, h, bytes, hipMemcpyHostToDevice, c.stream);
+      if (!e) e = launch_plane_copy(c, buf, d, n, row, (long)r.swap_stride, to_dev);
+      if (!e && !to_dev) e = hipMemcpyAsync(h, buf, bytes, hipMemcpyDeviceToHost, c.stream);
+    }
+  const hipError_t done = hipStreamSynchronize(c.stream);
+  (void)hipFree(buf);
+  return e ? e : done;
+}
+
 // Between the caller's layout (the reference's: [field][plane][k][j], rows
 // of ny) and the device's plane-interleaved [plane][field][k][jpad + j] with
 // rows of py; to_dev selects the direction.  The slab buffer is the one
 // exception on the caller's side: it is [plane][field][k][j] there too.
-// Between the caller's [field][plane][words] and the device's
-// [plane][field][words], planes swap_stride words apart.
-static size_t swap_bytes(const FieldRef& r) {  // device extent of such a field
-  return ((r.swap_n - 1) * r.swap_stride + r.count / r.swap_n) * dsize(r.dtype);
-}
-static void swap_copy(const FieldRef& r, const char* from, char* to, bool to_dev) {
-  const size_t np = (size_t)r.swap_n, row = r.count / 9 / np * dsize(r.dtype);
-  for (size_t f = 0; f < 9; f++)
-    for (size_t i = 0; i < np; i++) {
-      const size_t dev = i * r.swap_stride * dsize(r.dtype) + f * row, ref = (f * np + i) * row;
-      std::memcpy(to + (to_dev ? dev : ref), from + (to_dev ? ref : dev), row);
-    }
-}
 static size_t dev_words(const Ctx& c, const FieldRef& r) { return (size_t)r.planes * r.nf * c.d.pyz; }
 static void interleave_copy(const Ctx& c, const FieldRef& r, const char* from, char* to, bool to_dev) {
   const size_t es = dsize(r.dtype), nz = (size_t)c.d.nz, ny = (size_t)c.d.ny, py = (size_t)c.d.py;
@@ -577,10 +592,8 @@ int cgfdm_get_field(cgfdm_ctx* h, const char* name, void* dst, size_t bytes) {
   }
   if (hipError_t e = hipStreamSynchronize(c.stream)) return fail(CGFDM_EHIP, hipGetErrorString(e));
   if (!r.nf) {
-    std::vector<char> tmp(r.swap_n ? swap_bytes(r) : 0);
-    if (hipMemcpy(r.swap_n ? tmp.data() : dst, r.ptr, r.swap_n ? tmp.size() : bytes, hipMemcpyDeviceToHost) != hipSuccess)
+    if ((r.swap_n ? swap_copy(c, r, (char*)dst, false) : hipMemcpy(dst, r.ptr, bytes, hipMemcpyDeviceToHost)) != hipSuccess)
       return fail(CGFDM_EHIP, "copy failed");
-    if (r.swap_n) swap_copy(r, tmp.data(), (char*)dst, false);
     return 0;
   }
   std::vector<char> tmp(dev_words(c, r) * dsize(r.dtype));
@@ -603,12 +616,7 @@ int cgfdm_put_field(cgfdm_ctx* h, const char* name, const void* src, size_t byte
   if (r.host) return fail(CGFDM_EPARAM, std::string("read-only field ") + name);
   if (hipError_t e = hipStreamSynchronize(c.stream)) return fail(CGFDM_EHIP, hipGetErrorString(e));
   if (!r.nf) {
-    std::vector<char> tmp(r.swap_n ? swap_bytes(r) : 0);
-    if (r.swap_n) {  // the other face's words between this one's stay as they are
-      if (hipMemcpy(tmp.data(), r.ptr, tmp.size(), hipMemcpyDeviceToHost) != hipSuccess) return fail(CGFDM_EHIP, "copy failed");
-      swap_copy(r, (const char*)src, tmp.data(), true);
-    }
-    if (hipMemcpy(r.ptr, r.swap_n ? tmp.data() : src, r.swap_n ? tmp.size() : bytes, hipMemcpyHostToDevice) != hipSuccess)
+    if ((r.swap_n ? swap_copy(c, r, (char*)src, true) : hipMemcpy(r.ptr, src, bytes, hipMemcpyHostToDevice)) != hipSuccess)
       return fail(CGFDM_EHIP, "copy failed");
     return 0;
   }

@@ -1093,6 +1093,14 @@ __global__ void fill_kernel(float* p, long n, float v) {
   for (; i < n; i += st) p[i] = v;
 }
 
+// Rows of `row` words, packed in buf and stride words apart in d; per blocks a row.
+__global__ void __launch_bounds__(256) plane_copy_kernel(float* buf, float* d, long row, long stride, unsigned per, bool to_d) {
+  const long i = blockIdx.x / per, x = (long)(blockIdx.x % per) * 256 + threadIdx.x;
+  if (x >= row) return;
+  if (to_d) d[i * stride + x] = buf[i * row + x];
+  else buf[i * row + x] = d[i * stride + x];
+}
+
 FArgs make_fargs(Ctx& c) {
   FArgs a{};
   a.F = c.f;
@@ -1195,6 +1203,12 @@ void launch_fill(Ctx& c, float* p, long n, float v) {
   long blocks = std::min<long>((n + 255) / 256, 65536);
   if (blocks < 1) blocks = 1;
   hipLaunchKernelGGL(fill_kernel, dim3((unsigned)blocks), dim3(256), 0, c.stream, p, n, v);
+}
+
+hipError_t launch_plane_copy(Ctx& c, float* buf, float* d, long n, long row, long stride, bool to_d) {
+  const unsigned per = (unsigned)((row + 255) / 256);
+  hipLaunchKernelGGL(plane_copy_kernel, dim3((unsigned)n * per), dim3(256), 0, c.stream, buf, d, row, stride, per, to_d);
+  return hipGetLastError();
 }
 
 }  // namespace cgfdm

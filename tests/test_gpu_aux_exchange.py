@@ -1,0 +1,36 @@
+"""put, get and check of the ADE-PML auxiliary fields where a field is larger
+than the piece that one copy takes (16 MB), and at odd sizes."""
+import numpy as np
+import pytest
+
+import cases
+
+pytestmark = pytest.mark.gpu
+
+dyn = pytest.importorskip("dynfd3dcuda_amd")
+
+
+@pytest.fixture(scope="module", params=[(501, 449, 45), (19, 37, 23)], ids=["pieces", "small"])
+def faces(request):
+    nx, ny, nz = request.param
+    s = dyn.Solver(cases.volume_case(curved=False, NX=nx, NY=ny, NZ=nz, PML_N=20 if nz > 40 else 8, FreeSurface=0)["params"])
+    s.setup()
+    rng = np.random.default_rng(7)
+    v = {}
+    for n in ("PMLx1", "PMLx2", "PMLy1", "PMLy2", "PMLz1", "PMLz2"):
+        v[n] = rng.standard_normal(s.field_info(n)[0], dtype=np.float32)
+        s.put(n, v[n])
+    yield s, v
+    s.close()
+
+
+def test_round_trip(faces):
+    s, v = faces
+    for n in v:
+        assert np.array_equal(s.get(n), v[n]), n
+    s.put("PMLz1", -v["PMLz1"])
+    s.put("PMLy2", 2.0 * v["PMLy2"])
+    assert np.array_equal(s.get("PMLz1"), -v["PMLz1"]) and np.array_equal(s.get("PMLz2"), v["PMLz2"])
+    assert np.array_equal(s.get("PMLy2"), 2.0 * v["PMLy2"]) and np.array_equal(s.get("PMLy1"), v["PMLy1"])
+    s.put("PMLz1", v["PMLz1"])
+    s.put("PMLy2", v["PMLy2"])
