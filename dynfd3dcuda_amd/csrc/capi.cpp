@@ -761,25 +761,11 @@ int cgfdm_check_field(cgfdm_ctx* h, const char* name, long long* nonfinite, long
   if (r.dtype != 0) return fail(CGFDM_EPARAM, std::string("not an FP32 field: ") + name);
   std::string err;
   const int fn = r.fn ? r.fn : r.nf;
-  if (r.swap_n && r.swap_stride != r.count / r.swap_n) {  // planes of one absorbing face, one after another
-    long long bad = 0, ghost = 0;
-    double most = 0.0;
-    for (int i = 0; i < r.swap_n; i++) {
-      long long b = 0, g = 0;
-      double m = 0.0;
-      if (field_check_host(c, (const float*)r.ptr + i * r.swap_stride, 0, 0, 1, (long)(r.count / r.swap_n), &b, &g, &m, err))
-        return fail(CGFDM_EHIP, err);
-      bad += b;
-      ghost += g;
-      most = std::max(most, m);
-    }
-    if (nonfinite) *nonfinite = bad;
-    if (ghost_nonzero) *ghost_nonzero = ghost;
-    if (maxabs) *maxabs = most;
-    return 0;
-  }
-  const int rc = r.nf ? field_check_host(c, (const float*)r.ptr, r.nf, r.f0, fn, 0, nonfinite, ghost_nonzero, maxabs, err)
-                      : field_check_host(c, (const float*)r.ptr, 0, 0, 1, (long)r.count, nonfinite, ghost_nonzero, maxabs, err);
+  // an absorbing face beside another: its planes lie apart
+  const long pieces = r.swap_n && r.swap_stride != r.count / r.swap_n ? r.swap_n : 1;
+  const int rc = r.nf ? field_check_host(c, (const float*)r.ptr, r.nf, r.f0, fn, 0, 0, 0, nonfinite, ghost_nonzero, maxabs, err)
+                      : field_check_host(c, (const float*)r.ptr, 0, 0, 1, (long)r.count / pieces, pieces, (long)r.swap_stride,
+                                         nonfinite, ghost_nonzero, maxabs, err);
   return rc ? fail(CGFDM_EHIP, err) : 0;
 }
 

@@ -19,13 +19,14 @@ constexpr int kCheckBlock = 256;
 // floats order like their bit patterns)
 __global__ void __launch_bounds__(kCheckBlock) field_check_kernel(const float* __restrict__ a, int nf, int f0, int fn,
                                                                    int nx, int ny, int nz, int py, int jpad, long pyz,
-                                                                   long flat_n, unsigned long long* counts) {
+                                                                   long flat_n, long stride, unsigned per,
+                                                                   unsigned long long* counts) {
   float v = 0.0f;
   bool valid, ghost = false;
-  if (flat_n > 0) {
-    const long idx = (long)blockIdx.x * kCheckBlock + threadIdx.x;
+  if (flat_n > 0) {  // pieces of flat_n words, stride words apart; per blocks a piece
+    const long idx = (long)(blockIdx.x % per) * kCheckBlock + threadIdx.x;
     valid = idx < flat_n;
-    if (valid) v = a[idx];
+    if (valid) v = a[blockIdx.x / per * stride + idx];
   } else {
     const int j = blockIdx.x * kCheckBlock + threadIdx.x, k = blockIdx.y;
     const int i = blockIdx.z / fn, c = f0 + blockIdx.z % fn;
@@ -52,8 +53,8 @@ __global__ void clear_counts_kernel(unsigned long long* counts) {
 
 }  // namespace
 
-int field_check_host(Ctx& c, const float* ptr, int nf, int f0, int fn, long flat_n, long long* nonfinite,
-                     long long* ghost_nonzero, double* maxabs, std::string& err) {
+int field_check_host(Ctx& c, const float* ptr, int nf, int f0, int fn, long flat_n, long pieces, long stride,
+                     long long* nonfinite, long long* ghost_nonzero, double* maxabs, std::string& err) {
   if (!c.check_counts) {
     void* p = nullptr;
     if (hipMalloc(&p, 3 * sizeof(unsigned long long)) != hipSuccess) { err = "hipMalloc of the check counters"; return 1; }
@@ -62,15 +63,15 @@ int field_check_host(Ctx& c, const float* ptr, int nf, int f0, int fn, long flat
   }
   hipLaunchKernelGGL(clear_counts_kernel, dim3(1), dim3(64), 0, c.stream, c.check_counts);
   if (flat_n > 0) {
-    const long blocks = (flat_n + kCheckBlock - 1) / kCheckBlock;
-    hipLaunchKernelGGL(field_check_kernel, dim3((unsigned)blocks), dim3(kCheckBlock), 0, c.stream, ptr, 0, 0, 1, 0, 0,
-                       0, 0, 0, 0L, flat_n, c.check_counts);
+    const long per = (flat_n + kCheckBlock - 1) / kCheckBlock;
+    hipLaunchKernelGGL(field_check_kernel, dim3((unsigned)(pieces * per)), dim3(kCheckBlock), 0, c.stream, ptr, 0, 0, 1, 0, 0,
+                       0, 0, 0, 0L, flat_n, stride, (unsigned)per, c.check_counts);
   } else {
     const long zdim = (long)c.d.nx * fn;
     if (zdim > 65535 || c.d.nz > 65535) { err = "field too large for the check grid"; return 1; }
     const dim3 grid((unsigned)((c.d.ny + kCheckBlock - 1) / kCheckBlock), (unsigned)c.d.nz, (unsigned)zdim);
     hipLaunchKernelGGL(field_check_kernel, grid, dim3(kCheckBlock), 0, c.stream, ptr, nf, f0, fn, c.d.nx, c.d.ny, c.d.nz,
-                       c.d.py, c.d.jpad, c.d.pyz, 0L, c.check_counts);
+                       c.d.py, c.d.jpad, c.d.pyz, 0L, 0L, 1u, c.check_counts);
   }
   if (hipError_t e = hipGetLastError()) { err = std::string("field check launch: ") + hipGetErrorString(e); return 1; }
   unsigned long long h[3];

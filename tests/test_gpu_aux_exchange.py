@@ -34,3 +34,23 @@ def test_round_trip(faces):
     assert np.array_equal(s.get("PMLy2"), 2.0 * v["PMLy2"]) and np.array_equal(s.get("PMLy1"), v["PMLy1"])
     s.put("PMLz1", v["PMLz1"])
     s.put("PMLy2", v["PMLy2"])
+
+
+def test_check_sees_its_own_face_only(faces):
+    """One face's planes lie between the other's: non-finite words and the
+    largest magnitude at the first, a middle and the last word of a face are
+    found there and not in its neighbour."""
+    s, v = faces
+    for n, other in (("PMLx2", "PMLx1"), ("PMLy1", "PMLy2"), ("PMLz2", "PMLz1")):
+        x = v[n].reshape(-1).copy()
+        x[[0, x.size // 2, -1]] = 40.0, np.nan, -50.0
+        s.put(n, x.reshape(v[n].shape))
+        c = s.check_field(n)
+        assert c["nonfinite"] == 1 and c["maxabs"] == 50.0, n
+        x[[0, -1]] = np.inf, 30.0
+        s.put(n, x.reshape(v[n].shape))
+        c = s.check_field(n)
+        assert c["nonfinite"] == 2 and c["maxabs"] == 30.0, n
+        c = s.check_field(other)
+        assert c["nonfinite"] == 0 and c["maxabs"] == np.abs(v[other]).max(), other
+        s.put(n, v[n])
