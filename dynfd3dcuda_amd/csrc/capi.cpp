@@ -533,6 +533,7 @@ int cgfdm_fault_smooth(cgfdm_ctx* h) {
 static hipError_t swap_copy(Ctx& c, const FieldRef& r, char* host, bool to_dev) {
   const long np = r.swap_n, row = (long)(r.count / 9) / np;
   const long step = std::min(np, std::max(1L, (1L << 22) / row));  // planes of a piece: 16 MB at most, or one plane
+  const OnDevice on(c);
   float* buf = nullptr;
   if (hipError_t e = hipMalloc(&buf, step * row * sizeof(float))) return e;
   hipError_t e = hipSuccess;
@@ -896,8 +897,7 @@ int cgfdm_open_outputs(cgfdm_ctx* h) {
     return fail(CGFDM_ENETCDF, err);
   }
   o->rd = RecordDims{ni, nj, nk, kz, jy, ix, c.p.Rupture ? 1 : 0};
-  const size_t bytes = (size_t)o->rd.words() * sizeof(uint32_t);
-  if (hipMalloc(&o->dev, bytes) != hipSuccess || hipHostMalloc(&o->host, bytes, hipHostMallocDefault) != hipSuccess) {
+  if (alloc_record(c, o->rd, &o->dev, &o->host) != hipSuccess) {
     delete o;
     return fail(CGFDM_EHIP, "no memory for an output record");
   }

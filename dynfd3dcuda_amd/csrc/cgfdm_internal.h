@@ -267,6 +267,24 @@ struct Ctx {
   struct NcOut* out = nullptr;
 };
 
+// Makes the context's GPU the calling thread's current one while it lives:
+// for calls that allocate or launch and may come from a thread of its own
+// (an output thread's current GPU is the first one, whatever the solver's is).
+class OnDevice {
+  int before = 0;
+  bool set = false;
+
+ public:
+  explicit OnDevice(const Ctx& c) {
+    if (hipGetDevice(&before) == hipSuccess && before != c.device) set = hipSetDevice(c.device) == hipSuccess;
+  }
+  ~OnDevice() {
+    if (set) (void)hipSetDevice(before);
+  }
+  OnDevice(const OnDevice&) = delete;
+  OnDevice& operator=(const OnDevice&) = delete;
+};
+
 // setup (host, double precision)
 int host_setup(Ctx& c, std::string& err);
 
@@ -279,6 +297,7 @@ struct RecordDims {
   long fault_words() const { return fault ? 13L * nj * nk : 0; }
   long words() const { return fault_words() + 3L * ((long)ni * nj + (long)ni * nk + (long)nk * nj); }
 };
+hipError_t alloc_record(Ctx& c, const RecordDims& d, uint32_t** dev, uint32_t** host);
 hipError_t gather_record(Ctx& c, const RecordDims& d, uint32_t* dev, uint32_t* host);
 
 // kernel launchers (kernels.hip)

@@ -86,9 +86,18 @@ __global__ void __launch_bounds__(256) record_kernel(RecordArgs a) {
 
 }  // namespace
 
+// A record's words on the context's GPU and in pinned host memory.
+hipError_t alloc_record(Ctx& c, const RecordDims& d, uint32_t** dev, uint32_t** host) {
+  const OnDevice on(c);
+  const size_t bytes = (size_t)d.words() * sizeof(uint32_t);
+  if (hipError_t e = hipMalloc(dev, bytes)) return e;
+  return hipHostMalloc(host, bytes, hipHostMallocDefault);
+}
+
 // Gathers the record of the current wavefield and waits for it in `host`
 // (pinned, d.words() words).
 hipError_t gather_record(Ctx& c, const RecordDims& d, uint32_t* dev, uint32_t* host) {
+  const OnDevice on(c);
   RecordArgs a{};
   a.F = c.f;
   a.W = c.cur;
