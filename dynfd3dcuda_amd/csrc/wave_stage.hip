@@ -139,6 +139,10 @@ static int cu_count() {
 // blocks (three per CU; fewer rounds leave the last ones ragged:
 // 1600 x 1000 x 500, 88 k blocks: 90-95 ms of interior per step against
 // 96-101 for 1; 400 x 300 x 200, 2 k blocks: 2.50 against 2.16 ms), else 1.
+// As the box beside the other tiles, ms per step with 3 and with 1, metric as
+// bfloat16 deviations | FP32: 600 x 640 x 500, 19 k blocks, 28.3 and 31.1 | 32.6
+// and 31.9; 400 x 300 x 200, 1.5 k blocks, 5.35 and 5.59 | 6.07 and 5.88 (the
+// buffers' places in memory alone make 5% between two solvers of a process).
 // cols: 64-wide tiles along j, rows along k, planes along i.
 static int interior_kernel(const Params& p, long cols, long rows, long planes, int cus) {
   if (p.WaveInteriorKernel >= 0) return p.WaveInteriorKernel;
