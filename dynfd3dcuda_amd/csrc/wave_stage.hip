@@ -284,8 +284,13 @@ static bool bands_disjoint(const Params& p) {
 //   251 x 187 x 143  2.15   2.05   2.83
 //   400 x 300 x 200  6.20   5.91   6.00
 //   512 x 384 x 256  11.1   10.5   12.2
+//   560 x 640 x 440         23.3   25.6
 //   640 x 512 x 400         25.1   27.3
+//   600 x 640 x 500         27.9   30.7
+//   700 x 750 x 500         39.3   38.5
 //   800 x 1000 x 500 71.8   57.1   55.8
+// (with FP32 metric words 560 x 640 x 440 25.9 and 31.4, 600 x 640 x 500 30.8
+// and 33.1, 700 x 750 x 500 44.2 and 44.1)
 bool wave_unified(const Params& p) {
   if (p.WaveUnified == 0 || !bands_disjoint(p)) return false;
   const bool box_kernel = p.WaveUnified == 2 && (p.WaveInteriorKernel == 1 || p.WaveInteriorKernel == 3);

@@ -860,7 +860,8 @@ __global__ void __launch_bounds__(NT_, MINB) wave_interior_kernel(WaveArgs<MT> a
   for (int i = ibeg; i < iend; ++i) {
     // band tiles read the arguments again in every plane: held in scalar
     // registers across the loop, with the field offsets and the masks of the
-    // bands, they spill to vector lanes (444 v_readlane in the FULL loop)
+    // bands, they spill to vector lanes (444 v_readlane in the loop of the
+    // tiles of any kind)
     const ArgPtr ap = BAND ? here(kargs) : kargs;
     const bool more = i + 1 < iend;       // uniform per block
     const bool ahead = i + LEAD < iend;   // uniform per block
@@ -1422,10 +1423,9 @@ void launch_wave_t(WaveArgs<MT> a, const Ctx& c, hipStream_t s) {
     (void)hipEventRecord(c.fence[2], ss);
     (void)hipStreamWaitEvent(s, c.fence[2], 0);
   }
-  // the auxiliary fields of the points the pipelined band tiles do not
-  // advance themselves (all of them with the general band kernel; with the
-  // fused update those of the free-surface rows k >= ktop and of the edges
-  // of the absorbing box, on two or three faces)
+  // the auxiliary fields of the points whose tiles do not advance them: all
+  // of them without the fused update, with it those of the free-surface rows
+  // k >= ktop when their tiles run the general kernel
   if (a.pml && !a.rhs_only) {
     PmlAuxArgs<MT> p{};
     p.Win = a.Win; p.met = a.met; p.N = c.pml.N;
