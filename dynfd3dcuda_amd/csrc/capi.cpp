@@ -764,7 +764,7 @@ int cgfdm_check_field(cgfdm_ctx* h, const char* name, long long* nonfinite, long
   const int fn = r.fn ? r.fn : r.nf;
   // an absorbing face beside another: its planes lie apart
   const long pieces = r.swap_n && r.swap_stride != r.count / r.swap_n ? r.swap_n : 1;
-  const int rc = r.nf ? field_check_host(c, (const float*)r.ptr, r.nf, r.f0, fn, 0, 0, 0, nonfinite, ghost_nonzero, maxabs, err)
+  const int rc = r.nf ? field_check_host(c, (const float*)r.ptr, r.nf, r.f0, fn, 0, r.planes, 0, nonfinite, ghost_nonzero, maxabs, err)
                       : field_check_host(c, (const float*)r.ptr, 0, 0, 1, (long)r.count / pieces, pieces, (long)r.swap_stride,
                                          nonfinite, ghost_nonzero, maxabs, err);
   return rc ? fail(CGFDM_EHIP, err) : 0;

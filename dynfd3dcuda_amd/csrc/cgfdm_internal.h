@@ -320,7 +320,8 @@ int mlp_grad_host(const float* blob, const float* feat, const float* target, lon
 int mlp_forward_noalloc_host(const float* P, const float* feat, long n, float* out, int mode, hipStream_t s,
                              std::string& err);
 // flat_n > 0: `pieces` runs of flat_n words, stride words apart, else the
-// fields f0 .. f0+fn-1 of a volume array of nf
+// fields f0 .. f0+fn-1 of an array of `pieces` planes of nf (all planes of the
+// grid, or the fault slab's)
 int field_check_host(Ctx& c, const float* ptr, int nf, int f0, int fn, long flat_n, long pieces, long stride,
                      long long* nonfinite, long long* ghost_nonzero, double* maxabs, std::string& err);
 int stream_probe_host(int nread, int nwrite, size_t bytes_per_array, int reps, double* gbps, std::string& err);

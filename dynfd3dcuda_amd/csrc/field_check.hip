@@ -18,7 +18,7 @@ constexpr int kCheckBlock = 256;
 // counts[2] the bit pattern of the largest finite magnitude (non-negative
 // floats order like their bit patterns)
 __global__ void __launch_bounds__(kCheckBlock) field_check_kernel(const float* __restrict__ a, int nf, int f0, int fn,
-                                                                   int nx, int ny, int nz, int py, int jpad, long pyz,
+                                                                   int xlo, int xhi, int ny, int nz, int py, int jpad, long pyz,
                                                                    long flat_n, long stride, unsigned per,
                                                                    unsigned long long* counts) {
   float v = 0.0f;
@@ -32,7 +32,7 @@ __global__ void __launch_bounds__(kCheckBlock) field_check_kernel(const float* _
     const int i = blockIdx.z / fn, c = f0 + blockIdx.z % fn;
     valid = j < ny;
     if (valid) v = a[((long)i * nf + c) * pyz + (long)k * py + jpad + j];
-    ghost = i < 3 || i >= nx - 3 || k < 3 || k >= nz - 3 || j < 3 || j >= ny - 3;
+    ghost = i < xlo || i >= xhi || k < 3 || k >= nz - 3 || j < 3 || j >= ny - 3;
   }
   const bool bad = valid && !isfinite(v);
   const bool gnz = valid && ghost && v != 0.0f;
@@ -65,12 +65,15 @@ int field_check_host(Ctx& c, const float* ptr, int nf, int f0, int fn, long flat
   if (flat_n > 0) {
     const long per = (flat_n + kCheckBlock - 1) / kCheckBlock;
     hipLaunchKernelGGL(field_check_kernel, dim3((unsigned)(pieces * per)), dim3(kCheckBlock), 0, c.stream, ptr, 0, 0, 1, 0, 0,
-                       0, 0, 0, 0L, flat_n, stride, (unsigned)per, c.check_counts);
+                       0, 0, 0, 0, 0L, flat_n, stride, (unsigned)per, c.check_counts);
   } else {
-    const long zdim = (long)c.d.nx * fn;
+    // the fault slab's planes are interior ones, seven of them
+    const bool slab = pieces != c.d.nx;
+    const int xlo = slab ? 0 : 3, xhi = slab ? (int)pieces : c.d.nx - 3;
+    const long zdim = pieces * fn;
     if (zdim > 65535 || c.d.nz > 65535) { err = "field too large for the check grid"; return 1; }
     const dim3 grid((unsigned)((c.d.ny + kCheckBlock - 1) / kCheckBlock), (unsigned)c.d.nz, (unsigned)zdim);
-    hipLaunchKernelGGL(field_check_kernel, grid, dim3(kCheckBlock), 0, c.stream, ptr, nf, f0, fn, c.d.nx, c.d.ny, c.d.nz,
+    hipLaunchKernelGGL(field_check_kernel, grid, dim3(kCheckBlock), 0, c.stream, ptr, nf, f0, fn, xlo, xhi, c.d.ny, c.d.nz,
                        c.d.py, c.d.jpad, c.d.pyz, 0L, 0L, 1u, c.check_counts);
   }
   if (hipError_t e = hipGetLastError()) { err = std::string("field check launch: ") + hipGetErrorString(e); return 1; }
