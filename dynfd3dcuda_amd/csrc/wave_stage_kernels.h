@@ -387,9 +387,38 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
   }
   const uint32_t hcol4 = hcol << 2;
 
+  // ADE-PML: the lane's byte offsets in a plane of its faces' auxiliary arrays
+  // (low and high band along y and z, which may overlap; kNoWord outside a
+  // band), and which of the four the wavefront has any lane in.  Found out in
+  // the plane loop, face by face from the kernel's arguments, the flags, sizes
+  // and bases were chains of scalar loads and 61 spilled scalar registers:
+  // bands 2.98 -> 1.75 ms per step at 251 x 187 x 143 with WaveBandKernel 0,
+  // 1.94 -> 1.05 at 30 x 80 x 50 with 20 layers, which overlap along x.
   float rb2 = 1.0f, rb3 = 1.0f, cjk = 1.0f;
-  if (act && pml) { rb2 = 1.0f / a.cold.pB[1][j]; rb3 = 1.0f / a.cold.pB[2][k]; }
+  uint32_t xo4 = kNoWord, yo4[2] = {kNoWord, kNoWord}, zo4[2] = {kNoWord, kNoWord};
+  const int N = KIND >= 1 ? a.cold.N : 0;
+  const uint32_t xpp = (uint32_t)nk * nj, ypp = (uint32_t)nk * N, zpp = (uint32_t)N * nj;  // words of a field of a face plane
+  const uint32_t nyf = KIND >= 1 ? a.cold.on[2] + a.cold.on[3] : 0, nzf = KIND >= 1 ? a.cold.on[4] + a.cold.on[5] : 0;
+  if (act && pml) {
+    rb2 = 1.0f / a.cold.pB[1][j];
+    rb3 = 1.0f / a.cold.pB[2][k];
+    xo4 = (uint32_t)(j + k * nj) << 2;
+    if (a.cold.on[2] && j < N) yo4[0] = (uint32_t)(j + k * N) << 2;
+    if (a.cold.on[3] && j >= nj - N) yo4[1] = ((uint32_t)(j - (nj - N) + k * N) + (a.cold.on[2] ? 9 * ypp : 0u)) << 2;
+    if (a.cold.on[4] && k < N) zo4[0] = (uint32_t)(j + k * nj) << 2;
+    if (a.cold.on[5] && k >= nk - N) zo4[1] = ((uint32_t)(j + (k - (nk - N)) * nj) + (a.cold.on[4] ? 9 * zpp : 0u)) << 2;
+  }
+  bool hasy[2], hasz[2];
+#pragma unroll
+  for (int side = 0; side < 2; side++) {
+    hasy[side] = __builtin_amdgcn_ballot_w64(yo4[side] != kNoWord) != 0;
+    hasz[side] = __builtin_amdgcn_ballot_w64(zo4[side] != kNoWord) != 0;
+  }
   if (act && cerjan) cjk = fminf(a.cold.cj[1][j + 3], a.cold.cj[2][k + 3]);
+  const int xend0 = pml && a.cold.on[0] ? N : 0;           // planes of the low x band end here,
+  const int xbeg1 = pml && a.cold.on[1] ? ni - N : nxp;    // those of the high one begin here
+  float pbx = pml ? uni(a.cold.pB[0], ibeg) : 1.0f;        // beta along x and the sponge factor of plane i
+  float cjx = cerjan ? uni(a.cold.cj[0], ibeg + 3) : 1.0f;
 
   float q[5][9];
 #pragma unroll
@@ -412,7 +441,10 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
   }
   __syncthreads();
 
+  typedef const __attribute__((address_space(4))) WaveArgs<MT>* ArgPtr;
+  const ArgPtr kargs = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();  // the argument a
   for (int i = ibeg; i < iend; ++i) {
+    const ArgPtr ap = KIND >= 1 ? here(kargs) : kargs;  // as in wave_interior_kernel
     const int b = (i - ibeg) & 1;
     const bool more = i + 1 < iend;  // uniform per block
     // next plane of the queue and the halo of plane i+1, in flight during the compute
@@ -428,9 +460,11 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
 #pragma unroll
       for (int c = 0; c < 9; c++) hv[c] = bld(r, hcol4, c * pb);
     }
+    const float pbxn = pml && more ? uni(a.cold.pB[0], i + 1) : 1.0f;
+    const float cjxn = cerjan && more ? uni(a.cold.cj[0], i + 4) : 1.0f;
 
     if (act) {
-      const Rsrc rm = plane_rsrc(a.met, i + 3, met_nf<MT>(), nyz);
+      const Rsrc rm = plane_rsrc(ap->met, i + 3, met_nf<MT>(), nyz);
       auto MET = [&](int c) { return bldmc<MT>(rm, mcol, c, mpb, c < 10 ? a.mref[c] : 0.0f); };
       const float xix = MET(0), xiy = MET(1), xiz = MET(2);
       const float etx = MET(3), ety = MET(4), etz = MET(5);
@@ -438,8 +472,8 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
       const float lam = MET(10), mu = MET(11);
       const float rrho = 1.0f / MET(12);
       const float l2m = lam + 2.0f * mu;
-      const float rDH = a.rDH;
-      const float rb1 = pml ? 1.0f / uni(a.cold.pB[0], i) : 1.0f;
+      const float rDH = ap->rDH;
+      const float rb1 = pml ? 1.0f / pbx : 1.0f;
       const float(*L)[LK][LJ] = lds[b];
       const int lj = tj + HJL, lk = tk + HKL;
       // one-sided DRP difference of field c along each axis (macdrp.h:91-95),
@@ -453,7 +487,7 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
         return FZ > 0 ? drp5<1>(L[c][lk - 1][lj], L[c][lk][lj], L[c][lk + 1][lj], L[c][lk + 2][lj], L[c][lk + 3][lj])
                       : drp5<-1>(L[c][lk - 3][lj], L[c][lk - 2][lj], L[c][lk - 1][lj], L[c][lk][lj], L[c][lk + 1][lj]);
       };
-      const bool top = KIND == 2 && a.freenode && k >= nk - 3;  // uniform per wavefront (one k-row)
+      const bool top = KIND == 2 && ap->freenode && k >= nk - 3;  // uniform per wavefront (one k-row)
       // RHS accumulated derivative by derivative (wave.cu:133-276): each
       // field's derivative adds its momentum / Hooke terms, metric rows
       // pre-scaled by the PML 1/beta of their axis.
@@ -470,8 +504,8 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
         float dzv[3];
         if (k == nk - 1) {  // DzV from the traction-free condition (wave.cu:207-232)
           const uint32_t ij = ((uint32_t)(j + 3) + (uint32_t)(i + 3) * (uint32_t)ny) * 9;
-          const float* mVx = a.cold.mVx;
-          const float* mVy = a.cold.mVy;
+          const float* mVx = ap->cold.mVx;
+          const float* mVy = ap->cold.mVy;
           const float dxv[3] = {rDH * Dx(0), rDH * Dx(1), rDH * Dx(2)}, dyv[3] = {rDH * Dy(0), rDH * Dy(1), rDH * Dy(2)};
 #pragma unroll
           for (int r = 0; r < 3; r++)
@@ -494,7 +528,7 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
         h[7] += (e2 * dzv[0] + e0 * dzv[2]) * mu;
         h[8] += (e2 * dzv[1] + e1 * dzv[2]) * mu;
         {  // the image velocity RHS (image_top_kernel)
-          const float* w = a.itop + ((size_t)i * 18 + (k - (nk - 3))) * nj + j;
+          const float* w = ap->itop + ((size_t)i * 18 + (k - (nk - 3))) * nj + j;
 #pragma unroll
           for (int c = 0; c < 3; c++) h[c] = w[(size_t)c * 3 * nj];
         }
@@ -504,45 +538,38 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
       // inside the band of face f gets -aux_f/beta; the auxiliary fields
       // themselves are advanced afterwards by pml_aux_kernel from the same
       // stage input.
+      // (a lane without the face adds 0: each face of an axis for all lanes)
       if (pml) {
-        const int N = a.cold.N;
+        auto face = [&](Rsrc r, uint32_t o, uint32_t fb, float rbb) {
+          float v[9];
 #pragma unroll
-        for (int ax = 0; ax < 3; ax++) {
-          const int li = ax == 0 ? i : ax == 1 ? j : k;
-          const int nn = ax == 0 ? ni : ax == 1 ? nj : nk;
+          for (int c = 0; c < 9; c++) v[c] = bld(r, o, c * fb);
 #pragma unroll
-          for (int side = 0; side < 2; side++) {
-            const int f = 2 * ax + side;
-            const int off = side ? nn - N : 0;
-            if (!a.cold.on[f] || li < off || li >= off + N) continue;
-            const int pi = ax == 0 ? i - off : i;
-            const uint32_t pj = ax == 1 ? j - off : j, pk = ax == 2 ? k - off : k;
-            const uint32_t pnj = ax == 1 ? N : nj, pnk = ax == 2 ? N : nk, pp = pnj * pnk;
-            const uint32_t pa4 = (pj + pk * pnj) << 2;
-            const float rbb = ax == 0 ? rb1 : ax == 1 ? rb2 : rb3;  // 1 / beta at li
-            const uint32_t np = ax == 0 ? 1u : (uint32_t)(a.cold.on[2 * ax] + a.cold.on[2 * ax + 1]);
-            const Rsrc ry = aux_rsrc(a.cold.auxY[f], pi, pp, np);
-#pragma unroll
-            for (int c = 0; c < 9; c++) h[c] += -bld(ry, pa4, c * 4 * pp) * rbb;
-          }
-        }
+          for (int c = 0; c < 9; c++) h[c] += -v[c] * rbb;
+        };
+        if (i < xend0) face(aux_rsrc(ap->cold.axY[0], i, xpp, 1), xo4, here(4 * xpp), rb1);
+        if (i >= xbeg1) face(aux_rsrc(ap->cold.axY[0], i - xbeg1 + xend0, xpp, 1), xo4, here(4 * xpp), rb1);
+        if (hasy[0]) face(aux_rsrc(ap->cold.axY[1], i, ypp, nyf), yo4[0], here(4 * ypp), rb2);
+        if (hasy[1]) face(aux_rsrc(ap->cold.axY[1], i, ypp, nyf), yo4[1], here(4 * ypp), rb2);
+        if (hasz[0]) face(aux_rsrc(ap->cold.axY[2], i, zpp, nzf), zo4[0], here(4 * zpp), rb3);
+        if (hasz[1]) face(aux_rsrc(ap->cold.axY[2], i, zpp, nzf), zo4[1], here(4 * zpp), rb3);
       }
 
-      if (a.rhs_only) {
+      if (ap->rhs_only) {
 #pragma unroll
-        for (int c = 0; c < 9; c++) bst(plane_rsrc(a.rhs, i + 3, 9, nyz), col4, c * pb, h[c]);
-      } else if (a.fault && i >= a.ii0 - 3 && i <= a.ii0 + 3 && i != a.ii0) {
-        const Rsrc r = plane_rsrc(a.slabH, i - (a.ii0 - 3), 9, nyz);  // slab planes share the layout
+        for (int c = 0; c < 9; c++) bst(plane_rsrc(ap->rhs, i + 3, 9, nyz), col4, c * pb, h[c]);
+      } else if (ap->fault && i >= ap->ii0 - 3 && i <= ap->ii0 + 3 && i != ap->ii0) {
+        const Rsrc r = plane_rsrc(ap->slabH, i - (ap->ii0 - 3), 9, nyz);  // slab planes share the layout
 #pragma unroll
         for (int c = 0; c < 9; c++) bst(r, col4, c * pb, h[c]);
       } else {
-        const float damp = cerjan ? fminf(uni(a.cold.cj[0], i + 3), cjk) : 1.0f;
-        const bool keep_t = damp != 1.0f || (a.fault && i == a.ii0);
-        const Rsrc rs = plane_rsrc(a.S, i + 3, 9, nyz), rt = plane_rsrc(a.T, i + 3, 9, nyz);
-        const Rsrc ro = plane_rsrc(a.Wout, i + 3, 9, nyz);
+        const float damp = cerjan ? fminf(cjx, cjk) : 1.0f;
+        const bool keep_t = damp != 1.0f || (ap->fault && i == ap->ii0);
+        const Rsrc rs = plane_rsrc(ap->S, i + 3, 9, nyz), rt = plane_rsrc(ap->T, i + 3, 9, nyz);
+        const Rsrc ro = plane_rsrc(ap->Wout, i + 3, 9, nyz);
 #pragma unroll
         for (int c = 0; c < 9; c++) {
-          const float w = rk_combine_b(a.irk, a.rka, a.rkb, q[CTR][c], h[c], rs, rt, col4, c * pb, keep_t);
+          const float w = rk_combine_b(ap->irk, ap->rka, ap->rkb, q[CTR][c], h[c], rs, rt, col4, c * pb, keep_t);
           bst(ro, col4, c * pb, w * damp);
         }
       }
@@ -562,6 +589,8 @@ __global__ void __launch_bounds__(NT_, KIND == 2 ? 2 : 4) wave_stage_kernel(Wave
       for (int c = 0; c < 9; c++) q[m][c] = q[m + 1][c];
 #pragma unroll
     for (int c = 0; c < 9; c++) q[4][c] = nq[c];
+    pbx = pbxn;
+    cjx = cjxn;
     __syncthreads();
   }
 }
