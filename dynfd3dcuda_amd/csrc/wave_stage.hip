@@ -480,11 +480,16 @@ std::vector<int4> wave_work_list(Ctx& c, int cus, std::vector<int>& boxes) {
     };
     for (int f = 0; f < 6; f++) {
       if (!c.pml.on[f] || (c.pml_fused && c.wave_surf_pipe)) continue;
-      const int ax = f / 2;
-      const int pnj = ax == 1 ? N : c.d.nj, pnk = ax == 2 ? N : c.d.nk, pni = ax == 0 ? N : c.d.ni;
-      const int off = f == 5 ? c.d.nk - N : 0;  // first row of the face
-      const int s0 = c.pml_fused ? std::max(ktop - off, 0) : 0;
-      add(f, 0, pnj, s0, pnk - s0, 0, pni);
+      // per axis the face's first point and the one past its last; of a layer
+      // wider than the axis only the points of the grid
+      int p0[3], p1[3];
+      for (int ax = 0; ax < 3; ax++) {
+        const bool own = ax == f / 2;
+        p0[ax] = own && (f & 1) ? std::max(N - n3[ax], 0) : 0;
+        p1[ax] = !own ? n3[ax] : (f & 1) ? N : std::min(N, n3[ax]);
+      }
+      if (c.pml_fused) p0[2] = std::max(p0[2], ktop - (f == 5 ? nk - N : 0));
+      add(f, p0[1], p1[1] - p0[1], p0[2], p1[2] - p0[2], p0[0], p1[0] - p0[0]);
     }
     c.pml_nbox = (int)bx.size() / kPmlBoxInts;
     c.pml_blocks = blocks;

@@ -132,3 +132,31 @@ def test_kernel_of_the_interior_box(tool, opts, rows):
     r = work(tool, **opts)
     assert r["unified"] and r["points"][0] > 0
     assert {it[6] for it in r["item"] if it[0] == 0} == {rows} and r["ring"] == (rows == 8)
+
+
+@pytest.mark.parametrize("free", [1, 0], ids=["surface", "no_surface"])
+@pytest.mark.parametrize("dims", [(18, 40, 24), (30, 17, 24), (18, 19, 15), (40, 44, 16)], ids=lambda d: "x".join(map(str, d)))
+def test_layers_wider_than_the_grid_stay_inside_it(tool, dims, free):
+    """A layer of 20 points along an axis of fewer: the boxes of the
+    auxiliary kernel hold the grid's points and none beside it, each
+    (point, face) pair once."""
+    N = 20
+    r = work(tool, **dict(zip(("NX", "NY", "NZ"), dims)), PML_N=N, FreeSurface=free)
+    faces, updated = np.zeros(dims, int), np.zeros(dims, int)
+    for f in range(5 if free else 6):
+        ax, n = f // 2, dims[f // 2]
+        band = np.zeros(n, int)
+        band[max(n - N, 0):] = 1 if f & 1 else band[max(n - N, 0):]
+        if not f & 1:
+            band[:N] = 1
+        faces += band.reshape([-1 if a == ax else 1 for a in range(3)])
+    for f, j, nj, k, nk, i, ni, _ in r["box"]:
+        first = [i, j, k]
+        first[f // 2] += dims[f // 2] - N if f & 1 else 0
+        for a, n in enumerate((ni, nj, nk)):
+            assert first[a] >= 0 and first[a] + n <= dims[a], (f, first)
+        updated[tuple(slice(x, x + n) for x, n in zip(first, (ni, nj, nk)))] += 1
+    assert bool(r["box"]) != bool(r["fused"])  # without overlap the tiles advance them all
+    if r["box"]:
+        assert np.array_equal(updated, faces)
+    assert sum(r["update"]) == faces.sum()
