@@ -100,13 +100,14 @@ static void clear_counts(Ctx& c) {
 // fields.  Every list counts what it pushes, so that a tile missed or listed
 // twice shows in the sums.
 static void count_block(Ctx& c, int kd, int i0, int i1, int j0, int j1, int k0, int k1, bool update) {
-  // points of [lo, hi) along axis ax inside that axis's absorbing bands
+  // points of [lo, hi) along axis ax inside that axis's absorbing bands, once
+  // for each of the two where they overlap
   auto in_bands = [&](int ax, int lo, int hi) {
     const int N = c.pml.N, nn = ax == 0 ? c.d.ni : ax == 1 ? c.d.nj : c.d.nk;
     const int a0 = 0, a1 = c.pml.on[2 * ax] ? std::min(N, nn) : 0;
     const int b0 = c.pml.on[2 * ax + 1] ? std::max(nn - N, 0) : nn, b1 = nn;
     auto len = [&](int x0, int x1) { return std::max(0, std::min(x1, hi) - std::max(x0, lo)); };
-    return len(a0, a1) + len(b0, b1) - len(std::max(a0, b0), std::min(a1, b1));
+    return len(a0, a1) + len(b0, b1);
   };
   const long Li = i1 - i0, Lj = j1 - j0, Lk = k1 - k0;
   const long bi = in_bands(0, i0, i1), bj = in_bands(1, j0, j1), bk = in_bands(2, k0, k1);

@@ -159,4 +159,4 @@ def test_layers_wider_than_the_grid_stay_inside_it(tool, dims, free):
     assert bool(r["box"]) != bool(r["fused"])  # without overlap the tiles advance them all
     if r["box"]:
         assert np.array_equal(updated, faces)
-    assert sum(r["update"]) == faces.sum()
+    assert sum(r["read"]) == sum(r["update"]) == faces.sum()
