@@ -524,29 +524,25 @@ int cgfdm_fault_smooth(cgfdm_ctx* h) {
 }
 
 // Between the caller's [field][plane][words] and the device's
-// [plane][field][words], planes swap_stride words apart: a field's planes at a
-// time gathered on the device into a buffer (or scattered from it) that one
-// copy brings over.  What is left is the copy of pageable memory: a y face of
+// [plane][field][words], planes swap_stride words apart: pieces of at most 16 MB
+// gathered on the device into a buffer (or scattered from it) that one copy
+// brings over.  What is left is the copy of pageable memory: a y face of
 // 400 x 300 x 200 (54 MB) takes 2.1 ms to put and 5.8 to get; swapped on the
 // host, with the words between the face's planes brought over as well, 35 and
 // 33 ms.
 static hipError_t swap_copy(Ctx& c, const FieldRef& r, char* host, bool to_dev) {
-  const long np = r.swap_n, row = (long)(r.count / 9) / np;
-  const long step = std::min(np, std::max(1L, (1L << 22) / row));  // planes of a piece: 16 MB at most, or one plane
+  const long n = (long)r.count, step = std::min(n, 1L << 22);
   const OnDevice on(c);
   float* buf = nullptr;
-  if (hipError_t e = hipMalloc(&buf, step * row * sizeof(float))) return e;
+  if (hipError_t e = hipMalloc(&buf, step * sizeof(float))) return e;
   hipError_t e = hipSuccess;
-  for (int f = 0; f < 9 && !e; f++)
-    for (long i = 0; i < np && !e; i += step) {
-      const long n = std::min(step, np - i);
-      const size_t bytes = n * row * sizeof(float);
-      char* h = host + (f * np + i) * row * sizeof(float);
-      float* d = (float*)r.ptr + i * (long)r.swap_stride + f * row;
-      if (to_dev) e = hipMemcpyAsync(buf, h, bytes, hipMemcpyHostToDevice, c.stream);
-      if (!e) e = launch_plane_copy(c, buf, d, n, row, (long)r.swap_stride, to_dev);
-      if (!e && !to_dev) e = hipMemcpyAsync(h, buf, bytes, hipMemcpyDeviceToHost, c.stream);
-    }
+  for (long q = 0; q < n && !e; q += step) {
+    const long m = std::min(step, n - q);
+    char* h = host + q * sizeof(float);
+    if (to_dev) e = hipMemcpyAsync(buf, h, m * sizeof(float), hipMemcpyHostToDevice, c.stream);
+    if (!e) e = launch_swap(c, buf, (float*)r.ptr, q, m, r.swap_n, n / 9 / r.swap_n, (long)r.swap_stride, to_dev);
+    if (!e && !to_dev) e = hipMemcpyAsync(h, buf, m * sizeof(float), hipMemcpyDeviceToHost, c.stream);
+  }
   const hipError_t done = hipStreamSynchronize(c.stream);
   (void)hipFree(buf);
   return e ? e : done;

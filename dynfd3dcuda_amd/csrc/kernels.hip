@@ -1093,12 +1093,15 @@ __global__ void fill_kernel(float* p, long n, float v) {
   for (; i < n; i += st) p[i] = v;
 }
 
-// Rows of `row` words, packed in buf and stride words apart in d; per blocks a row.
-__global__ void __launch_bounds__(256) plane_copy_kernel(float* buf, float* d, long row, long stride, unsigned per, bool to_d) {
-  const long i = blockIdx.x / per, x = (long)(blockIdx.x % per) * 256 + threadIdx.x;
-  if (x >= row) return;
-  if (to_d) d[i * stride + x] = buf[i * row + x];
-  else buf[i * row + x] = d[i * stride + x];
+// Words q .. q + n - 1 of an array [9][planes][row], packed in buf and
+// [planes][9][row] in d with the planes stride words apart.
+__global__ void __launch_bounds__(256) swap_kernel(float* buf, float* d, long q, long n, long planes, long row, long stride, bool to_d) {
+  const long t = (long)blockIdx.x * 256 + threadIdx.x;
+  if (t >= n) return;
+  const long w = q + t, fi = w / row, f = fi / planes;
+  float* p = d + (fi - f * planes) * stride + f * row + (w - fi * row);
+  if (to_d) *p = buf[t];
+  else buf[t] = *p;
 }
 
 FArgs make_fargs(Ctx& c) {
@@ -1205,9 +1208,8 @@ void launch_fill(Ctx& c, float* p, long n, float v) {
   hipLaunchKernelGGL(fill_kernel, dim3((unsigned)blocks), dim3(256), 0, c.stream, p, n, v);
 }
 
-hipError_t launch_plane_copy(Ctx& c, float* buf, float* d, long n, long row, long stride, bool to_d) {
-  const unsigned per = (unsigned)((row + 255) / 256);
-  hipLaunchKernelGGL(plane_copy_kernel, dim3((unsigned)n * per), dim3(256), 0, c.stream, buf, d, row, stride, per, to_d);
+hipError_t launch_swap(Ctx& c, float* buf, float* d, long q, long n, long planes, long row, long stride, bool to_d) {
+  hipLaunchKernelGGL(swap_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c.stream, buf, d, q, n, planes, row, stride, to_d);
   return hipGetLastError();
 }
 
