@@ -523,48 +523,51 @@ int cgfdm_fault_smooth(cgfdm_ctx* h) {
   return check_hip("fault smoothing launch");
 }
 
-// Between the caller's [field][plane][words] and the device's
-// [plane][field][words], planes swap_stride words apart: pieces of at most 16 MB
-// gathered on the device into a buffer (or scattered from it) that one copy
-// brings over.  What is left is the copy of pageable memory: a y face of
-// 400 x 300 x 200 (54 MB) takes 2.1 ms to put and 5.8 to get; swapped on the
-// host, with the words between the face's planes brought over as well, 35 and
-// 33 ms.
-static hipError_t swap_copy(Ctx& c, const FieldRef& r, char* host, bool to_dev) {
-  const long n = (long)r.count, step = std::min(n, 1L << 22);
+// Between the caller's layout and the device's, for the fields that are laid
+// out anew: pieces of at most 16 MB gathered on the device into a buffer (or
+// scattered from it), which one copy brings over.  Volume arrays are the
+// reference's [field][plane][k][j] with rows of ny for the caller (the fault
+// slab [plane][field][k][j]) and [plane][field][k][jpad + j] with rows of py on
+// the device; the auxiliary fields of an absorbing face [field][plane][words]
+// and [plane][field][words], planes swap_stride words apart.  What is left is
+// the copy of pageable memory.  Laid out anew on the host, with the padding and
+// the other face's words brought over as well, the wavefield of
+// 100 x 200 x 100 (81 MB) took 36 ms to put or get (now 3.2 and 8.9) and a y
+// face of 400 x 300 x 200 (54 MB) 35 and 33 (2.1 and 5.9).
+static hipError_t exchange(Ctx& c, const FieldRef& r, char* host, bool to_dev) {
+  Exchange x;
+  const size_t es = dsize(r.dtype);
+  char* d = (char*)r.ptr;
+  if (r.nf) {
+    const long nfo = r.fn ? r.fn : r.nf, plane = r.nf * c.d.pyz;
+    const bool slab = r.planes != c.d.nx;
+    x = Exchange{slab ? nfo : r.planes, c.d.nz, c.d.ny, slab ? plane : c.d.pyz, slab ? c.d.pyz : plane, c.d.py};
+    d += (r.f0 * c.d.pyz + c.d.jpad) * es;
+  } else {
+    const long row = (long)(r.count / 9) / r.swap_n;
+    x = Exchange{r.swap_n, 1, row, row, (long)r.swap_stride, 0};
+  }
   const OnDevice on(c);
-  float* buf = nullptr;
-  if (hipError_t e = hipMalloc(&buf, step * sizeof(float))) return e;
-  hipError_t e = hipSuccess;
+  const long n = (long)r.count;
+  long step = std::min(n, (long)((16u << 20) / es));
+  void* buf = nullptr;
+  hipError_t e = hipMalloc(&buf, step * es);
+  while (e != hipSuccess && step > 4096) {  // a card that is full: smaller pieces
+    (void)hipGetLastError();
+    step /= 2;
+    e = hipMalloc(&buf, step * es);
+  }
+  if (e) return e;
   for (long q = 0; q < n && !e; q += step) {
     const long m = std::min(step, n - q);
-    char* h = host + q * sizeof(float);
-    if (to_dev) e = hipMemcpyAsync(buf, h, m * sizeof(float), hipMemcpyHostToDevice, c.stream);
-    if (!e) e = launch_swap(c, buf, (float*)r.ptr, q, m, r.swap_n, n / 9 / r.swap_n, (long)r.swap_stride, to_dev);
-    if (!e && !to_dev) e = hipMemcpyAsync(h, buf, m * sizeof(float), hipMemcpyDeviceToHost, c.stream);
+    char* h = host + q * es;
+    if (to_dev) e = hipMemcpyAsync(buf, h, m * es, hipMemcpyHostToDevice, c.stream);
+    if (!e) e = launch_exchange(c, buf, d, (int)es, q, m, x, to_dev);
+    if (!e && !to_dev) e = hipMemcpyAsync(h, buf, m * es, hipMemcpyDeviceToHost, c.stream);
   }
   const hipError_t done = hipStreamSynchronize(c.stream);
   (void)hipFree(buf);
   return e ? e : done;
-}
-
-// Between the caller's layout (the reference's: [field][plane][k][j], rows
-// of ny) and the device's plane-interleaved [plane][field][k][jpad + j] with
-// rows of py; to_dev selects the direction.  The slab buffer is the one
-// exception on the caller's side: it is [plane][field][k][j] there too.
-static size_t dev_words(const Ctx& c, const FieldRef& r) { return (size_t)r.planes * r.nf * c.d.pyz; }
-static void interleave_copy(const Ctx& c, const FieldRef& r, const char* from, char* to, bool to_dev) {
-  const size_t es = dsize(r.dtype), nz = (size_t)c.d.nz, ny = (size_t)c.d.ny, py = (size_t)c.d.py;
-  const size_t np = (size_t)r.planes, nf = (size_t)r.nf, pyz = (size_t)c.d.pyz, nyz = ny * nz;
-  const bool slab = np != (size_t)c.d.nx;
-  for (size_t i = 0; i < np; i++)
-    for (size_t f = (size_t)r.f0; f < (r.fn ? (size_t)(r.f0 + r.fn) : nf); f++)
-      for (size_t k = 0; k < nz; k++) {
-        const size_t fo = f - (size_t)r.f0, nfo = r.fn ? (size_t)r.fn : nf;
-        const size_t dev = ((i * nf + f) * pyz + k * py + c.d.jpad) * es;
-        const size_t ref = ((slab ? i * nfo + fo : fo * np + i) * nyz + k * ny) * es;
-        std::memcpy(to + (to_dev ? dev : ref), from + (to_dev ? ref : dev), ny * es);
-      }
 }
 
 int cgfdm_field_info(cgfdm_ctx* h, const char* name, size_t* count, int* dtype) {
@@ -588,14 +591,8 @@ int cgfdm_get_field(cgfdm_ctx* h, const char* name, void* dst, size_t bytes) {
     return 0;
   }
   if (hipError_t e = hipStreamSynchronize(c.stream)) return fail(CGFDM_EHIP, hipGetErrorString(e));
-  if (!r.nf) {
-    if ((r.swap_n ? swap_copy(c, r, (char*)dst, false) : hipMemcpy(dst, r.ptr, bytes, hipMemcpyDeviceToHost)) != hipSuccess)
-      return fail(CGFDM_EHIP, "copy failed");
-    return 0;
-  }
-  std::vector<char> tmp(dev_words(c, r) * dsize(r.dtype));
-  if (hipMemcpy(tmp.data(), r.ptr, tmp.size(), hipMemcpyDeviceToHost) != hipSuccess) return fail(CGFDM_EHIP, "copy failed");
-  interleave_copy(c, r, tmp.data(), (char*)dst, false);
+  if ((r.nf || r.swap_n ? exchange(c, r, (char*)dst, false) : hipMemcpy(dst, r.ptr, bytes, hipMemcpyDeviceToHost)) != hipSuccess)
+    return fail(CGFDM_EHIP, "copy failed");
   return 0;
 }
 
@@ -612,16 +609,8 @@ int cgfdm_put_field(cgfdm_ctx* h, const char* name, const void* src, size_t byte
   if (bytes != r.count * dsize(r.dtype)) return fail(CGFDM_ESIZE, std::string("size mismatch for ") + name);
   if (r.host) return fail(CGFDM_EPARAM, std::string("read-only field ") + name);
   if (hipError_t e = hipStreamSynchronize(c.stream)) return fail(CGFDM_EHIP, hipGetErrorString(e));
-  if (!r.nf) {
-    if ((r.swap_n ? swap_copy(c, r, (char*)src, true) : hipMemcpy(r.ptr, src, bytes, hipMemcpyHostToDevice)) != hipSuccess)
-      return fail(CGFDM_EHIP, "copy failed");
-    return 0;
-  }
-  // read-modify-write keeps the row padding of the device array as it is
-  std::vector<char> tmp(dev_words(c, r) * dsize(r.dtype));
-  if (hipMemcpy(tmp.data(), r.ptr, tmp.size(), hipMemcpyDeviceToHost) != hipSuccess) return fail(CGFDM_EHIP, "copy failed");
-  interleave_copy(c, r, (const char*)src, tmp.data(), true);
-  if (hipMemcpy(r.ptr, tmp.data(), tmp.size(), hipMemcpyHostToDevice) != hipSuccess) return fail(CGFDM_EHIP, "copy failed");
+  if ((r.nf || r.swap_n ? exchange(c, r, (char*)src, true) : hipMemcpy(r.ptr, src, bytes, hipMemcpyHostToDevice)) != hipSuccess)
+    return fail(CGFDM_EHIP, "copy failed");
   return 0;
 }
 

@@ -328,9 +328,13 @@ int stream_probe_host(int nread, int nwrite, size_t bytes_per_array, int reps, d
 int mlp_train_host(float* blob, const float* feat, const float* target, long n, int epochs, int batch, float lr,
                    unsigned seed, float* loss_hist, std::string& err);
 void launch_fill(Ctx& c, float* p, long n, float v);
-// the n words from word q on of an array [9][planes][row], packed in buf, from
-// d, where it is [planes][9][row] with the planes stride words apart, or back
-hipError_t launch_swap(Ctx& c, float* buf, float* d, long q, long n, long planes, long row, long stride, bool to_d);
+// An array [.][b][k][j] of the caller whose element (a, b, k, j) sits at
+// a*as + b*bs + k*ks + j on the device.
+struct Exchange {
+  long b, k, j, as, bs, ks;
+};
+// its n elements of es bytes (2 or 4) from element q on, from d to the packed buf or back
+hipError_t launch_exchange(Ctx& c, void* buf, void* d, int es, long q, long n, const Exchange& x, bool to_d);
 int upload_wave_work(Ctx& c);  // nonzero on a HIP error
 
 // The stage kernels' work list (two int4 per block) for a device of cus

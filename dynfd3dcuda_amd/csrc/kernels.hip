@@ -1093,13 +1093,12 @@ __global__ void fill_kernel(float* p, long n, float v) {
   for (; i < n; i += st) p[i] = v;
 }
 
-// Words q .. q + n - 1 of an array [9][planes][row], packed in buf and
-// [planes][9][row] in d with the planes stride words apart.
-__global__ void __launch_bounds__(256) swap_kernel(float* buf, float* d, long q, long n, long planes, long row, long stride, bool to_d) {
+template <class T>
+__global__ void __launch_bounds__(256) exchange_kernel(T* buf, T* d, long q, long n, Exchange x, bool to_d) {
   const long t = (long)blockIdx.x * 256 + threadIdx.x;
   if (t >= n) return;
-  const long w = q + t, fi = w / row, f = fi / planes;
-  float* p = d + (fi - f * planes) * stride + f * row + (w - fi * row);
+  const long w = q + t, row = w / x.j, bk = row / x.k, a = bk / x.b;
+  T* p = d + a * x.as + (bk - a * x.b) * x.bs + (row - bk * x.k) * x.ks + (w - row * x.j);
   if (to_d) *p = buf[t];
   else buf[t] = *p;
 }
@@ -1208,8 +1207,12 @@ void launch_fill(Ctx& c, float* p, long n, float v) {
   hipLaunchKernelGGL(fill_kernel, dim3((unsigned)blocks), dim3(256), 0, c.stream, p, n, v);
 }
 
-hipError_t launch_swap(Ctx& c, float* buf, float* d, long q, long n, long planes, long row, long stride, bool to_d) {
-  hipLaunchKernelGGL(swap_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c.stream, buf, d, q, n, planes, row, stride, to_d);
+hipError_t launch_exchange(Ctx& c, void* buf, void* d, int es, long q, long n, const Exchange& x, bool to_d) {
+  const dim3 g((unsigned)((n + 255) / 256));
+  if (es == 2)
+    hipLaunchKernelGGL(exchange_kernel<uint16_t>, g, dim3(256), 0, c.stream, (uint16_t*)buf, (uint16_t*)d, q, n, x, to_d);
+  else
+    hipLaunchKernelGGL(exchange_kernel<uint32_t>, g, dim3(256), 0, c.stream, (uint32_t*)buf, (uint32_t*)d, q, n, x, to_d);
   return hipGetLastError();
 }
 

@@ -54,3 +54,18 @@ def test_check_sees_its_own_face_only(faces):
         c = s.check_field(other)
         assert c["nonfinite"] == 0 and c["maxabs"] == np.abs(v[other]).max(), other
         s.put(n, v[n])
+
+
+def test_wavefield_round_trip(faces):
+    """Pieces end in the middle of rows; the check reads the device's own layout."""
+    s, _ = faces
+    d = s.dims()
+    W = np.random.default_rng(9).standard_normal(s.field_info("W")[0], dtype=np.float32).reshape(9, d["nx"], d["nz"], d["ny"])
+    W[4, 2, 5, 7] = np.nan  # a ghost plane
+    s.put("W", W)
+    assert np.array_equal(s.get("W").reshape(W.shape), W, equal_nan=True)
+    inner = W[:, 3:-3, 3:-3, 3:-3]
+    c = s.check_field("W")
+    assert c == {"nonfinite": 1, "ghost_nonzero": np.count_nonzero(W) - np.count_nonzero(inner), "maxabs": np.abs(inner).max()}
+    s.put("W", np.zeros_like(W))
+    assert s.check_field("W") == {"nonfinite": 0, "ghost_nonzero": 0, "maxabs": 0.0}
