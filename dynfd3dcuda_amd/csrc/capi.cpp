@@ -557,7 +557,10 @@ static hipError_t exchange(Ctx& c, const FieldRef& r, char* host, bool to_dev) {
     step /= 2;
     e = hipMalloc(&buf, step * es);
   }
-  if (e) return e;
+  if (e) {
+    (void)hipGetLastError();  // reported here, not by the next launch's check
+    return e;
+  }
   for (long q = 0; q < n && !e; q += step) {
     const long m = std::min(step, n - q);
     char* h = host + q * es;
