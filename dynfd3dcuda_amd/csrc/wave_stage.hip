@@ -135,7 +135,7 @@ static int cu_count() {
   return cus;
 }
 
-// The interior kernel (WaveInteriorKernel, see upload_wave_work): -1 (default)
+// The interior kernel (WaveInteriorKernel, see wave_work_list): -1 (default)
 // picks 3 when the interior launch holds at least 16 rounds of resident 64 x 4
 // blocks (three per CU; fewer rounds leave the last ones ragged:
 // 1600 x 1000 x 500, 88 k blocks: 90-95 ms of interior per step against

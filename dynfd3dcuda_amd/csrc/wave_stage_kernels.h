@@ -1466,7 +1466,7 @@ void launch_wave_t(WaveArgs<MT> a, const Ctx& c, hipStream_t s) {
     for (int ax = 0; ax < 3; ax++) p.np[ax] = c.pml.parts(ax);
     p.mat[0] = c.matVx2Vz; p.mat[1] = c.matVy2Vz;
     for (int f = 0; f < 6; f++) { p.Y[f] = c.pml.Y[f]; p.S[f] = c.pml.S[f]; p.T[f] = c.pml.T[f]; }
-    // the boxes (upload_wave_work): every face whole, or with the fused
+    // the boxes (wave_work_list): every face whole, or with the fused
     // update the free-surface rows when their tiles run the general kernel
     p.boxes = c.pml_boxes;
     p.nbox = c.pml_nbox;
